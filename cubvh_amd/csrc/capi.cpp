@@ -36,8 +36,8 @@ int fail_hip(hipError_t e, const char* what) {
 
 constexpr int kMaxDevices = 64;
 constexpr int kDefaultLeaf = 16;  // faces per leaf unless the caller asks otherwise
-// Point-query batches at least this large are sorted into Morton order and walked as
-// wave packets; smaller ones are walked one lane per query in input order.
+// Raystab batches at least this large are sorted into Morton order; smaller ones are
+// walked one lane per query in input order.
 constexpr int64_t kMortonMin = 1 << 11;
 
 // Keeps freed stream-ordered allocations in the device's default pool instead of
@@ -357,7 +357,7 @@ int run_distance(cubvh_bvh* bvh, int device, int64_t n, int kmode, const float* 
     // Large batches are walked in Morton order (stream-ordered scratch from the
     // device's default memory pool, released after the launch).
     void* scratch = nullptr;
-    if (n >= kMortonMin && n < ((int64_t)1 << 31)) {
+    if (n >= (kmode == 2 ? kMortonMin : kWaveMax) && n < ((int64_t)1 << 31)) {
         rc = ensure_pool(device);
         if (rc != CUBVH_OK) return rc;
         const size_t ob = ((size_t)n * 4 + 255) & ~(size_t)255;
@@ -766,7 +766,7 @@ int cubvh_unsigned_distance_noalloc(cubvh_bvh* bvh, int device, int64_t n, const
     q.out_v = uvw;
     q.packet = false;
     hipStream_t hs = (hipStream_t)stream;
-    if (n >= kMortonMin) {
+    if (n >= kWaveMax) {
         void* ws = nullptr;
         hipError_t e = noalloc_scratch(device, &ws);
         if (e != hipSuccess) return fail_hip(e, "hipGetSymbolAddress(scratch)");
@@ -893,9 +893,9 @@ int cubvh_ray_trace(cubvh_bvh* bvh, int device, int64_t n, const float* rays_o, 
     q.out_v = positions;
     q.out_id = face_id;
     q.out_f = depth;
-    // packets from 2,048 rays on, walked in an order that keeps rays of close origins and
-    // directions together (stream-ordered scratch, released after the launch)
-    q.packet = n >= kMortonMin;
+    // packets are walked in an order that keeps rays of close origins and directions
+    // together (stream-ordered scratch, released after the launch)
+    q.packet = n >= kWaveMax;
     hipStream_t hs = (hipStream_t)stream;
     void* scratch = nullptr;
     if (q.packet && n < ((int64_t)1 << 31)) {

@@ -1,6 +1,9 @@
 // query.hip -- BVH traversal kernels for gfx950 (wave64).
 //
-// One lane per query.  Each lane walks the 4-wide tree nearest-child-first: the
+// Three forms: one lane per query (stab rays, incoherent rays), a packet of 64 queries per
+// wave (below, "Packet traversal") and one wave per query (wave_walk.hpp).
+//
+// One lane per query: each lane walks the 4-wide tree nearest-child-first: the
 // four child bounds of a node arrive as six 16-byte loads (structure-of-arrays
 // inside the 128-byte node), the four box tests run as independent lane-local
 // arithmetic, the surviving children are ordered with a 5-comparator network, the
@@ -17,8 +20,6 @@
 //   any-hit:  exists a face with t < 1000
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-
-
 
 
 #include "bvh.hpp"
@@ -52,8 +53,9 @@ __host__ __device__ inline Tree make_tree(const TreeArrays& a, int64_t face0_slo
 // |p - x|^2 >= max(|h| - t, 0)^2 + max(rho - r, 0)^2 with h = n.(p - c) and rho the
 // in-plane distance from c.  The margin 2^-15 (|p-c|^2 + r^2) exceeds the fp32
 // rounding of this bound and of the exact face test, so a rejected face could not
-// have produced a squared distance <= bound (nor tied the best).
-__device__ __forceinline__ bool disk_rejects(f3 p, float4 cb, float4 nb, float bound) {
+// have produced a squared distance <= bound (nor tied the best).  disk_bound is that
+// lower bound less the margin.
+__device__ __forceinline__ float disk_bound(f3 p, float4 cb, float4 nb) {
     f3 d = mk3(p.x - cb.x, p.y - cb.y, p.z - cb.z);
     float dd = dot3(d, d);
     float h = dot3(mk3(nb.x, nb.y, nb.z), d);
@@ -62,7 +64,10 @@ __device__ __forceinline__ bool disk_rejects(f3 p, float4 cb, float4 nb, float b
     float t = fmaxf(rho - cb.w, 0.0f);
     float lb = ah * ah + t * t;
     float margin = 3.0517578125e-05f * (dd + cb.w * cb.w);
-    return lb - margin > bound;
+    return lb - margin;
+}
+__device__ __forceinline__ bool disk_rejects(f3 p, float4 cb, float4 nb, float bound) {
+    return disk_bound(p, cb, nb) > bound;
 }
 
 __device__ __forceinline__ FaceConst load_face(const float4* __restrict__ tpre, int32_t slot) {
@@ -821,6 +826,14 @@ __device__ __forceinline__ void store_pt(float* __restrict__ p, int64_t i, f3 v)
     p[3 * i + 2] = v.z;
 }
 
+}  // namespace dev
+}  // namespace cubvh_amd
+
+#include "wave_walk.hpp"
+
+namespace cubvh_amd {
+namespace dev {
+
 // mode: 0 unsigned, 1 signed watertight, 2 signed raystab
 template <int BLOCK, int LDS_N, int MODE>
 __global__ __launch_bounds__(BLOCK) void distance_kernel(int64_t n, const float* __restrict__ positions,
@@ -1200,30 +1213,6 @@ __global__ __launch_bounds__(64 * WAVES, PERSISTENT ? 7 : 8) void forest_distanc
     }
 }
 
-template <int BLOCK, int LDS_N>
-__global__ __launch_bounds__(BLOCK) void ray_kernel(int64_t n, const float* __restrict__ rays_o,
-                                                    const float* __restrict__ rays_d, float* __restrict__ positions,
-                                                    int64_t* __restrict__ face_id, float* __restrict__ depth, Tree T) {
-    __shared__ int32_t s_ref[LDS_N * BLOCK];
-    __shared__ float s_key[LDS_N * BLOCK];
-    const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if (i >= n) return;
-    LaneStack<BLOCK, LDS_N> st;
-    st.ref = s_ref;
-    st.key = s_key;
-    st.tid = (int)threadIdx.x;
-    st.sp = 0;
-    const f3 o = load_pt(rays_o, i);
-    const f3 d = load_pt(rays_d, i);
-    float t;
-    int32_t slot = closest_hit(T, o, d, st, t);
-    depth[i] = t;
-    store_pt(positions, i, mk3(__builtin_fmaf(t, d.x, o.x), __builtin_fmaf(t, d.y, o.y), __builtin_fmaf(t, d.z, o.z)));
-    int64_t fid = -1;
-    if (slot >= 0) fid = (int64_t)__float_as_int(T.tris[3 * slot].w);
-    face_id[i] = fid;
-}
-
 // Rays in the caller's order, one wave per 64.  A wave whose rays are nearly parallel
 // and start close together (camera rays in pixel order: directions within ~5.7 degrees
 // of its first ray, origins within 1% of the scene's diagonal) walks as a packet;
@@ -1309,6 +1298,11 @@ uint32_t xcd_chunk_for(unsigned nb) {
 hipError_t launch_distance_impl(const QueryArgs& q, int mode) {
     const dev::Tree T = dev::make_tree(q.tree, q.face0_slot);
     hipStream_t s = (hipStream_t)q.stream;
+    if (mode != 2 && q.n < kWaveMax && !q.order) {
+        hipLaunchKernelGGL((mode == 0 ? dev::distance_wave_kernel<0> : dev::distance_wave_kernel<1>), dim3((unsigned)q.n),
+                           dim3(64), 0, s, q.in0, q.out_f, q.out_id, q.out_v, T);
+        return hipGetLastError();
+    }
     if ((mode == 0 || mode == 1) && q.packet) {
         constexpr int W = kDistanceWaves;
         const unsigned grid = (unsigned)((q.n + 64 * W - 1) / (64 * W));
@@ -1438,9 +1432,8 @@ hipError_t launch_ray(const QueryArgs& q) {
                            q.in1, q.order, q.out_v, q.out_id, q.out_f, T);
         return hipGetLastError();
     }
-    const unsigned grid = (unsigned)((q.n + kBlock - 1) / kBlock);
-    hipLaunchKernelGGL((dev::ray_kernel<kBlock, kLdsEntries>), dim3(grid), dim3(kBlock), 0, (hipStream_t)q.stream, q.n,
-                       q.in0, q.in1, q.out_v, q.out_id, q.out_f, T);
+    hipLaunchKernelGGL(dev::ray_wave_kernel, dim3((unsigned)q.n), dim3(64), 0, (hipStream_t)q.stream, q.in0, q.in1, q.out_v,
+                       q.out_id, q.out_f, T);
     return hipGetLastError();
 }
 

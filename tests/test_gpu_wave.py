@@ -1,0 +1,78 @@
+"""One wave per query (small calls) against packets of queries and the oracle.
+
+Calls below 2^18 queries walk one wave per query, larger ones as packets of 64 in Morton
+order; distance_ordered always walks packets.  Both have to give the oracle's bits, so
+each is held to the other bit for bit on inputs that the oracle tests also cover.
+"""
+import numpy as np
+import pytest
+import torch
+
+import cubvh_amd
+from cubvh_amd import synthetic as S
+
+pytestmark = pytest.mark.gpu
+
+WAVE_MAX = 1 << 18
+
+
+def _same(a, b):
+    """Equal bits, NaN included (+0 and -0 differ)."""
+    for x, y in zip(a, b):
+        assert x.dtype == y.dtype
+        if x.dtype == torch.float32:
+            x, y = x.view(torch.int32), y.view(torch.int32)
+        assert torch.equal(x, y)
+
+
+def _mesh(kind):
+    if kind == "copies":  # one face many times, all tied: more pending nodes than any real mesh
+        t = np.array([[0.1, 0.0, 0.0], [0.0, 0.1, 0.0], [0.0, 0.0, 0.1]], dtype=np.float32)
+        return np.tile(t, (3000, 1)), np.arange(9000, dtype=np.int32).reshape(-1, 3)
+    if kind == "flat":  # zero-area faces among the others
+        v, f = S.icosphere(4, 0.5)
+        f = f.copy()
+        f[::7, 1] = f[::7, 0]
+        return v, f
+    if kind == "nine":
+        v, f = S.icosphere(0, 0.5)
+        return v, f[:9]
+    return S.soup(5, seed=3, n_random=4000)
+
+
+def _points(n):
+    p = S.uniform_points(n, seed=n)
+    p[: n // 4] *= 0.05  # near the middle, where thousands of faces are about as far
+    special = np.array([[np.nan, 0, 0], [0, np.inf, 0], [np.nan] * 3, [2000, 0, 0], [0, 0, 0]], dtype=np.float32)
+    p[: min(n, 5)] = special[: min(n, 5)]
+    return torch.from_numpy(p).cuda()
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 2047, 30011])
+@pytest.mark.parametrize("kind", ["nine", "soup", "copies", "flat"])
+def test_wave_distance_equals_packets(gpu, kind, n):
+    v, f = _mesh(kind)
+    bvh = cubvh_amd.cuBVH(v, f)
+    p = _points(n)
+    order = torch.arange(n, dtype=torch.int32, device=gpu)
+    _same(bvh.unsigned_distance(p, return_uvw=True), bvh.distance_ordered(p, order, return_uvw=True))
+    _same(bvh.signed_distance(p)[:2], bvh.distance_ordered(p, order, signed=True)[:2])
+
+
+@pytest.mark.parametrize("kind", ["nine", "soup", "copies"])
+def test_wave_results_at_the_size_limit(gpu, kind):
+    """The same queries in one call at the limit (packets) and in two below it (waves)."""
+    v, f = _mesh(kind)
+    bvh = cubvh_amd.cuBVH(v, f)
+    n = WAVE_MAX if kind == "nine" else WAVE_MAX + 77
+    m = 30011 if kind == "copies" else n // 2
+    p = _points(n)
+    whole = bvh.unsigned_distance(p, return_uvw=True)
+    for part in (slice(0, m), slice(n - m, n)):
+        _same([t[part] for t in whole], bvh.unsigned_distance(p[part], return_uvw=True))
+    o, d = (torch.from_numpy(t).cuda() for t in S.sphere_rays(n, seed=5))
+    d[:3] = torch.tensor([[0.0, 0.0, 0.0], [float("nan"), 1.0, 0.0], [0.0, 0.0, 1.0]])
+    o[3:9] = torch.from_numpy(v[f[:6]].mean(axis=1)).cuda()  # origins on faces: hits at 0 and -0
+    hits = bvh.ray_trace(o, d)
+    for part in (slice(0, m), slice(n - m, n)):
+        _same([t[part] for t in hits], bvh.ray_trace(o[part], d[part]))
