@@ -363,10 +363,12 @@ int run_distance(cubvh_bvh* bvh, int device, int64_t n, int kmode, const float* 
         const size_t ob = ((size_t)n * 4 + 255) & ~(size_t)255;
         // raystab: the stab passes' lists after the order, the ordering workspace after them
         const size_t sb = kmode == 2 ? ((stab_workspace_bytes(n) + 255) & ~(size_t)255) : 0;
-        hipError_t e = hipMallocAsync(&scratch, ob + sb + morton_workspace_bytes(n), hs);
+        const size_t rb = rest_bytes(n);
+        hipError_t e = hipMallocAsync(&scratch, ob + sb + rb + morton_workspace_bytes(n), hs);
         if (e != hipSuccess) return fail_hip(e, "hipMallocAsync(query order)");
         uint32_t* order = (uint32_t*)scratch;
-        e = morton_order(n, positions, (char*)scratch + ob + sb, order, hs);
+        q.rest = (char*)scratch + ob + sb;
+        e = morton_order(n, positions, (char*)scratch + ob + sb + rb, order, hs);
         if (e != hipSuccess) {
             (void)hipFreeAsync(scratch, hs);
             return fail_hip(e, "query ordering");
@@ -771,10 +773,12 @@ int cubvh_unsigned_distance_noalloc(cubvh_bvh* bvh, int device, int64_t n, const
         hipError_t e = noalloc_scratch(device, &ws);
         if (e != hipSuccess) return fail_hip(e, "hipGetSymbolAddress(scratch)");
         const size_t ob = ((size_t)n * 4 + 255) & ~(size_t)255;
-        if (ob + morton_workspace_bytes(n) > kNoAllocScratchBytes)
+        const size_t rb = rest_bytes(n);
+        if (ob + rb + morton_workspace_bytes(n) > kNoAllocScratchBytes)
             return fail(CUBVH_ERR_STATE, "the ordering workspace does not fit the static scratch");
         uint32_t* order = (uint32_t*)ws;
-        e = morton_order(n, positions, (char*)ws + ob, order, hs);
+        q.rest = (char*)ws + ob;
+        e = morton_order(n, positions, (char*)ws + ob + rb, order, hs);
         if (e != hipSuccess) return fail_hip(e, "query ordering");
         q.order = order;
         q.packet = true;
@@ -863,7 +867,22 @@ int cubvh_distance_ordered(cubvh_bvh* bvh, int device, int64_t n, int32_t kind, 
     q.out_id = face_id;
     q.out_v = uvw;
     q.packet = true;
-    hipError_t e = launch_distance(q, kind);
+    // a captured call allocates nothing: its walks all run to their end
+    hipStream_t hs = (hipStream_t)stream;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(hs, &cs);
+    if (e != hipSuccess) return fail_hip(e, "hipStreamIsCapturing");
+    if (cs == hipStreamCaptureStatusNone && n < kRestLast) {
+        rc = ensure_pool(device);
+        if (rc != CUBVH_OK) return rc;
+        e = hipMallocAsync(&q.rest, rest_bytes(n), hs);
+        if (e != hipSuccess) return fail_hip(e, "hipMallocAsync(rest of the walks)");
+    }
+    e = launch_distance(q, kind);
+    if (q.rest) {
+        const hipError_t e2 = hipFreeAsync(q.rest, hs);
+        if (e == hipSuccess) e = e2;
+    }
     if (e != hipSuccess) return fail_hip(e, "distance kernel launch");
     return CUBVH_OK;
     CUBVH_GUARD_END
@@ -902,9 +921,11 @@ int cubvh_ray_trace(cubvh_bvh* bvh, int device, int64_t n, const float* rays_o, 
         rc = ensure_pool(device);
         if (rc != CUBVH_OK) return rc;
         const size_t ob = ((size_t)n * 4 + 255) & ~(size_t)255;
-        hipError_t e = hipMallocAsync(&scratch, ob + morton_workspace_bytes(n), hs);
+        const size_t rb = rest_bytes(n);
+        hipError_t e = hipMallocAsync(&scratch, ob + rb + morton_workspace_bytes(n), hs);
         if (e != hipSuccess) return fail_hip(e, "hipMallocAsync(ray order)");
-        e = ray_order(n, rays_o, rays_d, (char*)scratch + ob, (uint32_t*)scratch, hs);
+        q.rest = (char*)scratch + ob;
+        e = ray_order(n, rays_o, rays_d, (char*)scratch + ob + rb, (uint32_t*)scratch, hs);
         if (e != hipSuccess) {
             (void)hipFreeAsync(scratch, hs);
             return fail_hip(e, "ray ordering");

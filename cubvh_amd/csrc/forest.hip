@@ -203,7 +203,7 @@ size_t forest_workspace_bytes(int64_t n, int32_t n_meshes, int32_t bits) {
     const int64_t nbins = (int64_t)n_meshes << bits;
     const int64_t nchunks = (nbins + 1023) / 1024;
     return al(64) + al(64) + al(8 * (size_t)(n_meshes + 1)) + al(4 * (size_t)npad) + 2 * al(4 * (size_t)n) +
-           al(4 * (size_t)nbins) + al(4 * (size_t)nchunks);
+           al(4 * (size_t)nbins) + al(4 * (size_t)nchunks) + rest_bytes(npad);
 }
 
 ForestWorkspace carve_forest_workspace(void* ws, int64_t n, int32_t n_meshes, int32_t bits) {
@@ -228,6 +228,8 @@ ForestWorkspace carve_forest_workspace(void* ws, int64_t n, int32_t n_meshes, in
     f.hist = (uint32_t*)w;
     w += al(4 * (size_t)nbins);
     f.sums = (uint32_t*)w;
+    w += al(4 * (size_t)nchunks);
+    f.rest = w;
     f.npad_max = npad;
     f.nbins = nbins;
     f.nchunks = nchunks;

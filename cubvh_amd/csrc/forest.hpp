@@ -18,6 +18,7 @@ struct ForestWorkspace {
     uint32_t* rank = nullptr;    // [n]
     uint32_t* hist = nullptr;    // [nbins] counts, then exclusive scan inside chunks
     uint32_t* sums = nullptr;    // [nchunks]
+    void* rest = nullptr;        // queries of given-up walks, of npad_max
     int64_t npad_max = 0, nbins = 0, nchunks = 0;
 };
 

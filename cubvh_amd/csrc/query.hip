@@ -252,9 +252,10 @@ __device__ __forceinline__ f3 ray_inverse(f3 d) {
     return mk3(1.0f / x, 1.0f / y, 1.0f / z);
 }
 
-// Closest hit.  Returns the leaf slot (-1 on a miss) and t in best_t.
+// Closest hit.  Returns the leaf slot (-1 on a miss) and t in best_t; budget is left
+// negative by a walk that has more to visit after that many steps (nodes and faces).
 template <int BLOCK, int LDS_N>
-__device__ int32_t closest_hit(const Tree& T, f3 o, f3 d, LaneStack<BLOCK, LDS_N>& st, float& best_t) {
+__device__ int32_t closest_hit(const Tree& T, f3 o, f3 d, LaneStack<BLOCK, LDS_N>& st, float& best_t, int32_t& budget) {
     f3 inv = ray_inverse(d);
     float best = MAX_DIST;
     float bound = MAX_DIST * BOUND_SLACK;
@@ -262,6 +263,7 @@ __device__ int32_t closest_hit(const Tree& T, f3 o, f3 d, LaneStack<BLOCK, LDS_N
     int32_t ref = 0;
     st.sp = 0;
     for (;;) {
+        --budget;
         if (ref >= 0) {
             WideNode nd = load_node(T.nodes, ref);
             float k[4];
@@ -278,6 +280,7 @@ __device__ int32_t closest_hit(const Tree& T, f3 o, f3 d, LaneStack<BLOCK, LDS_N
         } else {
             int32_t first, count;
             leaf_range(ref, first, count);
+            budget -= count;
             for (int j = 0; j < count; ++j) {
                 f3 a, b, c;
                 int32_t id;
@@ -299,7 +302,11 @@ __device__ int32_t closest_hit(const Tree& T, f3 o, f3 d, LaneStack<BLOCK, LDS_N
                 break;
             }
         }
-        if (ref == CHILD_EMPTY) break;
+        if (ref == CHILD_EMPTY) {
+            budget = 0;
+            break;
+        }
+        if (budget < 0) break;
     }
     best_t = best;
     return bslot;
@@ -532,6 +539,14 @@ struct WaveStack {
         mhi = here ? (int32_t)(uint32_t)(m >> 32) : mhi;
         ++sp;
     }
+    // the lanes that some entry is held for
+    __device__ __forceinline__ uint64_t lanes() const {
+        uint64_t m = 0;
+        for (int e = 0; e < sp; ++e)
+            m |= (uint64_t)(uint32_t)__builtin_amdgcn_readlane(mlo, e) |
+                 ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(mhi, e) << 32);
+        return m;
+    }
     __device__ __forceinline__ bool pop(int32_t& r, uint64_t& m) {
         if (sp == 0) return false;
         --sp;
@@ -620,26 +635,95 @@ __device__ __forceinline__ void run_exact(const Tree& T, ExactQueue& q, int32_t&
     wave_fence();
 }
 
+// Queries and rays whose walk, shared with 63 others, used up its budget of steps.  A tile
+// whose queries lie far apart visits the union of 64 unlike walks, one dependent load
+// after another: on 2^20 normal points the slowest tile took 3.8 ms where the average took
+// 0.25 ms, and a call lasts as long as its slowest tile.  Such a tile hands its unfinished
+// queries over to a later launch that gives each a wave of its own.
+struct PacketRest {
+    uint32_t count, cap;
+    uint32_t factor;  // a walk ends after factor / 16 times the average walk's steps
+    uint32_t tiles;   // sampled walks that have ended, and their steps
+    unsigned long long steps;
+    uint32_t pad[58];  // the list follows: (query, best so far bits, its face slot, root)
+    __host__ __device__ int4* list() const { return (int4*)(this + 1); }
+};
+static_assert(sizeof(PacketRest) == 256, "the list is 256-byte aligned");
+constexpr int32_t kFirstCheck = 512;  // steps before a walk is compared with the average
+
+// Steps at which a walk of `steps` steps ends, or is looked at again, from the walks that
+// have ended so far.
+__device__ __forceinline__ int32_t step_limit(const PacketRest* rest, int32_t steps) {
+    const uint32_t n = __hip_atomic_load(&rest->tiles, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (n < 16) return steps + kFirstCheck / 4;  // too few to tell
+    const unsigned long long s = __hip_atomic_load(&rest->steps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return uniform((int32_t)min((s * rest->factor) / (16ull * n), (unsigned long long)INT32_MAX));
+}
+
+// Every 16th walk reports its steps (all of them would queue on one address).
+__device__ __forceinline__ void report_steps(PacketRest* rest, int64_t tile, int32_t steps) {
+    if ((tile & 15) == 0 && (threadIdx.x & 63) == 0) {
+        atomicAdd(&rest->steps, (unsigned long long)steps);
+        atomicAdd(&rest->tiles, 1u);
+    }
+}
+
+__global__ void rest_init(PacketRest* rest, uint32_t cap, uint32_t factor) {
+    if (threadIdx.x == 0) {
+        rest->count = rest->tiles = 0;
+        rest->steps = 0;
+        rest->cap = cap;
+        rest->factor = factor;
+    }
+}
+
+// Room for the lanes in `left`: their first place in the list, or -1 when it is full
+// (places taken all the same are marked empty).
+__device__ __forceinline__ int32_t reserve_rest(PacketRest* rest, uint64_t left) {
+    const uint32_t lane = threadIdx.x & 63, c = (uint32_t)__builtin_popcountll(left), cap = rest->cap;
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(&rest->count, c);
+    base = (uint32_t)uniform((int32_t)base);
+    if (base + c <= cap) return (int32_t)base;
+    if (lane < c && base + lane < cap) rest->list()[base + lane] = make_int4(-1, 0, 0, 0);
+    return -1;
+}
+
+// Writes the lane's query (lane in `left`) to the list.
+__device__ __forceinline__ void leave_rest(PacketRest* rest, uint64_t left, int32_t base, int64_t q, float best,
+                                           int32_t slot, int32_t root) {
+    if ((left >> (threadIdx.x & 63)) & 1)
+        rest->list()[base + (int32_t)lanes_below(left)] =
+            make_int4((int32_t)(uint32_t)q, __float_as_int(best), slot, root);
+}
+
 // A leaf wanted by more lanes than this is tested one face at a time (a round of 64
 // pairs per face would cost more than the step); fewer lanes are packed into rounds.
 constexpr int kStepLanes = 32;
 
 // Nearest face for every lane of the wave (lanes with active = false only ride
 // along).  Results in the lane's best / bslot / bid, as closest_face.  q is this
-// wave's own LDS queue.
-__device__ void closest_face_packet(const Tree& T, int32_t root, f3 p, bool active, float& best, int32_t& bslot,
-                                    int32_t& bid, ExactQueue& q) {
+// wave's own LDS queue.  A walk of many more steps (nodes, leaves, four dense faces,
+// rounds: each about one memory latency) than the average ends early, with REST, if `rest`
+// has room (places from `base`) for the lanes that have subtrees left, which it returns.
+template <bool REST>
+__device__ uint64_t closest_face_packet(const Tree& T, int32_t root, f3 p, bool active, float& best, int32_t& bslot,
+                                        int32_t& bid, ExactQueue& q, PacketRest* rest, int64_t tile,
+                                        int32_t& base) {
     const int lane = (int)(threadIdx.x & 63);
     best = MAX_DIST_SQ;
     float bound = MAX_DIST_SQ * BOUND_SLACK;
     bslot = -1;
     bid = 0x7fffffff;
     uint64_t mask = ballot(active && !has_nan(p));
-    if (mask == 0) return;
+    if (mask == 0) return 0;
     WaveStack st;
     int32_t qn = 0;  // queued pairs (wave-uniform)
     int32_t ref = uniform(root);
+    uint64_t left = 0;
+    int32_t steps = 0, check = kFirstCheck;
     for (;;) {
+        ++steps;
         if (ref >= 0) {
             UNode nd = load_unode(T.nodes, ref);
             // every lane computes; the uniform lane mask selects the interested ones
@@ -680,6 +764,7 @@ __device__ void closest_face_packet(const Tree& T, int32_t root, f3 p, bool acti
             const uint64_t lm = ballot(!disk_rejects(p, ld4(lp), ld4(lp + 4), bound)) & mask;
             if (__builtin_popcountll(lm) > kStepLanes) {
                 // most lanes want the leaf: one step per face, face records uniform
+                steps += count >> 2;
                 for (int j = 0; j < count; ++j) {
                     cfloat_ptr bp = (cfloat_ptr)(T.tbnd + 2 * (first + j));
                     const uint64_t cm = ballot(!disk_rejects(p, ld4(bp), ld4(bp + 4), bound)) & lm;
@@ -691,6 +776,7 @@ __device__ void closest_face_packet(const Tree& T, int32_t root, f3 p, bool acti
                     }
                     qn += __builtin_popcountll(cm);
                     if (qn >= 64) {
+                        ++steps;
                         wave_fence();
                         run_exact(T, q, qn, p, best, bound, bslot, bid);
                     }
@@ -717,6 +803,7 @@ __device__ void closest_face_packet(const Tree& T, int32_t root, f3 p, bool acti
                         const float4* bp = T.tbnd + 2 * (first + j);
                         pass = !disk_rejects(ps, bp[0], bp[1], bs);
                     }
+                    ++steps;
                     const uint64_t pm = ballot(pass);
                     if (pass) {
                         const uint32_t at = (uint32_t)qn + lanes_below(pm);
@@ -725,6 +812,7 @@ __device__ void closest_face_packet(const Tree& T, int32_t root, f3 p, bool acti
                     }
                     qn += __builtin_popcountll(pm);
                     if (qn >= 64) {
+                        ++steps;
                         wave_fence();
                         run_exact(T, q, qn, p, best, bound, bslot, bid);
                     }
@@ -734,16 +822,31 @@ __device__ void closest_face_packet(const Tree& T, int32_t root, f3 p, bool acti
         }
         if (!st.pop(ref, mask)) break;
         ref = uniform(ref);
+        if (REST && steps >= check) {
+            check = step_limit(rest, steps);
+            if (steps >= check) {
+                left = mask | st.lanes();
+                base = reserve_rest(rest, left);
+                if (base >= 0) break;
+                left = 0;
+                check = INT32_MAX;  // no room: this wave walks to the end
+            }
+        }
     }
     if (qn > 0) {
         wave_fence();
         run_exact(T, q, qn, p, best, bound, bslot, bid);
     }
+    if (REST) report_steps(rest, tile, steps);
+    return left;
 }
 
 // Packet form of closest_hit: every lane traces its own ray; node and face records
 // are wave-uniform.  Children are ordered by the entry distance of their lowest
-// interested lane.  Results (t, slot, id) as closest_hit.
+// interested lane.  Results (t, slot, id) as closest_hit; a walk of more than kRaySteps
+// steps (nodes and faces) ends early, with rest, base and the return value as
+// closest_face_packet's.
+constexpr int32_t kRaySteps = 2000;
 __device__ __forceinline__ float slab_entry(float lx, float hx, float ly, float hy, float lz, float hz, f3 o, f3 inv) {
     const float tx0 = (lx - o.x) * inv.x, tx1 = (hx - o.x) * inv.x;
     const float ty0 = (ly - o.y) * inv.y, ty1 = (hy - o.y) * inv.y;
@@ -753,19 +856,21 @@ __device__ __forceinline__ float slab_entry(float lx, float hx, float ly, float 
     return (tn <= tf && tf >= 0.0f) ? tn : INFINITY;
 }
 
-__device__ void closest_hit_packet(const Tree& T, f3 o, f3 d, bool active, float& best, int32_t& bslot,
-                                   int32_t& bid) {
+__device__ uint64_t closest_hit_packet(const Tree& T, f3 o, f3 d, bool active, float& best, int32_t& bslot,
+                                       int32_t& bid, PacketRest* rest, int32_t& base) {
     const int lane = (int)(threadIdx.x & 63);
     const f3 inv = ray_inverse(d);
     best = MAX_DIST;
     float bound = MAX_DIST * BOUND_SLACK;
     bslot = -1;
     bid = 0x7fffffff;
-    uint64_t mask = ballot(active);
-    if (mask == 0) return;
+    uint64_t mask = ballot(active), left = 0;
+    if (mask == 0) return 0;
     WaveStack st;
     int32_t ref = 0;
+    int32_t budget = rest ? kRaySteps : INT32_MAX;
     for (;;) {
+        --budget;
         if (ref >= 0) {
             UNode nd = load_unode(T.nodes, ref);
             float k0 = nd.child.x != CHILD_EMPTY ? slab_entry(nd.lx.x, nd.hx.x, nd.ly.x, nd.hy.x, nd.lz.x, nd.hz.x, o, inv) : INFINITY;
@@ -797,6 +902,7 @@ __device__ void closest_hit_packet(const Tree& T, f3 o, f3 d, bool active, float
         } else {
             int32_t first, count;
             leaf_range(ref, first, count);
+            budget -= count;
             for (int j = 0; j < count; ++j) {
                 f3 a, b, c;
                 int32_t id;
@@ -814,7 +920,15 @@ __device__ void closest_hit_packet(const Tree& T, f3 o, f3 d, bool active, float
         }
         if (!st.pop(ref, mask)) break;
         ref = uniform(ref);
+        if (budget < 0) {
+            left = mask | st.lanes();
+            base = reserve_rest(rest, left);
+            if (base >= 0) break;
+            left = 0;
+            budget = INT32_MAX;  // no room: this wave walks to the end
+        }
     }
+    return left;
 }
 
 __device__ __forceinline__ f3 load_pt(const float* __restrict__ p, int64_t i) {
@@ -824,6 +938,20 @@ __device__ __forceinline__ void store_pt(float* __restrict__ p, int64_t i, f3 v)
     p[3 * i] = v.x;
     p[3 * i + 1] = v.y;
     p[3 * i + 2] = v.z;
+}
+
+// Workgroup b of a launch runs on XCD b % 8: the dispatcher deals workgroups round-robin
+// over the 8 XCDs, each with its own L2.  xcd_remap gives workgroup b the logical block
+// it works on so that each XCD takes runs of `chunk` consecutive logical blocks (within
+// every group of 8 chunk workgroups; a last partial group keeps its order): neighbouring
+// tiles, which walk the same part of a tree, then share one L2 instead of eight.  A
+// bijection of [0, nb), so every tile is still walked once.
+__device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb, uint32_t chunk) {
+    if (chunk == 0) return b;
+    const uint32_t group = 8u * chunk;
+    if (b >= nb / group * group) return b;
+    const uint32_t r = b % group;
+    return b - r + (r % 8u) * chunk + r / 8u;
 }
 
 }  // namespace dev
@@ -887,20 +1015,6 @@ __global__ __launch_bounds__(BLOCK) void distance_kernel(int64_t n, const float*
         f3 cp = tri_closest_pt(a, b, c, p);
         store_pt(uvw, i, tri_barycentric(a, b, c, cp));
     }
-}
-
-// Workgroup b of a launch runs on XCD b % 8: the dispatcher deals workgroups round-robin
-// over the 8 XCDs, each with its own L2.  xcd_remap gives workgroup b the logical block
-// it works on so that each XCD takes runs of `chunk` consecutive logical blocks (within
-// every group of 8 chunk workgroups; a last partial group keeps its order): neighbouring
-// tiles, which walk the same part of a tree, then share one L2 instead of eight.  A
-// bijection of [0, nb), so every tile is still walked once.
-__device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb, uint32_t chunk) {
-    if (chunk == 0) return b;
-    const uint32_t group = 8u * chunk;
-    if (b >= nb / group * group) return b;
-    const uint32_t r = b % group;
-    return b - r + (r % 8u) * chunk + r / 8u;
 }
 
 // Raystab sign of distances already computed (src/bvh.cu:408-427): a query is inside,
@@ -1101,28 +1215,14 @@ __global__ __launch_bounds__(256) void stab_negate(const uint32_t* __restrict__ 
 
 constexpr int kNormalLds = 4;  // LDS entries per lane of the per-lane normal search
 
-// Packet kernel for the unsigned (MODE 0) and watertight signed (MODE 1) distance, WAVES
-// waves per workgroup.  Workgroup b walks tile xcd_remap(b) (runs of xchunk consecutive
-// tiles of the Morton order per XCD); its lane i handles query order[64 tile + i] (or
-// that index without a permutation).
+// Writes query q's outputs from its nearest face (slot < 0: none within MAX_DIST, which
+// reports distance 0 to face 0).  Lanes with valid = false write nothing.
 template <int MODE, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, 8) void distance_packet_kernel(int64_t n, const float* __restrict__ positions,
-                                                              const uint32_t* __restrict__ order,
-                                                              float* __restrict__ distances,
-                                                              int64_t* __restrict__ face_id, float* __restrict__ uvw,
-                                                              Tree T, uint32_t xchunk) {
-    const int64_t i = (int64_t)xcd_remap(blockIdx.x, gridDim.x, xchunk) * (64 * WAVES) + threadIdx.x;
-    int64_t q = i;
-    if (i < n && order) q = (int64_t)order[i];
-    const bool valid = i < n && q < n;  // order entries >= n are skipped
-    f3 p = mk3(0.0f, 0.0f, 0.0f);
-    if (valid) p = load_pt(positions, q);
-    float d2;
-    int32_t slot, bid;
-    __shared__ ExactQueue queues[WAVES];
-    closest_face_packet(T, 0, p, valid, d2, slot, bid, queues[threadIdx.x >> 6]);
-    if (slot < 0) {  // nothing within MAX_DIST: distance 0 and face 0
-        slot = (int32_t)T.face0_slot;
+__device__ __forceinline__ void finish_query(const Tree& T, int32_t face0_slot, bool valid, int64_t q, f3 p, float d2,
+                                             int32_t slot, float* __restrict__ distances,
+                                             int64_t* __restrict__ face_id, float* __restrict__ uvw) {
+    if (slot < 0) {
+        slot = face0_slot;
         d2 = 0.0f;
     }
     f3 a, b, c;
@@ -1155,6 +1255,33 @@ __global__ __launch_bounds__(64 * WAVES, 8) void distance_packet_kernel(int64_t 
     if (uvw) store_pt(uvw, q, tri_barycentric(a, b, c, cp));
 }
 
+// Packet kernel for the unsigned (MODE 0) and watertight signed (MODE 1) distance, WAVES
+// waves per workgroup.  Workgroup b walks tile xcd_remap(b) (runs of xchunk consecutive
+// tiles of the Morton order per XCD); its lane i handles query order[64 tile + i] (or
+// that index without a permutation).  The queries of walks given up go to `rest`.
+template <int MODE, int WAVES, bool REST>
+__global__ __launch_bounds__(64 * WAVES, 8) void distance_packet_kernel(int64_t n, const float* __restrict__ positions,
+                                                              const uint32_t* __restrict__ order,
+                                                              float* __restrict__ distances,
+                                                              int64_t* __restrict__ face_id, float* __restrict__ uvw,
+                                                              Tree T, uint32_t xchunk,
+                                                              PacketRest* rest) {
+    const int64_t i = (int64_t)xcd_remap(blockIdx.x, gridDim.x, xchunk) * (64 * WAVES) + threadIdx.x;
+    int64_t q = i;
+    if (i < n && order) q = (int64_t)order[i];
+    const bool valid = i < n && q < n;  // order entries >= n are skipped
+    f3 p = mk3(0.0f, 0.0f, 0.0f);
+    if (valid) p = load_pt(positions, q);
+    float d2;
+    int32_t slot, bid, base;
+    __shared__ ExactQueue queues[WAVES];
+    const uint64_t left =
+        closest_face_packet<REST>(T, 0, p, valid, d2, slot, bid, queues[threadIdx.x >> 6], rest, i >> 6, base);
+    if (REST && left != 0) leave_rest(rest, left, base, q, d2, slot >= 0 ? slot : ~(int32_t)T.face0_slot, 0);
+    const bool mine = valid && !(REST && ((left >> (threadIdx.x & 63)) & 1));
+    finish_query<MODE, WAVES>(T, (int32_t)T.face0_slot, mine, q, p, d2, slot, distances, face_id, uvw);
+}
+
 // Unsigned distance over a forest: one wave per 64-slot tile of the padded query
 // order; every tile belongs to one mesh, whose root node and face-0 slot come from
 // mesh_info.  PERSISTENT waves take tiles from an atomic counter until none is left.
@@ -1166,7 +1293,7 @@ __global__ __launch_bounds__(64 * WAVES, PERSISTENT ? 7 : 8) void forest_distanc
                                                               float* __restrict__ distances,
                                                               int64_t* __restrict__ face_id, float* __restrict__ uvw,
                                                               TreeArrays arrays, uint32_t* counter,
-                                                              int64_t max_tiles, uint32_t xcd_chunk) {
+                                                              int64_t max_tiles, uint32_t xcd_chunk, PacketRest* rest) {
     __shared__ ExactQueue queues[WAVES];
     const int lane = (int)(threadIdx.x & 63);
     // max_tiles: the tiles the order array holds (bounds the walk even when the offsets
@@ -1195,20 +1322,15 @@ __global__ __launch_bounds__(64 * WAVES, PERSISTENT ? 7 : 8) void forest_distanc
         if (valid) p = load_pt(positions, qi);
         const Tree T = make_tree(arrays, (int64_t)mi.y);
         float d2;
-        int32_t slot, bid;
-        closest_face_packet(T, uniform(mi.x), p, valid, d2, slot, bid, queues[threadIdx.x >> 6]);
-        if (valid) {
-            if (slot < 0) {
-                slot = mi.y;
-                d2 = 0.0f;
-            }
-            f3 a, b, c;
-            int32_t id;
-            load_tri(T.tris, slot, a, b, c, id);
-            distances[qi] = sqrtf(d2);
-            face_id[qi] = (int64_t)id;
-            if (uvw) store_pt(uvw, qi, tri_barycentric(a, b, c, tri_closest_pt(a, b, c, p)));
-        }
+        int32_t slot, bid, base;
+        const uint64_t left = closest_face_packet<true>(T, uniform(mi.x), p, valid, d2, slot, bid, queues[threadIdx.x >> 6],
+                                                  rest, tile, base);
+        if (left != 0) leave_rest(rest, left, base, (int64_t)qi, d2, slot >= 0 ? slot : ~mi.y, mi.x);
+        const bool mine = valid && !((left >> lane) & 1);
+        finish_query<0, WAVES>(T, mi.y, mine, (int64_t)qi, p, d2, slot, distances, face_id, uvw);
+        // One back edge: without it the compiler may thread a lane test at the loop's end
+        // to the one at its start, sending some lanes around without lane 0.
+        __builtin_amdgcn_wave_barrier();
         if (!PERSISTENT) return;
     }
 }
@@ -1218,12 +1340,13 @@ __global__ __launch_bounds__(64 * WAVES, PERSISTENT ? 7 : 8) void forest_distanc
 // of its first ray, origins within 1% of the scene's diagonal) walks as a packet;
 // any other wave walks lane by lane.  Both give closest_hit's results.
 constexpr int kRayLds = 8;
+constexpr int32_t kLaneSteps = 512;  // steps of a lane's walk before a wave takes over
 template <int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void ray_packet_kernel(int64_t n, const float* __restrict__ rays_o,
+__global__ __launch_bounds__(64 * WAVES, 8) void ray_packet_kernel(int64_t n, const float* __restrict__ rays_o,
                                                          const float* __restrict__ rays_d,
                                                          const uint32_t* __restrict__ order,
                                                          float* __restrict__ positions, int64_t* __restrict__ face_id,
-                                                         float* __restrict__ depth, Tree T) {
+                                                         float* __restrict__ depth, Tree T, PacketRest* rest) {
     __shared__ int32_t s_ref[kRayLds * 64 * WAVES];
     __shared__ float s_key[kRayLds * 64 * WAVES];
     const int64_t g = (int64_t)blockIdx.x * (64 * WAVES) + threadIdx.x;
@@ -1254,20 +1377,27 @@ __global__ __launch_bounds__(64 * WAVES) void ray_packet_kernel(int64_t n, const
     const float dd = dot3(d, d0), n2 = dot3(d, d) * dot3(d0, d0);
     const bool near = !valid || (dd > 0.0f && dd * dd >= 0.99f * n2 && dot3(od, od) <= 1e-4f * diag2);
     float t;
-    int32_t slot, bid;
+    int32_t slot = -1, bid = 0, base = -1;
+    uint64_t left;
     if (ballot(near) == ~0ull) {
-        closest_hit_packet(T, o, d, valid, t, slot, bid);
+        left = closest_hit_packet(T, o, d, valid, t, slot, bid, rest, base);
     } else {
-        if (!valid) return;
         LaneStack<64 * WAVES, kRayLds> st;
         st.ref = s_ref;
         st.key = s_key;
         st.tid = (int)threadIdx.x;
-        st.sp = 0;
-        slot = closest_hit(T, o, d, st, t);
-        bid = slot >= 0 ? __float_as_int(T.tris[3 * slot].w) : 0;
+        for (int32_t budget = rest ? kLaneSteps : INT32_MAX;; budget = INT32_MAX) {
+            int32_t b = valid ? budget : 0;
+            if (valid) slot = closest_hit(T, o, d, st, t, b);
+            left = ballot(b < 0);
+            if (left == 0) break;
+            base = reserve_rest(rest, left);
+            if (base >= 0) break;  // else no room: the wave walks to the end
+        }
+        if (slot >= 0) bid = __float_as_int(T.tris[3 * slot].w);
     }
-    if (!valid) return;
+    if (left != 0) leave_rest(rest, left, base, i, t, slot, 0);
+    if (!valid || ((left >> (threadIdx.x & 63)) & 1)) return;
     depth[i] = t;
     store_pt(positions, i, mk3(__builtin_fmaf(t, d.x, o.x), __builtin_fmaf(t, d.y, o.y), __builtin_fmaf(t, d.z, o.z)));
     face_id[i] = slot >= 0 ? (int64_t)bid : -1;
@@ -1284,6 +1414,7 @@ constexpr int kLdsEntries = 12;
 // with 4 and 13.47 with 8; the watertight SDF 889 against 868 Mq/s; camera rays 3119
 // against 2899 Mrays/s).
 constexpr int kDistanceWaves = 1;
+constexpr uint32_t kRestBlocks = 8192;  // one-wave workgroups of a rest launch: what the chip holds at once
 
 // Runs of consecutive workgroups per XCD for a grid of nb one-wave workgroups over a
 // Morton order: the largest power of two <= nb / 128, so that each XCD's L2 serves one
@@ -1293,6 +1424,21 @@ uint32_t xcd_chunk_for(unsigned nb) {
     uint32_t c = 1;
     while ((uint64_t)c * 2 * 128 <= nb) c *= 2;
     return nb >= 128 * 8 ? c : 0u;
+}
+
+uint32_t rest_cap(int64_t n) { return (uint32_t)std::min<int64_t>(n, kRestMax); }
+
+// A call of n queries hands over the walks of more than `least` times the average steps.  A
+// long walk does not matter when many more rounds of tiles follow, and a wave per query
+// costs several times a packet's share, so the factor grows with the rounds of tiles the
+// chip takes (measured at 2^20 normal points on 81,920 faces: 1.31 ms with 2, 1.29 with 2.5,
+// 1.33 with 3, 1.73 with 6, 3.06 without; 2^23 uniform points on 1.3 M faces: 9.0 ms with
+// slope 0.3, 9.9 with 0.6, 13.6 without).  The watertight sign needs more of a walk's wave:
+// 2^21 grid points on 327,680 faces 2.83 ms with 2, 2.40 with 3, 2.37 with 4, 2.58 with 6.
+void launch_rest_init(dev::PacketRest* rest, int64_t n, double least, hipStream_t s) {
+    const double rounds = (double)n / (64.0 * kRestBlocks);
+    const uint32_t factor = (uint32_t)(16.0 * std::max(least, 0.4 * rounds));
+    hipLaunchKernelGGL(dev::rest_init, dim3(1), dim3(64), 0, s, rest, rest_cap(n), factor);
 }
 
 hipError_t launch_distance_impl(const QueryArgs& q, int mode) {
@@ -1307,12 +1453,16 @@ hipError_t launch_distance_impl(const QueryArgs& q, int mode) {
         constexpr int W = kDistanceWaves;
         const unsigned grid = (unsigned)((q.n + 64 * W - 1) / (64 * W));
         const uint32_t xchunk = xcd_chunk_for(grid);
-        if (mode == 0)
-            hipLaunchKernelGGL((dev::distance_packet_kernel<0, W>), dim3(grid), dim3(64 * W), 0, s, q.n, q.in0, q.order,
-                               q.out_f, q.out_id, q.out_v, T, xchunk);
-        else
-            hipLaunchKernelGGL((dev::distance_packet_kernel<1, W>), dim3(grid), dim3(64 * W), 0, s, q.n, q.in0, q.order,
-                               q.out_f, q.out_id, q.out_v, T, xchunk);
+        dev::PacketRest* rest = (dev::PacketRest*)q.rest;
+        if (q.n >= kRestLast) rest = nullptr;
+        if (rest) launch_rest_init(rest, q.n, mode == 0 ? 2.5 : 3.5, s);
+        const auto kernel = mode == 0 ? (rest ? dev::distance_packet_kernel<0, W, true> : dev::distance_packet_kernel<0, W, false>)
+                                      : (rest ? dev::distance_packet_kernel<1, W, true> : dev::distance_packet_kernel<1, W, false>);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), 0, s, q.n, q.in0, q.order, q.out_f, q.out_id, q.out_v, T, xchunk, rest);
+        if (rest)
+            hipLaunchKernelGGL((mode == 0 ? dev::distance_rest_kernel<0> : dev::distance_rest_kernel<1>),
+                               dim3(std::min<uint32_t>(rest_cap(q.n), kRestBlocks)), dim3(64), 0, s, rest, q.in0, q.out_f, q.out_id,
+                               q.out_v, T);
         return hipGetLastError();
     }
     const unsigned grid = (unsigned)((q.n + kBlock - 1) / kBlock);
@@ -1341,17 +1491,21 @@ namespace {
 template <int WAVES>
 hipError_t launch_forest_shape(const ForestArgs& a, const ForestWorkspace& ws, hipStream_t s) {
     const int64_t max_tiles = ws.npad_max / 64;
+    dev::PacketRest* rest = (dev::PacketRest*)ws.rest;
+    launch_rest_init(rest, ws.npad_max, 2.5, s);
     if (a.persistent) {
         const unsigned blocks = (unsigned)std::max(1, a.n_cu * a.waves_per_cu / WAVES);
         hipLaunchKernelGGL((dev::forest_distance_kernel<1, WAVES>), dim3(blocks), dim3(64 * WAVES), 0, s, a.positions,
                            ws.order, ws.pbase, a.n_meshes, a.mesh_info, a.distances, a.face_id, a.uvw, a.tree,
-                           ws.counter, max_tiles, 0u);
+                           ws.counter, max_tiles, 0u, rest);
     } else {
         const unsigned blocks = (unsigned)((max_tiles + WAVES - 1) / WAVES);
         hipLaunchKernelGGL((dev::forest_distance_kernel<0, WAVES>), dim3(blocks), dim3(64 * WAVES), 0, s, a.positions,
                            ws.order, ws.pbase, a.n_meshes, a.mesh_info, a.distances, a.face_id, a.uvw, a.tree,
-                           ws.counter, max_tiles, (uint32_t)a.xcd_chunk);
+                           ws.counter, max_tiles, (uint32_t)a.xcd_chunk, rest);
     }
+    hipLaunchKernelGGL(dev::distance_rest_kernel<0>, dim3(std::min<uint32_t>(rest_cap(ws.npad_max), kRestBlocks)), dim3(64), 0, s, rest,
+                       a.positions, a.distances, a.face_id, a.uvw, dev::make_tree(a.tree, 0));
     return hipGetLastError();
 }
 
@@ -1367,6 +1521,8 @@ hipError_t launch_forest_distance(const ForestArgs& a, const ForestWorkspace& ws
         default: return hipErrorInvalidValue;
     }
 }
+
+size_t rest_bytes(int64_t n) { return (sizeof(dev::PacketRest) + 16 * (size_t)rest_cap(n) + 255) & ~(size_t)255; }
 
 int stack_capacity_for(int need) { return need <= dev::STACK_TOTAL ? dev::STACK_TOTAL : -1; }
 
@@ -1428,8 +1584,14 @@ hipError_t launch_ray(const QueryArgs& q) {
         // no runs per XCD here: ray costs differ between image regions, and runs put the
         // costly ones on one XCD (camera rays 2475 Mrays/s with the distance kernels' runs)
         const unsigned grid = (unsigned)((q.n + 64 * W - 1) / (64 * W));
-        hipLaunchKernelGGL(dev::ray_packet_kernel<W>, dim3(grid), dim3(64 * W), 0, (hipStream_t)q.stream, q.n, q.in0,
-                           q.in1, q.order, q.out_v, q.out_id, q.out_f, T);
+        hipStream_t s = (hipStream_t)q.stream;
+        dev::PacketRest* rest = (dev::PacketRest*)q.rest;
+        if (rest) launch_rest_init(rest, q.n, 1.0, s);
+        hipLaunchKernelGGL(dev::ray_packet_kernel<W>, dim3(grid), dim3(64 * W), 0, s, q.n, q.in0, q.in1, q.order, q.out_v,
+                           q.out_id, q.out_f, T, rest);
+        if (rest)
+            hipLaunchKernelGGL(dev::ray_rest_kernel, dim3(std::min<uint32_t>(rest_cap(q.n), kRestBlocks)), dim3(64), 0, s, rest, q.in0,
+                               q.in1, q.out_v, q.out_id, q.out_f, T);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(dev::ray_wave_kernel, dim3((unsigned)q.n), dim3(64), 0, (hipStream_t)q.stream, q.in0, q.in1, q.out_v,

@@ -30,6 +30,7 @@ struct QueryArgs {
     int64_t face0_slot = 0;
     int32_t stack_need = 0;
     bool packet = true;  // walk as wave packets (queries in Morton order)
+    void* rest = nullptr;  // packets: rest_bytes(n) bytes for the queries of given-up walks, or null: none is
     void* stream = nullptr;
 };
 
@@ -44,6 +45,15 @@ constexpr int64_t kWaveMax = (int64_t)1 << 18;
 
 // Stack capacity instantiated for a tree that needs `need` entries (-1 if none).
 int stack_capacity_for(int need);
+
+// Queries one call's packet walks may hand on to waves of their own (query.hip); the
+// walks past that many run to their end.
+constexpr int64_t kRestMax = 1 << 19;
+// Calls of this many queries hand nothing over: their 20 and more rounds of tiles cover the
+// long walks, and without the hand-over the walk needs no scratch (2^24 grid points on 1.3 M
+// faces: 12.45 ms without, 12.76 with; on 327,680: 7.12 and 7.29).
+constexpr int64_t kRestLast = (int64_t)1 << 23;
+size_t rest_bytes(int64_t n);
 
 // mode 0 unsigned distance, 1 signed (watertight), 2 signed (raystab)
 hipError_t launch_distance(const QueryArgs& q, int mode);
@@ -70,7 +80,7 @@ hipError_t ray_order(int64_t n, const float* rays_o, const float* rays_d, void* 
 // Static per-device scratch of the allocation-free distance call (order.hip): room for
 // the Morton order and ordering workspace of kNoAllocMaxQueries queries.
 constexpr int64_t kNoAllocMaxQueries = (int64_t)1 << 20;
-constexpr size_t kNoAllocScratchBytes = (size_t)32 << 20;
+constexpr size_t kNoAllocScratchBytes = (size_t)40 << 20;
 constexpr int kNoAllocDevices = 64;
 // Device address of the scratch on `device` (the current device); looked up once per device.
 hipError_t noalloc_scratch(int device, void** ptr);

@@ -11,10 +11,15 @@
 // taken one by one: 117 node rounds a query on 1.3 M faces, now 12), and the leaves are
 // always taken nearest first (640 exact face tests a query, now 143).
 //
-// What bounds it: instruction issue and latency.  A query on 81,920 faces takes 8 node,
-// 5 face and 2 exact rounds, about 2,600 cycles each with one wave per SIMD and 4,000
-// with eight.  777 points on 5,120 faces: 19 us (369 us with a lane each); 50,003 on
-// 81,920: 0.26 ms (2.77 ms as packets); 1,501 rays on 81,920: 19 us (156).
+// What bounds it: instruction issue.  A query on 81,920 faces takes 8 node, 5 face and 2
+// exact rounds, some 1,730 vector and as many scalar instructions (each 84% of the issue
+// slots of a full chip); the bytes (about 20 KB a query) come out of L2 and the Infinity
+// Cache.  Exact tests recompute the face's terms from its 48-byte record: the 144-byte
+// record that packets read made 250,000 points on 1.3 M faces 1.48 ms instead of 1.19.
+// Measured: 777 points on 5,120 faces 16 us (351 us with a lane each); 50,003 on 81,920
+// 0.22 ms (3.8 ms as packets); 1,501 rays on 81,920 14 us (146).  Not taken: 16 lanes per
+// query, four walks a wave (0.9-1.4 times as long), and queries in Morton order (5%, less
+// than the ordering costs).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -58,6 +63,8 @@ __device__ __forceinline__ uint32_t wave_min(uint32_t x) {
 
 // Lanes of m (not empty) with the smallest keys (non-negative floats): at most k of them,
 // as many as eight bisections of the keys' range can tell apart, or the smallest alone.
+// (Taking the keys within 3% of the smallest instead costs a third of the instructions but
+// 38% more time on 1.3 M faces, where it tells far points' leaves apart too coarsely.)
 __device__ __forceinline__ uint64_t nearest_lanes(uint64_t m, float key, int k) {
     const bool in = (m >> (threadIdx.x & 63)) & 1;
     const uint32_t bits = __float_as_uint(key);
@@ -238,9 +245,11 @@ __device__ void closest_face_wave(const Tree& T, int32_t root, f3 p, WaveLists& 
             int32_t slot = 0;
             if (lane < take) {
                 slot = (int32_t)L.face[w.nf - take + lane];
-                const FaceConst fc = load_face(T.tpre, slot);
-                bits = __float_as_uint(tri_dist2_pre(fc, p));  // >= 0, or a NaN that orders last
-                id = (uint32_t)fc.id;
+                f3 a, b, c;
+                int32_t i;
+                load_tri(T.tris, slot, a, b, c, i);
+                bits = __float_as_uint(tri_dist2(a, b, c, p));  // >= 0, or a NaN that orders last
+                id = (uint32_t)i;
             }
             w.nf -= take;
             const uint32_t m = wave_min(bits);
@@ -310,13 +319,12 @@ __device__ f3 avg_normal_wave(const Tree& T, f3 c, WaveLists& L) {
     return mk3((float)sx / cnt, (float)sy / cnt, (float)sz / cnt);
 }
 
-// Closest hit of the ray (wave-uniform arguments and results), as closest_hit.
-__device__ int32_t closest_hit_wave(const Tree& T, f3 o, f3 d, WaveLists& L, float& best_t, int32_t& best_id) {
+// Closest hit of the ray (wave-uniform arguments and results), as closest_hit; best / bslot
+// hold a candidate or the unset values.
+__device__ void closest_hit_wave(const Tree& T, f3 o, f3 d, WaveLists& L, float& best, int32_t& bslot, uint32_t& bid) {
     const int lane = (int)(threadIdx.x & 63);
     const f3 inv = ray_inverse(d);
-    float best = MAX_DIST, bound = MAX_DIST * BOUND_SLACK;
-    int32_t bslot = -1;
-    uint32_t bid = 0;
+    float bound = best * BOUND_SLACK + 1e-30f;
     WaveWork w{L};
     w.start(0);
     for (;;) {
@@ -361,9 +369,6 @@ __device__ int32_t closest_hit_wave(const Tree& T, f3 o, f3 d, WaveLists& L, flo
             break;
         }
     }
-    best_t = best;
-    best_id = (int32_t)bid;
-    return bslot;
 }
 
 // Query q at p from a candidate (d2, slot; slot < 0: none) to its outputs, by one wave.
@@ -403,21 +408,63 @@ __global__ __launch_bounds__(64) void distance_wave_kernel(const float* __restri
                      uvw);
 }
 
+// The queries that packet walks gave up (see PacketRest), a wave each.
+template <int MODE>
+__global__ __launch_bounds__(64) void distance_rest_kernel(const PacketRest* __restrict__ rest,
+                                                           const float* __restrict__ positions,
+                                                           float* __restrict__ distances,
+                                                           int64_t* __restrict__ face_id, float* __restrict__ uvw,
+                                                           Tree T) {
+    __shared__ WaveLists lists;
+    const uint32_t total = min(rest->count, rest->cap);
+    for (uint32_t t = blockIdx.x; t < total; t += gridDim.x) {
+        const int4 e = rest->list()[t];
+        if (uniform(e.x) == -1) continue;  // an empty place
+        const int64_t q = (int64_t)(uint32_t)uniform(e.x);
+        const int32_t slot = uniform(e.z);
+        wave_query<MODE>(T, uniform(e.w), ~slot, q, load_pt(positions, q), __int_as_float(uniform(e.y)), slot, lists,
+                         distances, face_id, uvw);
+        __builtin_amdgcn_wave_barrier();  // one back edge: every lane starts the next walk together
+    }
+}
+
+// Ray q from a candidate (t, slot; slot < 0: none) to its outputs, by one wave.
+__device__ __forceinline__ void wave_ray(const Tree& T, int64_t q, f3 o, f3 d, float t, int32_t slot, WaveLists& L,
+                                         float* __restrict__ positions, int64_t* __restrict__ face_id,
+                                         float* __restrict__ depth) {
+    uint32_t id = slot >= 0 ? (uint32_t)__float_as_int(T.tris[3 * slot].w) : 0u;
+    closest_hit_wave(T, o, d, L, t, slot, id);
+    if ((threadIdx.x & 63) == 0) {
+        depth[q] = t;
+        store_pt(positions, q,
+                 mk3(__builtin_fmaf(t, d.x, o.x), __builtin_fmaf(t, d.y, o.y), __builtin_fmaf(t, d.z, o.z)));
+        face_id[q] = slot >= 0 ? (int64_t)id : -1;
+    }
+}
+
 // Rays, one wave per ray.
 __global__ __launch_bounds__(64) void ray_wave_kernel(const float* __restrict__ rays_o, const float* __restrict__ rays_d,
                                                       float* __restrict__ positions, int64_t* __restrict__ face_id,
                                                       float* __restrict__ depth, Tree T) {
     __shared__ WaveLists lists;
     const int64_t q = blockIdx.x;
-    const f3 o = load_pt(rays_o, q), d = load_pt(rays_d, q);
-    float t;
-    int32_t id;
-    const int32_t slot = closest_hit_wave(T, o, d, lists, t, id);
-    if (threadIdx.x == 0) {
-        depth[q] = t;
-        store_pt(positions, q,
-                 mk3(__builtin_fmaf(t, d.x, o.x), __builtin_fmaf(t, d.y, o.y), __builtin_fmaf(t, d.z, o.z)));
-        face_id[q] = slot >= 0 ? (int64_t)id : -1;
+    wave_ray(T, q, load_pt(rays_o, q), load_pt(rays_d, q), MAX_DIST, -1, lists, positions, face_id, depth);
+}
+
+// The rays that packet and lane walks gave up, a wave each.
+__global__ __launch_bounds__(64) void ray_rest_kernel(const PacketRest* __restrict__ rest,
+                                                      const float* __restrict__ rays_o, const float* __restrict__ rays_d,
+                                                      float* __restrict__ positions, int64_t* __restrict__ face_id,
+                                                      float* __restrict__ depth, Tree T) {
+    __shared__ WaveLists lists;
+    const uint32_t total = min(rest->count, rest->cap);
+    for (uint32_t t = blockIdx.x; t < total; t += gridDim.x) {
+        const int4 e = rest->list()[t];
+        if (uniform(e.x) == -1) continue;  // an empty place
+        const int64_t q = (int64_t)(uint32_t)uniform(e.x);
+        wave_ray(T, q, load_pt(rays_o, q), load_pt(rays_d, q), __int_as_float(uniform(e.y)), uniform(e.z), lists,
+                 positions, face_id, depth);
+        __builtin_amdgcn_wave_barrier();  // one back edge: every lane starts the next walk together
     }
 }
 

@@ -133,7 +133,7 @@ int cubvh_unsigned_distance(cubvh_bvh* bvh, int device, int64_t n, const float* 
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same arguments and results, bit for bit, as
  * cubvh_unsigned_distance; at most 2^20 queries per call (larger n is refused).  The
- * Morton order of the queries and its workspace live in a static 32 MiB device array
+ * Morton order of the queries and its workspace live in a static 40 MiB device array
  * that each GPU running the library holds until the process ends; the call allocates
  * and frees nothing.  The tree must already be on `device` (cubvh_bvh_upload or an
  * earlier query there), otherwise the call fails.  Every call on one GPU uses that
