@@ -5,21 +5,26 @@
 // device synchronization and a 4-byte copy back to the host) by a fixed sequence of
 // three kernels with no host round trip, working in place in the output array:
 //
-//   1. tiles  : each workgroup labels one 16^3 tile in LDS (runs along the last
-//               axis, then union-find with LDS atomics between overlapping runs of
-//               neighbouring rows) and writes, for every free voxel, the global index
-//               of its tile-local root; occupied voxels get -1.
+//   1. tiles  : each workgroup labels one tile of 64 x 8 x 8 voxels (64 along the last
+//               axis: one row per wave, a lane per voxel, so that occupancy is one ballot,
+//               loads and stores are whole lines, and runs are bit arithmetic).
+//               Union-find in LDS between overlapping runs of neighbouring rows; every
+//               free voxel gets the global index of its tile-local root, others -1.
 //   2. merge  : voxels on a tile's low faces union themselves with their free
-//               neighbour in the adjacent tile (one launch per axis over the face
-//               voxels only; a pair with the same two labels as the pair before it
-//               on the face is skipped).  Union-find over the label array: a
-//               node's parent is always a smaller index of the same component, roots
-//               are linked smaller-under-larger with atomicMin and the link is
+//               neighbour in the adjacent tile, one wave per face, whose pairs with the
+//               same two labels are united once.  Union-find over the label
+//               array: a node's parent is always a smaller index of the same component,
+//               roots are linked smaller-under-larger with atomicMin and the link is
 //               retried until it lands on a root, so concurrent unions never lose an
 //               edge.
 //   3. flatten: label[i] = root(i).  Since parents only ever point to smaller
 //               indices, the root of each component is its minimum linear index.
-// Only the ~19% of voxels on tile faces touch global atomics.
+//
+// At 256^3 (a shell; 67 MB of labels, written, read at the faces, read and written): tiles
+// 57 us, merge 66 us, flatten 21 us, bound by latency (chains of dependent loads of a few
+// lanes) and for flatten by its 134 MB.  With tiles of 16^3 loaded a byte per lane, a
+// union per row of every face and a root search per voxel these were 118, 287 and 54 us.
+// A third of the voxels occupied at random: 760 -> 187 us; 64^3: 78 -> 38 us.
 //
 // The result equals the reference's converged output (the minimum linear index of
 // each free component, -1 for occupied voxels, indices global across the batch)
@@ -46,10 +51,24 @@ __device__ __forceinline__ int32_t find_root(const int32_t* L, int32_t x) {
     return x;
 }
 
+// find_root that points every node it passes at its grandparent.  A store may undo a
+// concurrent link of a node that was no root any more; unite goes on from the value that
+// link replaced, so no edge is lost.
+__device__ __forceinline__ int32_t find_root_halving(int32_t* L, int32_t x) {
+    int32_t p = ld_parent(L, x);
+    while (p != x) {
+        const int32_t g = ld_parent(L, p);
+        if (g != p) __hip_atomic_store(L + x, g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        x = p;
+        p = g;
+    }
+    return x;
+}
+
 __device__ __forceinline__ void unite(int32_t* L, int32_t a, int32_t b) {
     for (;;) {
-        a = find_root(L, a);
-        b = find_root(L, b);
+        a = find_root_halving(L, a);
+        b = find_root_halving(L, b);
         if (a == b) return;
         if (a > b) {
             int32_t t = a; a = b; b = t;
@@ -61,9 +80,11 @@ __device__ __forceinline__ void unite(int32_t* L, int32_t a, int32_t b) {
     }
 }
 
-constexpr int TILE = 16;          // tile edge (voxels)
-constexpr int TILE_N = TILE * TILE * TILE;
-constexpr int TILE_THREADS = 256;
+constexpr int TD = 64, TW = 8, TH = 8;  // tile edges along the last, middle and first axis
+constexpr int TILE_ROWS = TW * TH;
+constexpr int TILE_WAVES = 4;
+constexpr int WAVE_ROWS = TILE_ROWS / TILE_WAVES;
+static_assert(TH == TILE_ROWS / TW && 2 * (2 * TILE_ROWS - TW - TH) <= 64 * TILE_WAVES, "threads of the row pairs");
 
 __device__ __forceinline__ int32_t lds_parent(const int32_t* L, int32_t x) {
     return __hip_atomic_load(L + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -90,125 +111,174 @@ __device__ __forceinline__ void lds_unite(int32_t* L, int32_t a, int32_t b) {
     }
 }
 
-// One workgroup of 256 threads per 16^3 tile; tiles numbered d fastest, then w, h, b.
-// In LDS a voxel (lh, lw, ld) sits at (lh * 16 + lw) * ROW + ld: rows of 16 voxels
-// along d, padded to ROW = 17 words so that one row per lane touches distinct banks.
-// The padded index orders voxels like the tile's linear index, so the smallest
-// index of a component is also its smallest voxel.
-//   0. all threads load the tile's occupancy (coalesced, 16 consecutive d per row);
-//   1. thread t labels the runs of free voxels of row t by their first voxel;
-//   2. it unites each run-overlap segment of its row with the rows at w - 1 and
-//      h - 1 (one union per segment: two runs meet in one contiguous segment);
-//   3. all threads write the global index of every free voxel's tile-local root.
-constexpr int ROW = TILE + 1;
-__device__ __forceinline__ int pad_index(int k) { return (k >> 4) * ROW + (k & 15); }
+// First voxel of the run of set bits of `free` that holds bit `lane` (which is set).
+__device__ __forceinline__ int run_start(uint64_t free, int lane) {
+    const uint64_t gaps = ~free & ((1ull << lane) - 1ull);
+    return gaps ? 64 - __builtin_clzll(gaps) : 0;
+}
 
-__global__ __launch_bounds__(TILE_THREADS) void ff_tiles(const uint8_t* __restrict__ grid, int32_t* __restrict__ out,
-                                                         int32_t H, int32_t W, int32_t D) {
-    __shared__ int32_t L[TILE * TILE * ROW];
-    __shared__ uint8_t occ[TILE * TILE * ROW];
-    const int32_t nd = (D + TILE - 1) / TILE, nw = (W + TILE - 1) / TILE, nh = (H + TILE - 1) / TILE;
-    const int64_t tile = blockIdx.x;
-    const int32_t d0 = (int32_t)(tile % nd) * TILE;
-    const int32_t w0 = (int32_t)((tile / nd) % nw) * TILE;
-    const int64_t rest = tile / ((int64_t)nd * nw);
-    const int32_t h0 = (int32_t)(rest % nh) * TILE;
-    const int32_t b = (int32_t)(rest / nh);
-    const int64_t base = (int64_t)b * H * W * D;
-    for (int k = threadIdx.x; k < TILE_N; k += TILE_THREADS) {
-        const int lh = k >> 8, lw = (k >> 4) & 15, ld = k & 15;
-        const int h = h0 + lh, w = w0 + lw, d = d0 + ld;
-        uint8_t o = 1;  // outside the grid counts as occupied
-        if (h < H && w < W && d < D) o = grid[base + ((int64_t)h * W + w) * D + d] ? 1 : 0;
-        occ[pad_index(k)] = o;
+// One workgroup per tile; tiles numbered along the last axis fastest, then w, h, b.  Voxel
+// `lane` of row r (w = r % TW, h = r / TW) has the local index 64 r + lane, which orders
+// voxels like the tile's linear index; only the first voxel of a run is a union-find node.
+__global__ __launch_bounds__(64 * TILE_WAVES) void ff_tiles(const uint8_t* __restrict__ grid, int32_t* __restrict__ out,
+                                                            int32_t H, int32_t W, int32_t D) {
+    __shared__ int32_t L[64 * TILE_ROWS];
+    __shared__ uint64_t rows[TILE_ROWS];
+    const int32_t nd = (D + TD - 1) / TD, nw = (W + TW - 1) / TW, nh = (H + TH - 1) / TH;
+    const uint32_t tile = blockIdx.x;
+    const int32_t d0 = (int32_t)(tile % nd) * TD;
+    const int32_t w0 = (int32_t)((tile / nd) % nw) * TW;
+    const uint32_t rest = tile / ((uint32_t)nd * nw);
+    const int32_t h0 = (int32_t)(rest % nh) * TH;
+    const int32_t base = (int32_t)(rest / nh) * H * W * D;  // the whole grid has fewer than 2^31 voxels
+    const int lane = (int)threadIdx.x & 63, r0 = ((int)threadIdx.x >> 6) * WAVE_ROWS;
+    const int32_t d = d0 + lane;
+    uint8_t occ[WAVE_ROWS];
+#pragma unroll
+    for (int k = 0; k < WAVE_ROWS; ++k) {
+        const int r = r0 + k, h = h0 + r / TW, w = w0 + r % TW;
+        occ[k] = 1;  // outside the grid counts as occupied
+        if (h < H && w < W && d < D) occ[k] = grid[base + (h * W + w) * D + d];
+    }
+    uint64_t free[WAVE_ROWS];
+#pragma unroll
+    for (int k = 0; k < WAVE_ROWS; ++k) {
+        free[k] = __builtin_amdgcn_ballot_w64(occ[k] == 0);
+        rows[r0 + k] = free[k];  // every lane the same value
+        L[64 * (r0 + k) + lane] = 64 * (r0 + k) + lane;
     }
     __syncthreads();
-    const int row = (int)threadIdx.x * ROW;
-    {
-        int32_t start = -1;
-        for (int ld = 0; ld < TILE; ++ld) {
-            const int k = row + ld;
-            if (occ[k]) {
-                L[k] = -1;
-                start = -1;
-            } else {
-                if (start < 0) start = k;
-                L[k] = start;
-            }
+    // two threads (one per half of the row) for each pair of neighbouring rows: two runs meet
+    // in one contiguous segment, united at its first voxel
+    const int pr = (int)threadIdx.x >> 1;
+    if (pr < 2 * TILE_ROWS - TW - TH) {
+        const bool along_w = pr < TILE_ROWS - TH;
+        const int r = along_w ? pr / (TW - 1) * TW + pr % (TW - 1) + 1 : pr - (TILE_ROWS - TH) + TW;
+        const int o = along_w ? r - 1 : r - TW;  // the row at w - 1, or at h - 1
+        const uint64_t mine = rows[r], other = rows[o], both = mine & other;
+        uint64_t segments = both & ~(both << 1) & (0xffffffffull << (32 * (threadIdx.x & 1)));
+        for (; segments != 0; segments &= segments - 1) {
+            const int l = __builtin_ctzll(segments);
+            lds_unite(L, 64 * r + run_start(mine, l), 64 * o + run_start(other, l));
         }
     }
     __syncthreads();
-    const int lh = (int)threadIdx.x >> 4, lw = (int)threadIdx.x & 15;
-    for (int nb = 0; nb < 2; ++nb) {
-        if (nb == 0 ? lw == 0 : lh == 0) continue;
-        const int off = nb == 0 ? ROW : TILE * ROW;  // row at w - 1, or at h - 1
-        bool prev = false;  // previous position was a free/free pair
-        for (int ld = 0; ld < TILE; ++ld) {
-            const int k = row + ld;
-            const bool pair = !occ[k] && !occ[k - off];
-            if (pair && !prev) lds_unite(L, lds_parent(L, k), lds_parent(L, k - off));
-            prev = pair;
-        }
-    }
-    __syncthreads();
-    for (int k = threadIdx.x; k < TILE_N; k += TILE_THREADS) {
-        const int lhk = k >> 8, lwk = (k >> 4) & 15, ld = k & 15;
-        const int h = h0 + lhk, w = w0 + lwk, d = d0 + ld;
+#pragma unroll
+    for (int k = 0; k < WAVE_ROWS; ++k) {
+        const int r = r0 + k, h = h0 + r / TW, w = w0 + r % TW;
         if (h >= H || w >= W || d >= D) continue;
-        const int pk = pad_index(k);
         int32_t lab = -1;
-        if (!occ[pk]) {
-            const int32_t r = lds_root(L, pk);
-            const int rrow = r / ROW, rd = r - rrow * ROW;
-            lab = (int32_t)(base + ((int64_t)(h0 + (rrow >> 4)) * W + (w0 + (rrow & 15))) * D + (d0 + rd));
+        if ((free[k] >> lane) & 1) {
+            const int32_t root = lds_root(L, 64 * r + run_start(free[k], lane)), rr = root >> 6;
+            lab = base + ((h0 + rr / TW) * W + (w0 + rr % TW)) * D + d0 + (root & 63);
         }
-        out[base + ((int64_t)h * W + w) * D + d] = lab;
+        out[base + (h * W + w) * D + d] = lab;
     }
 }
 
-// Unions across the tile faces normal to one axis: thread t takes voxel v on a face
-// (coordinate along the axis a positive multiple of TILE) and its neighbour one step
-// back along the axis.  Both start from their tile-local labels; a pair whose labels
-// equal those of the pair one step back along the face's fastest in-plane axis is
-// the same union and is skipped, so only the first pair of every run unites (the
-// comparison is safe whatever concurrent unions have changed: equal starting labels
-// give the identical union).  AXIS 0 = last tensor axis (stride 1), 1 = middle (stride
-// D), 2 = first spatial axis (stride D * W).
-template <int AXIS>
-__global__ __launch_bounds__(256) void ff_merge_axis(const uint8_t* __restrict__ grid, int32_t* L, int32_t B,
-                                                     int32_t H, int32_t W, int32_t D) {
-    const int32_t dims[3] = {D, W, H};
-    const int32_t na = (dims[AXIS] - 1) / TILE;  // faces along the axis
-    // in-face axes: the fastest one (`u`) and the other (`v`), plus the batch
-    const int32_t ua = AXIS == 0 ? 1 : 0, va = AXIS == 2 ? 1 : 2;
-    const int32_t nu = dims[ua], nv = dims[va];
-    const int64_t total = (int64_t)B * na * nu * nv;
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= total) return;
-    int32_t c[3];
-    c[ua] = (int32_t)(t % nu);
-    c[AXIS] = TILE * (1 + (int32_t)((t / nu) % na));
-    const int64_t rest = t / ((int64_t)nu * na);
-    c[va] = (int32_t)(rest % nv);
-    const int32_t b = (int32_t)(rest / nv);
-    const int64_t strides[3] = {1, D, (int64_t)D * W};
-    const int64_t i = (int64_t)b * H * W * D + c[2] * strides[2] + c[1] * strides[1] + c[0];
-    const int64_t step = strides[AXIS];
-    if (grid[i] || grid[i - step]) return;
-    const int32_t li = L[i], lj = L[i - step];
-    if (c[ua] > 0) {
-        const int64_t k = i - strides[ua];  // the same pair one step back along u
-        if (!grid[k] && !grid[k - step] && L[k] == li && L[k - step] == lj) return;
+// Unions across the tile faces: the voxels on a tile's low faces with their neighbour one
+// step back, one wave per face normal to the middle or the first axis (8 rows of 64 pairs),
+// and per 512 pairs of the faces normal to the last axis.  Pairs with the same two labels
+// are the same union: a pair that repeats the one before it in its lane is dropped, the
+// others leave their number in a small table, and one that finds another pair's number
+// there with the same labels is done (a pair whose entry was taken by different labels is
+// united as often as it occurs).  A wave per face and not a workgroup: the unions are
+// chains of dependent loads by a few lanes, so what counts is the faces in flight.
+constexpr int MERGE_ROWS = 8;
+constexpr uint32_t MERGE_SLOTS = 1024;
+static_assert(MERGE_ROWS == TW && MERGE_ROWS == TH && TD == 64, "one wave per face");
+
+__global__ __launch_bounds__(64) void ff_merge(int32_t* L, int32_t B, int32_t H, int32_t W, int32_t D, uint32_t b0,
+                                               uint32_t b1) {
+    __shared__ int32_t low[64 * MERGE_ROWS], high[64 * MERGE_ROWS];
+    __shared__ uint16_t owner[MERGE_SLOTS];
+    const int t = (int)threadIdx.x;
+    const uint32_t nd = (D + TD - 1) / TD, nw = (W + TW - 1) / TW, nh = (H + TH - 1) / TH;
+    int32_t li[MERGE_ROWS], lj[MERGE_ROWS];
+#pragma unroll
+    for (int r = 0; r < MERGE_ROWS; ++r) li[r] = lj[r] = -1;
+    if (blockIdx.x < b0) {  // the last axis: w fastest, then the boundary, then h, then b
+#pragma unroll
+        for (int r = 0; r < MERGE_ROWS; ++r) {
+            const uint32_t k = (blockIdx.x * MERGE_ROWS + r) * 64 + t, q = k / W, q2 = q / (nd - 1);
+            const int32_t b = (int32_t)(q2 / H);
+            if (b >= B) continue;
+            const int32_t i = ((b * H + (int32_t)(q2 % H)) * W + (int32_t)(k % W)) * D + (int32_t)(q % (nd - 1) + 1) * TD;
+            li[r] = L[i];
+            lj[r] = L[i - 1];
+        }
+    } else {
+        const bool middle = blockIdx.x < b0 + b1;
+        const uint32_t k = blockIdx.x - b0 - (middle ? 0 : b1), q = k / nd;
+        const int32_t d = (int32_t)(k % nd) * TD + t;
+        const uint32_t cw = middle ? nw - 1 : nw, ch = middle ? nh : nh - 1;  // faces along w and h
+        const int32_t w0 = (int32_t)(q % cw + (middle ? 1 : 0)) * TW, h0 = (int32_t)(q / cw % ch + (middle ? 0 : 1)) * TH;
+        const int32_t b = (int32_t)(q / cw / ch), step = middle ? D : D * W;
+#pragma unroll
+        for (int r = 0; r < MERGE_ROWS; ++r) {
+            const int32_t w = middle ? w0 : w0 + r, h = middle ? h0 + r : h0;
+            if (d >= D || w >= W || h >= H) continue;
+            const int32_t i = ((b * H + h) * W + w) * D + d;
+            li[r] = L[i];
+            lj[r] = L[i - step];
+        }
     }
-    unite(L, (int32_t)i, (int32_t)(i - step));
+    uint32_t todo = 0;
+#pragma unroll
+    for (int r = 0; r < MERGE_ROWS; ++r) {
+        if (li[r] < 0 || lj[r] < 0 || (r > 0 && li[r] == li[r - 1] && lj[r] == lj[r - 1])) continue;
+        const int at = 64 * r + t;
+        low[at] = lj[r];
+        high[at] = li[r];
+        owner[(((uint32_t)li[r] * 0x9e3779b1u) ^ ((uint32_t)lj[r] * 0x85ebca77u)) >> 22] = (uint16_t)at;
+        todo |= 1u << r;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < MERGE_ROWS; ++r) {
+        if (!((todo >> r) & 1u)) continue;
+        const int o = owner[(((uint32_t)li[r] * 0x9e3779b1u) ^ ((uint32_t)lj[r] * 0x85ebca77u)) >> 22];
+        if (o != 64 * r + t && low[o] == lj[r] && high[o] == li[r]) continue;
+        unite(L, li[r], lj[r]);
+    }
 }
 
-__global__ void ff_flatten(int32_t* L, int32_t ntot) {
-    int32_t i = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i >= ntot) return;
-    int32_t p = L[i];
-    if (p < 0 || p == i) return;
-    L[i] = find_root(L, p);
+// label[i] = root(i), a workgroup per tile.  A tile's voxels have few distinct labels (its
+// local roots), whose roots are kept in a table: most voxels find theirs there.
+constexpr uint32_t FLAT_SLOTS = 512;
+__global__ __launch_bounds__(64 * TILE_WAVES) void ff_flatten(int32_t* L, int32_t H, int32_t W, int32_t D) {
+    __shared__ unsigned long long known[FLAT_SLOTS];  // (label, root)
+    const int32_t nd = (D + TD - 1) / TD, nw = (W + TW - 1) / TW, nh = (H + TH - 1) / TH;
+    const uint32_t tile = blockIdx.x;
+    const int32_t d = (int32_t)(tile % nd) * TD + ((int)threadIdx.x & 63);
+    const int32_t w0 = (int32_t)((tile / nd) % nw) * TW;
+    const uint32_t rest = tile / ((uint32_t)nd * nw);
+    const int32_t h0 = (int32_t)(rest % nh) * TH;
+    const int32_t base = (int32_t)(rest / nh) * H * W * D;
+    const int r0 = ((int)threadIdx.x >> 6) * WAVE_ROWS;
+    for (int k = (int)threadIdx.x; k < (int)FLAT_SLOTS; k += 64 * TILE_WAVES) known[k] = ~0ull;
+    int32_t lab[WAVE_ROWS];
+#pragma unroll
+    for (int k = 0; k < WAVE_ROWS; ++k) {
+        const int r = r0 + k, h = h0 + r / TW, w = w0 + r % TW;
+        lab[k] = -1;
+        if (h < H && w < W && d < D) lab[k] = L[base + (h * W + w) * D + d];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < WAVE_ROWS; ++k) {
+        if (lab[k] < 0) continue;  // occupied, or outside the grid
+        unsigned long long* at = known + (((uint32_t)lab[k] * 0x9e3779b1u) >> 23);
+        const unsigned long long e = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        int32_t root = (int32_t)(uint32_t)e;
+        if ((uint32_t)(e >> 32) != (uint32_t)lab[k]) {
+            root = find_root(L, lab[k]);
+            __hip_atomic_store(at, ((unsigned long long)(uint32_t)lab[k] << 32) | (uint32_t)root, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        const int r = r0 + k, h = h0 + r / TW, w = w0 + r % TW;
+        if (root != lab[k]) L[base + (h * W + w) * D + d] = root;
+    }
 }
 
 }  // namespace dev
@@ -217,27 +287,19 @@ hipError_t launch_floodfill(const uint8_t* grid, int32_t B, int32_t H, int32_t W
                             hipStream_t stream) {
     const int64_t ntot64 = (int64_t)B * H * W * D;
     if (ntot64 <= 0) return hipSuccess;
-    const int32_t ntot = (int32_t)ntot64;
-    const int block = 256;
-    const unsigned grid_n = (unsigned)((ntot64 + block - 1) / block);
-    const int64_t n_tiles = (int64_t)B * ((H + dev::TILE - 1) / dev::TILE) * ((W + dev::TILE - 1) / dev::TILE) *
-                            ((D + dev::TILE - 1) / dev::TILE);
-    hipLaunchKernelGGL(dev::ff_tiles, dim3((unsigned)n_tiles), dim3(dev::TILE_THREADS), 0, stream, grid, labels, H, W,
+    const int64_t n_tiles = (int64_t)B * ((H + dev::TH - 1) / dev::TH) * ((W + dev::TW - 1) / dev::TW) *
+                            ((D + dev::TD - 1) / dev::TD);
+    hipLaunchKernelGGL(dev::ff_tiles, dim3((unsigned)n_tiles), dim3(64 * dev::TILE_WAVES), 0, stream, grid, labels, H, W,
                        D);
-    // unions across tile faces normal to each axis (no launch when the axis has one tile)
-    const int64_t nd = (int64_t)B * ((D - 1) / dev::TILE) * W * H;
-    const int64_t nw = (int64_t)B * ((W - 1) / dev::TILE) * D * H;
-    const int64_t nh = (int64_t)B * ((H - 1) / dev::TILE) * D * W;
-    if (nd > 0)
-        hipLaunchKernelGGL(dev::ff_merge_axis<0>, dim3((unsigned)((nd + block - 1) / block)), dim3(block), 0, stream,
-                           grid, labels, B, H, W, D);
-    if (nw > 0)
-        hipLaunchKernelGGL(dev::ff_merge_axis<1>, dim3((unsigned)((nw + block - 1) / block)), dim3(block), 0, stream,
-                           grid, labels, B, H, W, D);
-    if (nh > 0)
-        hipLaunchKernelGGL(dev::ff_merge_axis<2>, dim3((unsigned)((nh + block - 1) / block)), dim3(block), 0, stream,
-                           grid, labels, B, H, W, D);
-    hipLaunchKernelGGL(dev::ff_flatten, dim3(grid_n), dim3(block), 0, stream, labels, ntot);
+    // waves of the faces normal to the last, the middle and the first axis
+    const int64_t nd = (D + dev::TD - 1) / dev::TD, nw = (W + dev::TW - 1) / dev::TW, nh = (H + dev::TH - 1) / dev::TH;
+    const uint32_t b0 = (uint32_t)(((int64_t)B * (nd - 1) * W * H + 64 * dev::MERGE_ROWS - 1) /
+                                   (64 * dev::MERGE_ROWS));
+    const uint32_t b1 = (uint32_t)(B * nh * (nw - 1) * nd), b2 = (uint32_t)(B * (nh - 1) * nw * nd);
+    if (b0 + b1 + b2 > 0) {  // labels of one tile are final already
+        hipLaunchKernelGGL(dev::ff_merge, dim3(b0 + b1 + b2), dim3(64), 0, stream, labels, B, H, W, D, b0, b1);
+        hipLaunchKernelGGL(dev::ff_flatten, dim3((unsigned)n_tiles), dim3(64 * dev::TILE_WAVES), 0, stream, labels, H, W, D);
+    }
     return hipGetLastError();
 }
 

@@ -55,3 +55,26 @@ def test_floodfill_occupancy_of_distance_field(gpu, oracle):
     ref = oracle.floodfill_bfs(occ.cpu().numpy())
     np.testing.assert_array_equal(lab, ref)
     assert len(np.unique(lab[lab >= 0])) >= 2
+
+
+@pytest.mark.parametrize("shape", [(1, 8, 8, 64), (1, 9, 17, 65), (2, 33, 3, 130), (1, 17, 40, 63), (1, 64, 64, 128)])
+@pytest.mark.parametrize("kind", ["noise", "open", "maze"])
+def test_floodfill_across_tiles(gpu, oracle, shape, kind):
+    """Sizes around the labelling tiles (64 x 8 x 8): random grids, one open component, and
+    one long winding corridor (walls with a gap at alternating ends)."""
+    rng = np.random.default_rng(sum(shape))
+    if kind == "noise":
+        g = rng.random(shape) < 0.55
+    elif kind == "open":
+        g = np.zeros(shape, dtype=bool)
+        g[..., shape[-1] // 2] = rng.random(shape[:-1]) < 0.9
+    else:
+        g = np.zeros(shape, dtype=bool)
+        g[:, 1::2] = True
+        g[:, 1::4, -1, -1] = False
+        g[:, 3::4, 0, 0] = False
+        g[:, ::2, 1::2] = True
+        g[:, ::2, 1::4, -1] = False
+        g[:, ::2, 3::4, 0] = False
+    lab = cubvh_amd.floodfill(torch.from_numpy(g).to(gpu)).cpu().numpy()
+    np.testing.assert_array_equal(lab, oracle.floodfill_bfs(g))
