@@ -157,3 +157,22 @@ def test_errors():
         ht.impl.search(_t([[1, 2, 3, 4]]))
     with pytest.raises(cubvh_amd._lib.CubvhError, match="prepare"):
         ht.impl.insert(_t([[1, 2, 3, 4]]))
+
+
+@pytest.mark.parametrize("d", [1, 3, 5, 15, 16])
+@pytest.mark.parametrize("capacity", [1, 2, 7, 8, 9, 13, 64, 1003])
+def test_probe_runs_reach_every_slot(d, capacity):
+    """Capacities around the slots of a 128-byte line (8, 4, 2 or 1): a table filled to its
+    last slot holds every row, whichever line it started in, and a search of absent keys
+    ends."""
+    rng = np.random.default_rng(capacity * 64 + d)
+    rows = rng.permutation(4 * capacity)[:capacity]
+    coords = np.zeros((capacity, d), dtype=np.int32)
+    coords[:, 0] = rows
+    coords[:, -1] += rows % 3
+    impl = cubvh_amd.create_cuHashTable()
+    impl.set_num_dims(d)
+    impl.resize(capacity)
+    impl.insert(_t(coords))
+    assert impl.search(_t(coords)).tolist() == list(range(capacity))
+    assert impl.search(_t(coords - 5 * capacity)).tolist() == [-1] * capacity
