@@ -36,8 +36,7 @@ int fail_hip(hipError_t e, const char* what) {
 
 constexpr int kMaxDevices = 64;
 constexpr int kDefaultLeaf = 16;  // faces per leaf unless the caller asks otherwise
-// Raystab batches at least this large are sorted into Morton order; smaller ones are
-// walked one lane per query in input order.
+// A captured raystab call of fewer queries walks one lane per query, without scratch.
 constexpr int64_t kMortonMin = 1 << 11;
 
 // Keeps freed stream-ordered allocations in the device's default pool instead of
@@ -354,33 +353,44 @@ int run_distance(cubvh_bvh* bvh, int device, int64_t n, int kmode, const float* 
     q.out_id = face_id;
     q.out_v = uvw;
     hipStream_t hs = (hipStream_t)stream;
-    // Large batches are walked in Morton order (stream-ordered scratch from the
-    // device's default memory pool, released after the launch).
+    // Large batches are walked in Morton order, and raystab needs lists (stream-ordered
+    // scratch from the device's default memory pool, released after the launch).  A captured
+    // raystab call of few queries allocates nothing: it walks one lane per query.
     void* scratch = nullptr;
-    if (n >= (kmode == 2 ? kMortonMin : kWaveMax) && n < ((int64_t)1 << 31)) {
+    const bool ordered = n >= kWaveMax && n < ((int64_t)1 << 31);
+    bool lists = kmode == 2 && n < ((int64_t)1 << 31);
+    if (lists && n < kMortonMin) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        hipError_t e = hipStreamIsCapturing(hs, &cs);
+        if (e != hipSuccess) return fail_hip(e, "hipStreamIsCapturing");
+        lists = cs == hipStreamCaptureStatusNone;
+    }
+    if (ordered || lists) {
         rc = ensure_pool(device);
         if (rc != CUBVH_OK) return rc;
-        const size_t ob = ((size_t)n * 4 + 255) & ~(size_t)255;
-        // raystab: the stab passes' lists after the order, the ordering workspace after them
-        const size_t sb = kmode == 2 ? ((stab_workspace_bytes(n) + 255) & ~(size_t)255) : 0;
-        const size_t rb = rest_bytes(n);
-        hipError_t e = hipMallocAsync(&scratch, ob + sb + rb + morton_workspace_bytes(n), hs);
+        // the stab passes' lists, then the order, the rest of the walks and the ordering workspace
+        const size_t sb = lists ? ((stab_workspace_bytes(n) + 255) & ~(size_t)255) : 0;
+        const size_t ob = ordered ? ((size_t)n * 4 + 255) & ~(size_t)255 : 0;
+        const size_t rb = ordered ? rest_bytes(n) : 0;
+        hipError_t e = hipMallocAsync(&scratch, sb + ob + rb + (ordered ? morton_workspace_bytes(n) : 0), hs);
         if (e != hipSuccess) return fail_hip(e, "hipMallocAsync(query order)");
-        uint32_t* order = (uint32_t*)scratch;
-        q.rest = (char*)scratch + ob + sb;
-        e = morton_order(n, positions, (char*)scratch + ob + sb + rb, order, hs);
-        if (e != hipSuccess) {
-            (void)hipFreeAsync(scratch, hs);
-            return fail_hip(e, "query ordering");
+        if (ordered) {
+            uint32_t* order = (uint32_t*)((char*)scratch + sb);
+            q.rest = (char*)scratch + sb + ob;
+            e = morton_order(n, positions, (char*)scratch + sb + ob + rb, order, hs);
+            if (e != hipSuccess) {
+                (void)hipFreeAsync(scratch, hs);
+                return fail_hip(e, "query ordering");
+            }
+            q.order = order;
         }
-        q.order = order;
     }
-    q.packet = scratch != nullptr;
+    q.packet = ordered;
     hipError_t e;
-    if (kmode == 2 && q.packet) {
-        // raystab over Morton-ordered queries: packet distance walk, then the stab rays
+    if (lists) {
+        // raystab: the distances, then the stab rays
         e = launch_distance(q, 0);
-        if (e == hipSuccess) e = launch_stab_sign(q, (char*)scratch + (((size_t)n * 4 + 255) & ~(size_t)255));
+        if (e == hipSuccess) e = launch_stab_sign(q, scratch);
     } else {
         e = launch_distance(q, kmode);
     }

@@ -1030,6 +1030,8 @@ __global__ __launch_bounds__(BLOCK) void distance_kernel(int64_t n, const float*
 //                hits both ways make list 0;
 //   stab_lines : lines k0 .. k0 + L - 1 of the listed queries, one item per (line,
 //                entry), line-major; a line that misses marks its entry (bit 31);
+//   stab_wave  : the work of stab_first or stab_lines with a wave per line instead of a
+//                lane, for calls that do not fill the chip with lanes' chains;
 //   stab_keep  : the unmarked entries make the next list;
 //   stab_negate: the queries of the last list are inside.
 // Lines after a query's first miss may be walked too; the decisions are the ones of
@@ -1186,6 +1188,47 @@ __global__ __launch_bounds__(BLOCK, kStabWaves) void stab_lines(uint32_t b, uint
     job.positions = positions;
     job.offs = offs;
     walk_lines(T, job, (unsigned long long*)(counts + 32) + b, st);
+}
+
+// One line by a wave.  Batch 0 (`first`): line 0 of query x, which joins the list when it
+// hits both ways; else line k0 + y of list entry x, which is marked when it misses.
+__device__ __forceinline__ void stab_line_wave(bool first, uint32_t k0, uint32_t x, uint32_t y, uint32_t* __restrict__ list,
+                                               uint32_t* __restrict__ counts, const float* __restrict__ positions,
+                                               float2* __restrict__ offs, const Tree& T, WaveLists& L) {
+    uint32_t q = x;
+    if (!first) q = (uint32_t)uniform((int32_t)__hip_atomic_load(&list[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    if (q & kStabMiss) return;  // an earlier line already missed
+    float2 r;
+    if (first) {
+        Pcg32 rng;
+        rng.advance((uint64_t)(uint32_t)(q * 2u));
+        r.x = rng.next_float();
+        r.y = rng.next_float();
+    } else {
+        r = offs[q];
+    }
+    const int found = any_hit_line_wave(T, load_pt(positions, q), fibonacci_dir32(k0 + y, r.x, r.y), L);
+    if (first) {
+        offs[q] = r;  // every lane the same value
+        if (found == 3 && (threadIdx.x & 63) == 0) list[atomicAdd(&counts[1], 1u)] = q;
+    } else if (found != 3) {
+        __hip_atomic_fetch_or(&list[x], kStabMiss, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// A whole batch by waves: batch 0 is line 0 of queries 0 .. n - 1, batch 1 + b the lines of
+// line batch b.
+__global__ __launch_bounds__(64) void stab_wave(uint32_t batch, uint32_t* __restrict__ list, uint32_t* __restrict__ counts,
+                                                const float* __restrict__ positions, float2* __restrict__ offs, Tree T) {
+    __shared__ WaveLists lists;
+    const bool first = batch == 0;
+    const uint32_t m = counts[batch], k0 = first ? 0u : kStabBatchFirst[batch - 1];
+    const unsigned long long total = (unsigned long long)m * (first ? 1u : kStabBatchFirst[batch] - k0);
+    for (unsigned long long t = blockIdx.x; t < total; t += gridDim.x) {
+        const uint32_t y = (uint32_t)(t / m);
+        stab_line_wave(first, k0, (uint32_t)(t - (unsigned long long)y * m), y, list, counts, positions, offs, T, lists);
+        __builtin_amdgcn_wave_barrier();  // one back edge: every lane starts the next line together
+    }
 }
 
 // The unmarked entries of list_in (count_in of them) make list_out (count_out).
@@ -1416,6 +1459,15 @@ constexpr int kLdsEntries = 12;
 constexpr int kDistanceWaves = 1;
 constexpr uint32_t kRestBlocks = 8192;  // one-wave workgroups of a rest launch: what the chip holds at once
 
+// Raystab calls of fewer queries walk their lines 1 .. 31 a wave per line (line 0 below
+// kWaveMax).  Measured, waves against lanes: 2,100 points 0.08-0.14 / 2.1-8.5 ms (the lanes
+// with the distances as packets, on 20,480 to 1.3 M faces), 200,000 1.0-1.6 / 2.6-6.4;
+// 600,011 2.0 / 3.2, 3.1 / 5.7, 4.1 / 7.9 ms on soups, 3.5 / 3.8 on a closed mesh; 2,000,000
+// 4.0 / 5.2, 5.8 / 8.5, 7.7 / 11.9, but 8.7 / 7.2 on the closed mesh, whose lines are short
+// and many.  Lanes that hand walks of more than 32 to 256 steps to waves were no better.
+constexpr int64_t kStabWaveMax = (int64_t)1 << 20;
+constexpr int64_t kStabWaveBlocks = 16384;
+
 // Runs of consecutive workgroups per XCD for a grid of nb one-wave workgroups over a
 // Morton order: the largest power of two <= nb / 128, so that each XCD's L2 serves one
 // aligned block of the order at a time (the 256^3 UDF walk: 10.80 ms with 2048 =
@@ -1540,7 +1592,8 @@ size_t stab_workspace_bytes(int64_t n) {
 hipError_t launch_stab_sign(const QueryArgs& q, void* ws) {
     if (q.n <= 0) return hipSuccess;
     if (stack_capacity_for(q.stack_need) < 0) return hipErrorInvalidValue;
-    if (!q.order || !ws || q.n >= ((int64_t)1 << 31)) return hipErrorInvalidValue;  // bit 31 marks list entries
+    // bit 31 marks list entries; the lane walks need the Morton order
+    if (!ws || q.n >= ((int64_t)1 << 31) || (q.n >= kWaveMax && !q.order)) return hipErrorInvalidValue;
     const dev::Tree T = dev::make_tree(q.tree, q.face0_slot);
     hipStream_t s = (hipStream_t)q.stream;
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
@@ -1562,13 +1615,20 @@ hipError_t launch_stab_sign(const QueryArgs& q, void* ws) {
     const unsigned keep_grid = (unsigned)((q.n + 255) / 256);
     hipLaunchKernelGGL(dev::stab_init, dim3(1), dim3(64), 0, s, counts, q.n);
     const unsigned first_grid = (unsigned)((q.n + SB - 1) / SB);
-    hipLaunchKernelGGL((dev::stab_first<SB, kLdsEntries>), dim3(first_grid), dim3(SB), 0, s, q.order, lists[0], counts,
-                       q.in0, offs, T, xcd_chunk_for(first_grid));
-    for (int b = 0; b < dev::kStabBatches; ++b) {
-        hipLaunchKernelGGL((dev::stab_lines<SB, kLdsEntries>), dim3(grid), dim3(SB), 0, s, (uint32_t)b, lists[b & 1],
-                           counts, q.in0, offs, T);
-        hipLaunchKernelGGL(dev::stab_keep, dim3(keep_grid), dim3(256), 0, s, lists[b & 1], counts + 1 + b,
-                           lists[(b + 1) & 1], counts + 2 + b);
+    for (int b = 0; b <= dev::kStabBatches; ++b) {
+        uint32_t* list = lists[b == 0 ? 0 : (b - 1) & 1];
+        if (q.n < (b == 0 ? kWaveMax : kStabWaveMax))
+            hipLaunchKernelGGL(dev::stab_wave, dim3((unsigned)std::min<int64_t>(q.n * (b == 0 ? 1 : 20), kStabWaveBlocks)),
+                               dim3(64), 0, s, (uint32_t)b, list, counts, q.in0, offs, T);
+        else if (b == 0)
+            hipLaunchKernelGGL((dev::stab_first<SB, kLdsEntries>), dim3(first_grid), dim3(SB), 0, s, q.order, list, counts,
+                               q.in0, offs, T, xcd_chunk_for(first_grid));
+        else
+            hipLaunchKernelGGL((dev::stab_lines<SB, kLdsEntries>), dim3(grid), dim3(SB), 0, s, (uint32_t)(b - 1), list, counts,
+                               q.in0, offs, T);
+        if (b > 0)
+            hipLaunchKernelGGL(dev::stab_keep, dim3(keep_grid), dim3(256), 0, s, list, counts + b, lists[b & 1],
+                               counts + 1 + b);
     }
     hipLaunchKernelGGL(dev::stab_negate, dim3(keep_grid), dim3(256), 0, s, lists[dev::kStabBatches & 1],
                        counts + 1 + dev::kStabBatches, q.out_f);

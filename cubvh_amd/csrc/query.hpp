@@ -59,7 +59,7 @@ size_t rest_bytes(int64_t n);
 hipError_t launch_distance(const QueryArgs& q, int mode);
 hipError_t launch_ray(const QueryArgs& q);
 // Negates q.out_f[i] of every query whose 64 raystab rays all hit (distances from mode 0),
-// walking the queries of q.order (required, n < 2^32) in passes over the undecided ones;
+// walking the queries of q.order (required from kWaveMax on, n < 2^31) in passes over the undecided ones;
 // ws holds stab_workspace_bytes(q.n) bytes.
 size_t stab_workspace_bytes(int64_t n);
 hipError_t launch_stab_sign(const QueryArgs& q, void* ws);

@@ -371,6 +371,85 @@ __device__ void closest_hit_wave(const Tree& T, f3 o, f3 d, WaveLists& L, float&
     }
 }
 
+// any_hit_line over one wave (wave-uniform arguments and result).  A pending entry's key
+// holds the directions it is open for in its two low bits; open1 / open2 count the entries
+// open for +d / -d: the pair is decided when a direction not hit yet has none left.
+__device__ int any_hit_line_wave(const Tree& T, f3 o, f3 d, WaveLists& L) {
+    const int lane = (int)(threadIdx.x & 63);
+    const f3 inv = ray_inverse(d);
+    const float limit = MAX_DIST * BOUND_SLACK;
+    int found = 0, open1 = 1, open2 = 1;
+    WaveWork w{L};
+    w.start(0);
+    L.key[0] = __uint_as_float(3u);
+    wave_fence();
+    for (;;) {
+        const uint32_t want = 3u & ~(uint32_t)found;
+        if (w.sp > 0 && w.nl < kWaveLeaves) {
+            const int quad = lane >> 2;
+            const int take = min(w.sp > kWaveChunk ? 1 : min(kWaveNodes, (64 - w.nl) >> 2), w.sp);
+            bool on = quad < take;
+            int32_t node = 0, ref = CHILD_EMPTY;
+            uint32_t dirs = 0;
+            if (on) {
+                node = L.ref[w.sp - 1 - quad];
+                dirs = __float_as_uint(L.key[w.sp - 1 - quad]) & 3u;
+            }
+            w.sp -= take;
+            const bool first = (lane & 3) == 0;  // one lane of the quad accounts for the entry
+            open1 -= __builtin_popcountll(ballot(first && (dirs & 1u)));
+            open2 -= __builtin_popcountll(ballot(first && (dirs & 2u)));
+            wave_fence();
+            on = on && (dirs & want) != 0;
+            uint32_t m = 0;
+            if (on) {
+                const LaneChild c = load_child(T.nodes, node, lane & 3);
+                ref = c.ref;
+                const float tx0 = (c.lx - o.x) * inv.x, tx1 = (c.hx - o.x) * inv.x;
+                const float ty0 = (c.ly - o.y) * inv.y, ty1 = (c.hy - o.y) * inv.y;
+                const float tz0 = (c.lz - o.z) * inv.z, tz1 = (c.hz - o.z) * inv.z;
+                const float tn = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fminf(tz0, tz1));
+                const float tf = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fmaxf(tz0, tz1));
+                if (ref != CHILD_EMPTY && tn <= tf)
+                    m = ((tf >= 0.0f && tn <= limit ? 1u : 0u) | (tn <= 0.0f && tf >= -limit ? 2u : 0u)) & want & dirs;
+            }
+            on = m != 0;
+            open1 += __builtin_popcountll(ballot(m & 1u));
+            open2 += __builtin_popcountll(ballot(m & 2u));
+            const uint64_t lm = ballot(on && ref < 0), im = ballot(on && ref >= 0);
+            append_ordered(L.leaf, L.lkey, w.nl, lm, 0, ref, __uint_as_float(m));
+            append_ordered(L.ref, L.key, w.sp, im, 0, ref, __uint_as_float(m));
+            w.nl += __builtin_popcountll(lm);
+            w.sp += __builtin_popcountll(im);
+            wave_fence();
+        } else {  // leaves: one of the two lists has an entry, or a count would be zero
+            const int take = min(kWaveLeaves, w.nl), g = lane >> 4;
+            int32_t slot = -1;
+            uint32_t dirs = 0;
+            if (g < take) {
+                const int32_t leaf = L.leaf[w.nl - 1 - g];
+                dirs = __float_as_uint(L.lkey[w.nl - 1 - g]) & 3u;
+                if ((lane & 15) < leaf_ref_count(leaf)) slot = leaf_ref_first(leaf) + (lane & 15);
+            }
+            w.nl -= take;
+            const bool first = (lane & 15) == 0;
+            open1 -= __builtin_popcountll(ballot(first && (dirs & 1u)));
+            open2 -= __builtin_popcountll(ballot(first && (dirs & 2u)));
+            uint32_t hit = 0;
+            if (slot >= 0 && (dirs & want) != 0) {
+                f3 a, b, c;
+                int32_t id;
+                load_tri(T.tris, slot, a, b, c, id);
+                hit = (uint32_t)tri_line(a, b, c, o, d, MAX_DIST) & dirs;
+            }
+            found |= (ballot(hit & 1u) != 0 ? 1 : 0) | (ballot(hit & 2u) != 0 ? 2 : 0);
+            wave_fence();
+        }
+        if (found == 3) return 3;
+        if ((!(found & 1) && open1 == 0) || (!(found & 2) && open2 == 0)) return found;
+    }
+}
+
 // Query q at p from a candidate (d2, slot; slot < 0: none) to its outputs, by one wave.
 template <int MODE>
 __device__ __forceinline__ void wave_query(const Tree& T, int32_t root, int32_t face0_slot, int64_t q, f3 p, float d2,

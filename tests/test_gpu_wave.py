@@ -76,3 +76,20 @@ def test_wave_results_at_the_size_limit(gpu, kind):
     hits = bvh.ray_trace(o, d)
     for part in (slice(0, m), slice(n - m, n)):
         _same([t[part] for t in hits], bvh.ray_trace(o[part], d[part]))
+
+
+@pytest.mark.parametrize("kind", ["nine", "soup", "copies", "closed"])
+def test_raystab_sizes_agree(gpu, oracle, kind):
+    """Raystab signs with lines by waves (small calls), by lanes and waves (from 2^18) and by
+    lanes (from 2^20) on the same leading queries (a query's directions depend on its index),
+    and against the oracle."""
+    v, f = S.icosphere(3, 0.5) if kind == "closed" else _mesh(kind)
+    bvh = cubvh_amd.cuBVH(v, f)
+    p = _points((1 << 20) + 77 if kind != "copies" else WAVE_MAX + 77)
+    p[5:400] *= 0.3
+    big = bvh.signed_distance(p, mode="raystab")[:2]
+    for n in (1, 65, 2049, WAVE_MAX - 1, WAVE_MAX + 1):
+        _same(bvh.signed_distance(p[:n], mode="raystab")[:2], [t[:n] for t in big])
+    od, of, _ = oracle.sdf_brute(v, f, p[5:500].cpu().numpy(), 1, return_uvw=False)
+    np.testing.assert_array_equal(big[0][5:500].cpu().numpy(), od)
+    np.testing.assert_array_equal(big[1][5:500].cpu().numpy(), of)
