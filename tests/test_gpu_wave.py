@@ -78,6 +78,40 @@ def test_wave_results_at_the_size_limit(gpu, kind):
         _same([t[part] for t in hits], bvh.ray_trace(o[part], d[part]))
 
 
+@pytest.mark.parametrize("scale", [1.0, 1e-3, 1e9])
+@pytest.mark.parametrize("kind", ["nine", "soup", "copies", "flat"])
+def test_ray_packets_equal_waves(gpu, kind, scale):
+    """Parallel and pinhole rays (packets) from outside, from a face and along a face's plane
+    against the same rays in calls small enough for a wave each.  A ray in a face's plane
+    can meet it at a rounded t before the mesh's own box; which of several copies of the face
+    it then reports is the order of the walk's, so such hits' face ids are not compared."""
+    v, f = _mesh(kind)
+    bvh = cubvh_amd.cuBVH(v, f)
+    x = torch.linspace(-0.6, 0.6, 181, device=gpu)
+    g = torch.stack(torch.meshgrid(x, x, indexing="ij"), dim=-1).reshape(-1, 2)
+    t = torch.from_numpy(v[f[1]]).to(gpu)
+    edge = t[1] - t[0]
+    z = torch.ones_like(g[:, :1])
+    eye = torch.tensor([0.3, -0.2, 1.7], device=gpu)
+    o = [torch.cat([g, 3.0 * z], 1), eye.expand(len(g), 3), (t[0] - 2.0 * edge).expand(len(g), 3) + 1e-7 * torch.cat([g, z], 1),
+         t.mean(0).expand(len(g), 3)]
+    d = [torch.tensor([0.0, 0.0, -1.0], device=gpu).expand(len(g), 3), torch.cat([0.4 * g, -1.7 * z], 1),
+         edge / edge.norm() + 1e-4 * torch.cat([g, z], 1), torch.cat([0.1 * g, z], 1)]
+    rep = WAVE_MAX // (4 * len(g)) + 1
+    o, d = torch.cat(o).repeat(rep, 1).contiguous(), (torch.cat(d) * scale).repeat(rep, 1).contiguous()
+    assert len(o) >= WAVE_MAX
+    whole = bvh.ray_trace(o, d)
+    lo, hi = (torch.from_numpy(e).to(gpu) for e in (v[f].min(axis=(0, 1)) - 1e-3, v[f].max(axis=(0, 1)) + 1e-3))
+    off = (whole[1] >= 0) & ~((whole[0] >= lo) & (whole[0] <= hi)).all(dim=1)
+    assert int(off.sum()) < len(o) // 1000
+    m = 4 * len(g)
+    for at in range(0, len(o), m):
+        part = slice(at, at + m)
+        small = bvh.ray_trace(o[part], d[part])
+        _same([whole[0][part], whole[2][part]], [small[0], small[2]])
+        _same([whole[1][part][~off[part]]], [small[1][~off[part]]])
+
+
 @pytest.mark.parametrize("kind", ["nine", "soup", "copies", "closed"])
 def test_raystab_sizes_agree(gpu, oracle, kind):
     """Raystab signs with lines by waves (small calls), by lanes and waves (from 2^18) and by
