@@ -20,6 +20,14 @@
 // and corner keys pack the lattice point relative to the minimum with B bits per axis
 // (B from the measured span), so the sorts run over 3B + 2 and 3B bits, with 32-bit
 // edge keys whenever 3B + 2 <= 32 (spans up to 1022).
+//
+// Cells in strictly ascending order of (x, y, z), as a lattice scan lists them, need no
+// sort when their bounding lattice is not too sparse (dense_words_most): a bit per lattice cell
+// and a prefix count per 32 of them find a cell's neighbours and count the cells before any
+// place.  An edge is owned by its first cell; edges of one (dx, dy) of their lowest point in
+// the owner's cell ("stream") ascend with the cells, up to the neighbours along z, so a
+// vertex's number is, over the four streams, the owned edges of the cells before its place
+// and a few bits of the two cells there.  0.8 M cut cells of a 512^3 lattice: 306 -> 257 us.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 #include <stdint.h>
@@ -49,10 +57,11 @@ __device__ __forceinline__ uint32_t edge_mask_of(uint32_t c) {
     return (lo ^ rlo) | ((hi ^ rhi) << 4) | ((lo ^ hi) << 8);
 }
 
-// info: [0..2] min x y z, [3..5] max x y z (int32).
+// info: [0..2] min x y z, [3..5] max x y z (int32), [6] 1 unless the cells ascend strictly.
+constexpr int kBounds = 7;
 
 // Bounds in two steps without same-address atomics: each block writes its six extremes
-// to part[6 * block], one block folds them into info.
+// to part[kBounds * block], one block folds them into info.
 __device__ __forceinline__ void block_extremes(int32_t (&lo)[3], int32_t (&hi)[3]) {
     __shared__ int32_t sh[6][kBlock / 64];
     for (int o = 32; o > 0; o >>= 1)
@@ -80,28 +89,43 @@ __device__ __forceinline__ void block_extremes(int32_t (&lo)[3], int32_t (&hi)[3
 __global__ __launch_bounds__(kBlock) void smc_bounds(const int32_t* __restrict__ coords, int64_t n,
                                                      int32_t* __restrict__ part) {
     int32_t lo[3] = {INT_MAX, INT_MAX, INT_MAX}, hi[3] = {INT_MIN, INT_MIN, INT_MIN};
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
+    int mixed = 0;
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
+        int32_t v[3], order = i == 0 ? -1 : 0;  // of the cell before against this one
         for (int k = 0; k < 3; ++k) {
-            const int32_t v = coords[3 * i + k];
-            lo[k] = min(lo[k], v);
-            hi[k] = max(hi[k], v);
+            v[k] = coords[3 * i + k];
+            lo[k] = min(lo[k], v[k]);
+            hi[k] = max(hi[k], v[k]);
+            if (i > 0 && order == 0) {
+                const int32_t u = coords[3 * (i - 1) + k];
+                order = u < v[k] ? -1 : (u > v[k] ? 1 : 0);
+            }
         }
-    block_extremes(lo, hi);
-    if (threadIdx.x < 3) {
-        part[6 * blockIdx.x + threadIdx.x] = lo[threadIdx.x];
-        part[6 * blockIdx.x + 3 + threadIdx.x] = hi[threadIdx.x];
+        mixed |= order >= 0;
     }
+    block_extremes(lo, hi);
+    mixed = __syncthreads_or(mixed);
+    if (threadIdx.x < 3) {
+        part[kBounds * blockIdx.x + threadIdx.x] = lo[threadIdx.x];
+        part[kBounds * blockIdx.x + 3 + threadIdx.x] = hi[threadIdx.x];
+    }
+    if (threadIdx.x == 0) part[kBounds * blockIdx.x + 6] = mixed;
 }
 
 __global__ __launch_bounds__(kBlock) void smc_fold_bounds(const int32_t* __restrict__ part, int n_part,
                                                           int32_t* __restrict__ info) {
     int32_t lo[3] = {INT_MAX, INT_MAX, INT_MAX}, hi[3] = {INT_MIN, INT_MIN, INT_MIN};
-    for (int b = (int)threadIdx.x; b < n_part; b += kBlock)
+    int mixed = 0;
+    for (int b = (int)threadIdx.x; b < n_part; b += kBlock) {
         for (int k = 0; k < 3; ++k) {
-            lo[k] = min(lo[k], part[6 * b + k]);
-            hi[k] = max(hi[k], part[6 * b + 3 + k]);
+            lo[k] = min(lo[k], part[kBounds * b + k]);
+            hi[k] = max(hi[k], part[kBounds * b + 3 + k]);
         }
+        mixed |= part[kBounds * b + 6];
+    }
     block_extremes(lo, hi);
+    mixed = __syncthreads_or(mixed);
+    if (threadIdx.x == 0) info[6] = mixed;
     if (threadIdx.x < 3) {
         info[threadIdx.x] = lo[threadIdx.x];
         info[3 + threadIdx.x] = hi[threadIdx.x];
@@ -204,6 +228,31 @@ __device__ __forceinline__ uint32_t raw_slot(uint64_t offset, uint32_t mask, int
     return (uint32_t)(offset >> 32) + (uint32_t)__popc(mask & ((1u << e) - 1u));
 }
 
+// Vertex on edge e of cell i.
+// include/gpu/spcumc.cuh:455-471: t = (iso - va) / (vb - va) clamped to [0, 1] (0.5
+// on a flat edge), p = pA + t (pB - pA); t (pB - pA) is exact for lattice points
+__device__ __forceinline__ void store_vertex(const int32_t* __restrict__ coords, const float* __restrict__ corners,
+                                             int64_t i, int e, float iso, float* __restrict__ out) {
+    const int a = mc::edge_a(e), b = mc::edge_b(e);
+    const float va = corners[8 * i + a], vb = corners[8 * i + b];
+    const float denom = vb - va;
+    float t;
+    if (fabsf(denom) < 1e-30f) {
+        t = 0.5f;
+    } else {
+        t = (iso - va) / denom;
+        t = fminf(fmaxf(t, 0.0f), 1.0f);
+    }
+    const int64_t x = coords[3 * i], y = coords[3 * i + 1], z = coords[3 * i + 2];
+    const float ax = (float)(x + mc::corner_dx(a)), ay = (float)(y + mc::corner_dy(a)),
+                az = (float)(z + mc::corner_dz(a));
+    const float bx = (float)(x + mc::corner_dx(b)), by = (float)(y + mc::corner_dy(b)),
+                bz = (float)(z + mc::corner_dz(b));
+    out[0] = ax + t * (bx - ax);
+    out[1] = ay + t * (by - ay);
+    out[2] = az + t * (bz - az);
+}
+
 template <typename K>
 __global__ __launch_bounds__(kBlock) void smc_vertices(const K* __restrict__ keys, const uint32_t* __restrict__ vals,
                                                        const uint32_t* __restrict__ ids, int64_t m,
@@ -220,26 +269,7 @@ __global__ __launch_bounds__(kBlock) void smc_vertices(const K* __restrict__ key
     const int e = (int)(v & 15u);
     map[raw_slot(offsets[i], edge_mask_of(cases[i]), e)] = (int32_t)id;
     if (s > 0 && keys[s - 1] == keys[s]) return;
-    // include/gpu/spcumc.cuh:455-471: t = (iso - va) / (vb - va) clamped to [0, 1] (0.5
-    // on a flat edge), p = pA + t (pB - pA); t (pB - pA) is exact for lattice points
-    const int a = mc::edge_a(e), b = mc::edge_b(e);
-    const float va = corners[8 * i + a], vb = corners[8 * i + b];
-    const float denom = vb - va;
-    float t;
-    if (fabsf(denom) < 1e-30f) {
-        t = 0.5f;
-    } else {
-        t = (iso - va) / denom;
-        t = fminf(fmaxf(t, 0.0f), 1.0f);
-    }
-    const int64_t x = coords[3 * i], y = coords[3 * i + 1], z = coords[3 * i + 2];
-    const float ax = (float)(x + mc::corner_dx(a)), ay = (float)(y + mc::corner_dy(a)),
-                az = (float)(z + mc::corner_dz(a));
-    const float bx = (float)(x + mc::corner_dx(b)), by = (float)(y + mc::corner_dy(b)),
-                bz = (float)(z + mc::corner_dz(b));
-    verts[3 * (int64_t)id] = ax + t * (bx - ax);
-    verts[3 * (int64_t)id + 1] = ay + t * (by - ay);
-    verts[3 * (int64_t)id + 2] = az + t * (bz - az);
+    store_vertex(coords, corners, i, e, iso, verts + 3 * (int64_t)id);
 }
 
 __global__ __launch_bounds__(kBlock) void smc_triangles(const uint8_t* __restrict__ cases,
@@ -261,6 +291,215 @@ __global__ __launch_bounds__(kBlock) void smc_triangles(const uint8_t* __restric
         o[3 * t] = map[raw_slot(off, mask, e0)];
         o[3 * t + 1] = map[raw_slot(off, mask, e2)];
         o[3 * t + 2] = map[raw_slot(off, mask, e1)];
+    }
+}
+
+// ---- ascending cells: no sort
+// The cells' bounding lattice, one cell wider on every side: bits[w] holds a bit per cell
+// of 32 along z, before[w] the cells in the words below w.
+struct Lattice {
+    int32_t mn[3];
+    int32_t ny, zw;  // rows per x, words per row
+    const uint32_t* bits;
+    const uint32_t* before;
+};
+
+// Row of (x, y) and place along z, x .. z within one cell of the bounds.
+__device__ __forceinline__ uint32_t lattice_row(const Lattice& L, int64_t x, int64_t y) {
+    return (uint32_t)(x - L.mn[0] + 1) * (uint32_t)L.ny + (uint32_t)(y - L.mn[1] + 1);
+}
+__device__ __forceinline__ uint32_t lattice_z(const Lattice& L, int64_t z) { return (uint32_t)(z - L.mn[2] + 1); }
+
+// Cells before place z of a row, whether that place holds one, and whether the next does.
+struct Place {
+    uint32_t at;
+    bool here, next;
+};
+__device__ __forceinline__ Place place_of(const Lattice& L, uint32_t row, uint32_t z) {
+    const uint32_t w = row * (uint32_t)L.zw + (z >> 5), b = z & 31u, m = L.bits[w];
+    Place p;
+    p.at = L.before[w] + (uint32_t)__popc(m & ((1u << b) - 1u));
+    p.here = (m >> b) & 1u;
+    p.next = b < 31u ? (m >> (b + 1u)) & 1u : (z + 1u < 32u * (uint32_t)L.zw ? L.bits[w + 1] & 1u : 0u);
+    return p;
+}
+
+// A cell's edges as 4 bits per axis (x, y, z from the least significant): bit u + 2 v for
+// the edge whose lowest point lies (u, v) along the other two axes in their order.
+__device__ __forceinline__ int edge_bit(int e) {
+    const int a = mc::edge_a(e), b = mc::edge_b(e), axis = mc::edge_axis(e);
+    const int x = min(mc::corner_dx(a), mc::corner_dx(b)), y = min(mc::corner_dy(a), mc::corner_dy(b)),
+              z = min(mc::corner_dz(a), mc::corner_dz(b));
+    return 4 * axis + (axis == 0 ? y : x) + 2 * (axis == 2 ? y : z);
+}
+// Streams s = dx + 2 dy, and the edges whose lowest point is at dz = 0 / 1.
+__device__ __forceinline__ uint32_t stream_mask(int s) { return s == 0 ? 0x155u : s == 1 ? 0x2a0u : s == 2 ? 0x40au : 0x800u; }
+constexpr uint32_t kLowZ = 0xf33u, kHighZ = 0x0ccu;
+
+// Owned edges per stream: of a cell, or of all cells before it.
+struct alignas(16) CellSums {
+    uint32_t edge[4];
+};
+struct AddSums {
+    __host__ __device__ CellSums operator()(const CellSums& a, const CellSums& b) const {
+        CellSums r;
+        for (int k = 0; k < 4; ++k) r.edge[k] = a.edge[k] + b.edge[k];
+        return r;
+    }
+};
+struct WordCells {
+    const uint32_t* bits;
+    __device__ uint32_t operator()(int64_t w) const { return (uint32_t)__popc(bits[w]); }
+};
+
+__global__ __launch_bounds__(kBlock) void smc_clear(uint32_t* __restrict__ p, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) p[i] = 0u;
+}
+
+// The first cell of each word writes the word.
+__global__ __launch_bounds__(kBlock) void smc_mark(const int32_t* __restrict__ coords, int64_t n, Lattice L,
+                                                   uint32_t* __restrict__ bits) {
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    auto word = [&](int64_t j, uint32_t& b) {
+        const uint32_t z = lattice_z(L, coords[3 * j + 2]);
+        b = z & 31u;
+        return lattice_row(L, coords[3 * j], coords[3 * j + 1]) * (uint32_t)L.zw + (z >> 5);
+    };
+    uint32_t b, u;
+    const uint32_t w = word(i, b);
+    if (i > 0 && word(i - 1, u) == w) return;
+    uint32_t m = 1u << b;
+    for (int64_t j = i + 1; j < n && word(j, u) == w; ++j) m |= 1u << u;
+    bits[w] = m;
+}
+
+// Corner means: the up to eight cells around a lattice point in ascending order.
+__global__ __launch_bounds__(kBlock) void smc_dense_mean(const int32_t* __restrict__ coords, int64_t n, Lattice L,
+                                                         const float* __restrict__ corners, float* __restrict__ out) {
+    const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (j >= 8 * n) return;
+    const int64_t i = j >> 3;
+    const int k = (int)(j & 7);
+    const int64_t x = (int64_t)coords[3 * i] + mc::corner_dx(k), y = (int64_t)coords[3 * i + 1] + mc::corner_dy(k),
+                  z = (int64_t)coords[3 * i + 2] + mc::corner_dz(k);
+    double sum = 0.0;
+    int cnt = 0;
+    for (int dx = 1; dx >= 0; --dx)
+        for (int dy = 1; dy >= 0; --dy) {
+            const Place p = place_of(L, lattice_row(L, x - dx, y - dy), lattice_z(L, z - 1));
+            const int c = dy ? (dx ? 2 : 3) : dx;  // the point's corner of a cell at dz = 0
+            if (p.here) {
+                sum += (double)corners[8 * (int64_t)p.at + 4 + c];
+                ++cnt;
+            }
+            if (p.next) {
+                sum += (double)corners[8 * ((int64_t)p.at + p.here) + c];
+                ++cnt;
+            }
+        }
+    out[j] = (float)(sum / (double)cnt);
+}
+
+// own[i]: the edge bits of cell i that no earlier cell has; counts[i] (counts[n] is zero).
+__global__ __launch_bounds__(kBlock) void smc_own_edges(const int32_t* __restrict__ coords,
+                                                        const uint8_t* __restrict__ cases, int64_t n, Lattice L,
+                                                        uint16_t* __restrict__ own, CellSums* __restrict__ counts) {
+    __shared__ uint16_t bits_of[256];  // edge bits of every case
+    static_assert(kBlock == 256, "one case per thread");
+    uint32_t of = 0;
+#pragma unroll
+    for (int e = 0; e < 12; ++e)
+        of |= (((threadIdx.x >> mc::edge_a(e)) ^ (threadIdx.x >> mc::edge_b(e))) & 1u) << edge_bit(e);
+    bits_of[threadIdx.x] = (uint16_t)of;
+    __syncthreads();
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i > n) return;
+    CellSums t = {{0u, 0u, 0u, 0u}};
+    if (i < n) {
+        uint32_t m = bits_of[cases[i]];
+        if (m) {
+            const int64_t x = coords[3 * i], y = coords[3 * i + 1];
+            const uint32_t z = lattice_z(L, coords[3 * i + 2]);
+            // edge bits of the cells at z - 1, z, z + 1 of a row
+            auto row = [&](int64_t rx, int64_t ry, uint32_t& below, uint32_t& level, uint32_t& above) {
+                const uint32_t r = lattice_row(L, rx, ry);
+                const Place p = place_of(L, r, z - 1);
+                const uint32_t w = r * (uint32_t)L.zw + ((z + 1) >> 5);
+                const bool top = (L.bits[w] >> ((z + 1) & 31u)) & 1u;
+                below = p.here ? bits_of[cases[p.at]] : 0u;
+                level = p.next ? bits_of[cases[p.at + p.here]] : 0u;
+                above = top ? bits_of[cases[p.at + p.here + p.next]] : 0u;
+            };
+            uint32_t b, l, a;
+            row(x - 1, y, b, l, a);
+            m &= ~((l >> 1) & 0x550u);   // shared face: y and z edges at dx = 0
+            m &= ~((b >> 3) & 0x010u);   // one y edge each
+            m &= ~((a << 1) & 0x040u);
+            row(x - 1, y - 1, b, l, a);
+            m &= ~((l >> 3) & 0x100u);   // one z edge
+            row(x - 1, y + 1, b, l, a);
+            m &= ~((l << 1) & 0x400u);
+            row(x, y - 1, b, l, a);
+            m &= ~((l >> 1) & 0x005u);   // shared face: x edges at dy = 0
+            m &= ~((l >> 2) & 0x300u);   // and z edges
+            m &= ~((b >> 3) & 0x001u);   // one x edge each
+            m &= ~((a << 1) & 0x004u);
+            row(x, y, b, l, a);
+            m &= ~((b >> 2) & 0x033u);   // shared face: x and y edges at dz = 0
+#pragma unroll
+            for (int s = 0; s < 4; ++s) t.edge[s] = (uint32_t)__popc(m & stream_mask(s));
+        }
+        own[i] = (uint16_t)m;
+    }
+    counts[i] = t;
+}
+
+// Number of the vertex of the edge along `axis` from lattice point (x, y, z).
+__device__ __forceinline__ uint32_t vertex_number(const Lattice& L, const uint16_t* __restrict__ own,
+                                                  const CellSums* __restrict__ sums, int64_t x, int64_t y, int64_t z,
+                                                  int axis) {
+    const uint32_t lower = (1u << (4 * axis)) - 1u;  // the axes before
+    uint32_t id = 0;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const Place p = place_of(L, lattice_row(L, x - (s & 1), y - (s >> 1)), lattice_z(L, z - 1));
+        id += sums[p.at].edge[s];
+        if (p.here) id += (uint32_t)__popc(own[p.at] & stream_mask(s) & (kLowZ | (kHighZ & lower)));
+        if (p.next) id += (uint32_t)__popc(own[p.at + p.here] & stream_mask(s) & kLowZ & lower);
+    }
+    return id;
+}
+
+// A thread per cell: its edges' vertex numbers, the vertices it owns, its triangles.
+__global__ __launch_bounds__(kBlock) void smc_dense_write(const int32_t* __restrict__ coords,
+                                                          const float* __restrict__ corners,
+                                                          const uint8_t* __restrict__ cases,
+                                                          const uint64_t* __restrict__ offsets, int64_t n, Lattice L,
+                                                          const uint16_t* __restrict__ own,
+                                                          const CellSums* __restrict__ sums, float iso,
+                                                          float* __restrict__ verts, int32_t* __restrict__ tris) {
+    __shared__ int32_t id[12][kBlock];
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t c = cases[i], mine = own[i];
+    const int64_t x = coords[3 * i], y = coords[3 * i + 1], z = coords[3 * i + 2];
+    for (uint32_t m = edge_mask_of(c); m; m &= m - 1) {
+        const int e = __ffs(m) - 1, a = mc::edge_a(e), b = mc::edge_b(e);
+        const uint32_t v = vertex_number(L, own, sums, x + min(mc::corner_dx(a), mc::corner_dx(b)),
+                                         y + min(mc::corner_dy(a), mc::corner_dy(b)),
+                                         z + min(mc::corner_dz(a), mc::corner_dz(b)), mc::edge_axis(e));
+        id[e][threadIdx.x] = (int32_t)v;
+        if ((mine >> edge_bit(e)) & 1u) store_vertex(coords, corners, i, e, iso, verts + 3 * (int64_t)v);
+    }
+    const uint64_t packed = c_triangles[c];
+    const int nt = mc::triangle_count(packed);
+    int32_t* o = tris + 3 * (int64_t)(uint32_t)offsets[i];
+    for (int t = 0; t < nt; ++t) {
+        o[3 * t] = id[mc::triangle_edge(packed, 3 * t)][threadIdx.x];
+        o[3 * t + 1] = id[mc::triangle_edge(packed, 3 * t + 2)][threadIdx.x];
+        o[3 * t + 2] = id[mc::triangle_edge(packed, 3 * t + 1)][threadIdx.x];
     }
 }
 
@@ -347,6 +586,13 @@ struct SmcState {
     uint32_t* vals = nullptr;  // sorted (cell, edge)
     uint32_t* ids = nullptr;   // vertex id + 1 per sorted position
     int32_t* map = nullptr;    // raw slot -> vertex id
+    // ascending cells
+    bool dense = false;
+    Lattice lattice = {};
+    uint16_t* own = nullptr;   // edge bits owned
+    CellSums* counts = nullptr;
+    CellSums* sums = nullptr;  // exclusive, n + 1 of them
+    char* sums_tmp = nullptr;
 };
 
 namespace {
@@ -458,6 +704,66 @@ void launch_vertices(const SmcState* st, float* verts, hipStream_t s) {
                        st->map);
 }
 
+// Words of the bounding lattice's bits up to which ascending cells go without the sort (a
+// word costs some 12 bytes of traffic, the sort's passes over a cell's edges about 300).
+int64_t dense_words_most(int64_t n) { return 8 * n + (1 << 14); }
+
+using WordIter = hipcub::TransformInputIterator<uint32_t, WordCells, hipcub::CountingInputIterator<int64_t>>;
+
+size_t word_scan_bytes(int64_t words) {
+    size_t b = 0;
+    WordIter it(hipcub::CountingInputIterator<int64_t>(0), WordCells{nullptr});
+    hipcub::DeviceScan::ExclusiveSum(nullptr, b, it, (uint32_t*)nullptr, (int)words);
+    return b;
+}
+
+size_t sums_scan_bytes(int64_t m) {
+    size_t b = 0;
+    hipcub::DeviceScan::ExclusiveScan(nullptr, b, (const CellSums*)nullptr, (CellSums*)nullptr, AddSums(), CellSums{{0, 0, 0, 0}},
+                                      (int)m);
+    return b;
+}
+
+// Region B of ascending cells, and their lattice's bits and prefix counts.
+hipError_t dense_lattice(SmcState* st, int64_t words, hipStream_t s) {
+    const int64_t n = st->n;
+    const size_t wbytes = word_scan_bytes(words), sbytes = sums_scan_bytes(n + 1);
+    uint32_t *bits, *before;
+    char* tmp;
+    auto lay = [&](Carve& c) {
+        bits = c.take<uint32_t>(words);
+        before = c.take<uint32_t>(words);
+        st->own = c.take<uint16_t>(n);
+        st->counts = c.take<CellSums>(n + 1);
+        st->sums = c.take<CellSums>(n + 1);
+        tmp = c.take<char>((int64_t)wbytes);
+        st->sums_tmp = c.take<char>((int64_t)sbytes);
+    };
+    Carve size;
+    lay(size);
+    Carve c;
+    hipError_t e = region(st, 1, size.used, s, &c.base);
+    if (e != hipSuccess) return e;
+    lay(c);
+    st->lattice.bits = bits;
+    st->lattice.before = before;
+    hipLaunchKernelGGL(smc_clear, dim3(blocks_for(words)), dim3(kBlock), 0, s, bits, words);
+    hipLaunchKernelGGL(smc_mark, dim3(blocks_for(n)), dim3(kBlock), 0, s, st->coords, n, st->lattice, bits);
+    WordIter it(hipcub::CountingInputIterator<int64_t>(0), WordCells{bits});
+    size_t bytes = wbytes;
+    return hipcub::DeviceScan::ExclusiveSum(tmp, bytes, it, before, (int)words, s);
+}
+
+// The owned edges of ascending cells (classified) and their sums.
+hipError_t dense_edges(SmcState* st, hipStream_t s) {
+    const int64_t n = st->n;
+    hipLaunchKernelGGL(smc_own_edges, dim3(blocks_for(n + 1)), dim3(kBlock), 0, s, st->coords, st->cases, n, st->lattice,
+                       st->own, st->counts);
+    size_t bytes = sums_scan_bytes(n + 1);
+    return hipcub::DeviceScan::ExclusiveScan(st->sums_tmp, bytes, st->counts, st->sums, AddSums(), CellSums{{0, 0, 0, 0}},
+                                             (int)(n + 1), s);
+}
+
 // Copies `bytes` from the device once the stream's work is done (through pinned memory
 // when the extraction owns the shared scratch).
 hipError_t read_back(SmcState* st, const void* src, size_t bytes, void* dst, hipStream_t s) {
@@ -531,7 +837,7 @@ SmcStatus smc_extract(const int32_t* coords, const float* corners, int64_t n, fl
     Carve corner_area;
     auto lay_a = [&](Carve& c) {
         st->info = c.take<int32_t>(16);
-        part = c.take<int32_t>(6 * (int64_t)nb);
+        part = c.take<int32_t>(kBounds * (int64_t)nb);
         st->cases = c.take<uint8_t>(n);
         counts = c.take<uint64_t>(n);
         st->offsets = c.take<uint64_t>(n);
@@ -569,14 +875,34 @@ SmcStatus smc_extract(const int32_t* coords, const float* corners, int64_t n, fl
         B = bits_for(span + 1);  // lattice points min .. max + 1
         return SmcStatus();
     };
+    // ascending cells whose bounding lattice is dense enough need no sort
+    auto try_dense = [&]() {
+        const int64_t nx = (int64_t)info[3] - info[0] + 3, ny = (int64_t)info[4] - info[1] + 3,
+                      zw = ((int64_t)info[5] - info[2] + 3 + 31) / 32;
+        const int64_t most = dense_words_most(n);
+        if (info[6] != 0 || nx * ny > most || nx * ny * zw > most) return hipSuccess;
+        st->dense = true;
+        for (int k = 0; k < 3; ++k) st->lattice.mn[k] = info[k];
+        st->lattice.ny = (int32_t)ny;
+        st->lattice.zw = (int32_t)zw;
+        return dense_lattice(st, nx * ny * zw, s);
+    };
     if (consistent) {
-        // the corner sort needs the key width before the cells are classified
-        e = read_back(st, st->info, 6 * sizeof(int32_t), info, s);
+        // the corners' means need the lattice or the key width before the cells are classified
+        e = read_back(st, st->info, kBounds * sizeof(int32_t), info, s);
         if (e != hipSuccess) return bail(hip_status(e, "cell bounds"));
         SmcStatus r = read_bounds();
         if (r.code) return bail(r);
-        e = 3 * B <= 32 ? average_corners<uint32_t>(st, corner_area, B, mean, s)
-                        : average_corners<uint64_t>(st, corner_area, B, mean, s);
+        e = try_dense();
+        if (e != hipSuccess) return bail(hip_status(e, "cell lattice"));
+        if (st->dense) {
+            hipLaunchKernelGGL(smc_dense_mean, dim3(blocks_for(8 * n)), dim3(kBlock), 0, s, coords, n, st->lattice, corners,
+                               mean);
+            e = hipGetLastError();
+        } else {
+            e = 3 * B <= 32 ? average_corners<uint32_t>(st, corner_area, B, mean, s)
+                            : average_corners<uint64_t>(st, corner_area, B, mean, s);
+        }
         if (e != hipSuccess) return bail(hip_status(e, "corner averaging"));
         st->corners = mean;
     }
@@ -604,6 +930,23 @@ SmcStatus smc_extract(const int32_t* coords, const float* corners, int64_t n, fl
         return SmcStatus();
     }
 
+    if (!consistent) {
+        e = try_dense();
+        if (e != hipSuccess) return bail(hip_status(e, "cell lattice"));
+    }
+    if (st->dense) {
+        e = dense_edges(st, s);
+        if (e != hipSuccess) return bail(hip_status(e, "edge numbering"));
+        CellSums all;
+        e = read_back(st, st->sums + n, sizeof all, &all, s);
+        if (e != hipSuccess) return bail(hip_status(e, "vertex count"));
+        for (int k = 0; k < 4; ++k) st->m += all.edge[k];
+        *out = st;
+        *n_verts = st->m;
+        *n_tris = st->t;
+        return SmcStatus();
+    }
+
     // region B: edge keys in cell order, stable sort, vertex ids from run starts
     st->wide = 3 * B + 2 > 32;
     e = st->wide ? order_edges<uint64_t>(st, B, s) : order_edges<uint32_t>(st, B, s);
@@ -620,7 +963,12 @@ SmcStatus smc_extract(const int32_t* coords, const float* corners, int64_t n, fl
 
 SmcStatus smc_write(SmcState* st, float* verts, int32_t* tris, hipStream_t s) {
     SmcStatus r;
-    if (st->m_raw > 0) {
+    if (st->dense) {
+        if (st->m > 0)
+            hipLaunchKernelGGL(smc_dense_write, dim3(blocks_for(st->n)), dim3(kBlock), 0, s, st->coords, st->corners, st->cases,
+                               st->offsets, st->n, st->lattice, st->own, st->sums, st->iso, verts, tris);
+        r = hip_status(hipGetLastError(), "marching cubes kernel launch");
+    } else if (st->m_raw > 0) {
         if (st->wide)
             launch_vertices<uint64_t>(st, verts, s);
         else

@@ -79,6 +79,23 @@ def test_dense_block_with_every_cell_equals_oracle():
     _check(coords, corners, 0.0, True)
 
 
+@pytest.mark.parametrize("consistent", [False, True])
+@pytest.mark.parametrize("keep", [0.2, 0.7, 1.0])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (1, 40, 1), (3, 5, 30), (2, 7, 31), (5, 3, 32), (1, 2, 95), (9, 9, 65)])
+def test_ascending_cells_equal_oracle(dims, keep, consistent):
+    """Cells in lattice order with holes (no sort), the same ones with the last repeated and in
+    descending order (sorted keys); values that differ between cells sharing a point."""
+    rng = np.random.default_rng(dims[0] * 1000 + dims[2])
+    coords = np.argwhere(rng.random(dims) < keep).astype(np.int32) + np.array([-7, 2000, -31], np.int32)
+    if len(coords) == 0:
+        coords = np.array([[4, -5, 6]], np.int32)
+    corners = rng.normal(size=(len(coords), 8)).astype(np.float32)
+    corners[rng.random(corners.shape) < 0.05] = 0.1
+    _check(coords, corners, 0.1, consistent)
+    _check(np.concatenate([coords, coords[-1:]]), np.concatenate([corners, corners[:1]]), 0.1, consistent)
+    _check(coords[::-1].copy(), corners[::-1].copy(), 0.1, consistent)
+
+
 def test_empty_and_uncut():
     V, T = _gpu(np.zeros((0, 3), np.int32), np.zeros((0, 8), np.float32), 0.0)
     assert V.shape == (0, 3) and T.shape == (0, 3)
