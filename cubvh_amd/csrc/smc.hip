@@ -22,12 +22,16 @@
 // edge keys whenever 3B + 2 <= 32 (spans up to 1022).
 //
 // Cells in strictly ascending order of (x, y, z), as a lattice scan lists them, need no
-// sort when their bounding lattice is not too sparse (dense_words_most): a bit per lattice cell
-// and a prefix count per 32 of them find a cell's neighbours and count the cells before any
-// place.  An edge is owned by its first cell; edges of one (dx, dy) of their lowest point in
-// the owner's cell ("stream") ascend with the cells, up to the neighbours along z, so a
-// vertex's number is, over the four streams, the owned edges of the cells before its place
-// and a few bits of the two cells there.  0.8 M cut cells of a 512^3 lattice: 306 -> 257 us.
+// sort when their bounding lattice is not too sparse (dense_words_most): a bit per lattice
+// cell and a prefix count per 32 of them find a cell's neighbours and count the cells before
+// any place.  An edge is owned by its first cell; edges of one (dx, dy) of their lowest
+// point in the owner's cell ("stream") ascend with the cells, up to the neighbours along z,
+// so a vertex's number is, over the four streams, the owned edges of the cells before its
+// place and a few bits of the two cells there.  Only owners compute it; the other cells of
+// an edge keep the owner's slot.  Latency of the gathers bounds these kernels.  Cut cells of
+// a lattice: 742,270 307 -> 198 us (257 with every cell computing the numbers of all its
+// edges), 174,056 231 -> 116, 3,850 142 -> 115; with averaged corners 454,180 515 -> 208.
+// Cells in random order are sorted as before: 742,270 340 -> 345, 25,542 158 -> 156.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 #include <stdint.h>
@@ -326,27 +330,37 @@ __device__ __forceinline__ Place place_of(const Lattice& L, uint32_t row, uint32
 
 // A cell's edges as 4 bits per axis (x, y, z from the least significant): bit u + 2 v for
 // the edge whose lowest point lies (u, v) along the other two axes in their order.
-__device__ __forceinline__ int edge_bit(int e) {
+__host__ __device__ constexpr int edge_bit(int e) {
     const int a = mc::edge_a(e), b = mc::edge_b(e), axis = mc::edge_axis(e);
-    const int x = min(mc::corner_dx(a), mc::corner_dx(b)), y = min(mc::corner_dy(a), mc::corner_dy(b)),
-              z = min(mc::corner_dz(a), mc::corner_dz(b));
+    const int x = mc::corner_dx(a) & mc::corner_dx(b), y = mc::corner_dy(a) & mc::corner_dy(b),
+              z = mc::corner_dz(a) & mc::corner_dz(b);
     return 4 * axis + (axis == 0 ? y : x) + 2 * (axis == 2 ? y : z);
 }
+// Edge bits of the 12 edges, and edges of the 12 bits, 4 bits each.
+constexpr uint64_t edge_table(bool inverse) {
+    uint64_t t = 0;
+    for (int e = 0; e < 12; ++e) t |= (uint64_t)(inverse ? e : edge_bit(e)) << (4 * (inverse ? edge_bit(e) : e));
+    return t;
+}
+constexpr uint64_t kBitOfEdge = edge_table(false), kEdgeOfBit = edge_table(true);
+__device__ __forceinline__ int nibble(uint64_t table, int k) { return (int)((table >> (4 * k)) & 15u); }
+__device__ __forceinline__ uint32_t bits_below(uint32_t m, int k) { return (uint32_t)__popc(m & ((1u << k) - 1u)); }
+
 // Streams s = dx + 2 dy, and the edges whose lowest point is at dz = 0 / 1.
 __device__ __forceinline__ uint32_t stream_mask(int s) { return s == 0 ? 0x155u : s == 1 ? 0x2a0u : s == 2 ? 0x40au : 0x800u; }
 constexpr uint32_t kLowZ = 0xf33u, kHighZ = 0x0ccu;
 
-// Owned edges per stream: of a cell, or of all cells before it.
-struct alignas(16) CellSums {
-    uint32_t edge[4];
+// Owned edges per stream before a cell: `base` before its block of kBlock cells, and four
+// 16-bit counts inside the block (at most 5 kBlock each).
+static_assert(5 * kBlock < 1 << 16, "block counts fit 16 bits");
+struct OwnSums {
+    const uint4* base;
+    const uint64_t* local;
 };
-struct AddSums {
-    __host__ __device__ CellSums operator()(const CellSums& a, const CellSums& b) const {
-        CellSums r;
-        for (int k = 0; k < 4; ++k) r.edge[k] = a.edge[k] + b.edge[k];
-        return r;
-    }
-};
+__device__ __forceinline__ uint32_t own_before(const OwnSums& t, uint32_t cell, int s) {
+    const uint32_t* b = reinterpret_cast<const uint32_t*>(t.base + cell / kBlock);
+    return b[s] + (uint32_t)((t.local[cell] >> (16 * s)) & 0xffffu);
+}
 struct WordCells {
     const uint32_t* bits;
     __device__ uint32_t operator()(int64_t w) const { return (uint32_t)__popc(bits[w]); }
@@ -402,11 +416,16 @@ __global__ __launch_bounds__(kBlock) void smc_dense_mean(const int32_t* __restri
     out[j] = (float)(sum / (double)cnt);
 }
 
-// own[i]: the edge bits of cell i that no earlier cell has; counts[i] (counts[n] is zero).
+// own[i]: the edge bits of cell i that no earlier cell has; ref of each raw slot (a cell's
+// edges by edge bit, from its first slot on): the owner's slot; local and block: the owned
+// edges per stream, of the cells before in the block and of the whole block.
 __global__ __launch_bounds__(kBlock) void smc_own_edges(const int32_t* __restrict__ coords,
-                                                        const uint8_t* __restrict__ cases, int64_t n, Lattice L,
-                                                        uint16_t* __restrict__ own, CellSums* __restrict__ counts) {
+                                                        const uint8_t* __restrict__ cases,
+                                                        const uint64_t* __restrict__ offsets, int64_t n, Lattice L,
+                                                        uint16_t* __restrict__ own, uint32_t* __restrict__ ref,
+                                                        uint64_t* __restrict__ local, uint4* __restrict__ block) {
     __shared__ uint16_t bits_of[256];  // edge bits of every case
+    __shared__ uint64_t wave_sum[kBlock / 64];
     static_assert(kBlock == 256, "one case per thread");
     uint32_t of = 0;
 #pragma unroll
@@ -415,91 +434,176 @@ __global__ __launch_bounds__(kBlock) void smc_own_edges(const int32_t* __restric
     bits_of[threadIdx.x] = (uint16_t)of;
     __syncthreads();
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i > n) return;
-    CellSums t = {{0u, 0u, 0u, 0u}};
+    uint32_t m = 0;
     if (i < n) {
-        uint32_t m = bits_of[cases[i]];
+        const uint32_t mask = bits_of[cases[i]];
+        m = mask;
         if (m) {
+            const uint32_t slot = (uint32_t)(offsets[i] >> 32);
             const int64_t x = coords[3 * i], y = coords[3 * i + 1];
             const uint32_t z = lattice_z(L, coords[3 * i + 2]);
-            // edge bits of the cells at z - 1, z, z + 1 of a row
-            auto row = [&](int64_t rx, int64_t ry, uint32_t& below, uint32_t& level, uint32_t& above) {
-                const uint32_t r = lattice_row(L, rx, ry);
-                const Place p = place_of(L, r, z - 1);
-                const uint32_t w = r * (uint32_t)L.zw + ((z + 1) >> 5);
-                const bool top = (L.bits[w] >> ((z + 1) & 31u)) & 1u;
-                below = p.here ? bits_of[cases[p.at]] : 0u;
-                level = p.next ? bits_of[cases[p.at + p.here]] : 0u;
-                above = top ? bits_of[cases[p.at + p.here + p.next]] : 0u;
+            // the edges of `shared` that cell j has too, as its edge bits `shift` higher
+            auto claim = [&](uint32_t j, int shift, uint32_t shared) {
+                const uint32_t nb = bits_of[cases[j]];
+                uint32_t t = m & shared & (shift > 0 ? nb >> shift : nb << -shift);
+                if (!t) return;
+                m &= ~t;
+                const uint32_t first = (uint32_t)(offsets[j] >> 32);
+                for (; t; t &= t - 1) {
+                    const int k = __ffs(t) - 1;
+                    ref[slot + bits_below(mask, k)] = first + bits_below(nb, k + shift);
+                }
             };
-            uint32_t b, l, a;
-            row(x - 1, y, b, l, a);
-            m &= ~((l >> 1) & 0x550u);   // shared face: y and z edges at dx = 0
-            m &= ~((b >> 3) & 0x010u);   // one y edge each
-            m &= ~((a << 1) & 0x040u);
-            row(x - 1, y - 1, b, l, a);
-            m &= ~((l >> 3) & 0x100u);   // one z edge
-            row(x - 1, y + 1, b, l, a);
-            m &= ~((l << 1) & 0x400u);
-            row(x, y - 1, b, l, a);
-            m &= ~((l >> 1) & 0x005u);   // shared face: x edges at dy = 0
-            m &= ~((l >> 2) & 0x300u);   // and z edges
-            m &= ~((b >> 3) & 0x001u);   // one x edge each
-            m &= ~((a << 1) & 0x004u);
-            row(x, y, b, l, a);
-            m &= ~((b >> 2) & 0x033u);   // shared face: x and y edges at dz = 0
-#pragma unroll
-            for (int s = 0; s < 4; ++s) t.edge[s] = (uint32_t)__popc(m & stream_mask(s));
+            // the earlier cells that share edges, in their order
+            uint32_t r = lattice_row(L, x - 1, y - 1);
+            Place p = place_of(L, r, z);
+            if (p.here) claim(p.at, 3, 0x100u);   // one z edge
+            r = lattice_row(L, x - 1, y);
+            p = place_of(L, r, z - 1);
+            const bool top = (L.bits[r * (uint32_t)L.zw + ((z + 1) >> 5)] >> ((z + 1) & 31u)) & 1u;
+            if (p.here) claim(p.at, 3, 0x010u);   // one y edge
+            if (p.next) claim(p.at + p.here, 1, 0x550u);  // a face: y and z edges at dx = 0
+            if (top) claim(p.at + p.here + p.next, -1, 0x040u);
+            p = place_of(L, lattice_row(L, x - 1, y + 1), z);
+            if (p.here) claim(p.at, -1, 0x400u);
+            r = lattice_row(L, x, y - 1);
+            p = place_of(L, r, z - 1);
+            const bool top2 = (L.bits[r * (uint32_t)L.zw + ((z + 1) >> 5)] >> ((z + 1) & 31u)) & 1u;
+            if (p.here) claim(p.at, 3, 0x001u);   // one x edge
+            if (p.next) {                         // a face: x and z edges at dy = 0
+                claim(p.at + p.here, 1, 0x005u);
+                claim(p.at + p.here, 2, 0x300u);
+            }
+            if (top2) claim(p.at + p.here + p.next, -1, 0x004u);
+            p = place_of(L, lattice_row(L, x, y), z - 1);
+            if (p.here) claim(p.at, 2, 0x033u);   // a face: x and y edges at dz = 0
+            for (uint32_t t = m; t; t &= t - 1) {
+                const uint32_t k = slot + bits_below(mask, __ffs(t) - 1);
+                ref[k] = k;
+            }
         }
         own[i] = (uint16_t)m;
     }
-    counts[i] = t;
+    uint64_t sum = 0;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) sum |= (uint64_t)__popc(m & stream_mask(s)) << (16 * s);
+    const uint64_t mine = sum;
+    const int lane = (int)(threadIdx.x & 63);
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint64_t u = __shfl_up((unsigned long long)sum, o);
+        if (lane >= o) sum += u;
+    }
+    if (lane == 63) wave_sum[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) sum += wave_sum[w];
+    if (i <= n) local[i] = sum - mine;
+    if (threadIdx.x == kBlock - 1)
+        block[blockIdx.x] = make_uint4((uint32_t)(sum & 0xffffu), (uint32_t)((sum >> 16) & 0xffffu),
+                                       (uint32_t)((sum >> 32) & 0xffffu), (uint32_t)(sum >> 48));
+}
+
+// base[b]: the sums of the blocks before b, b = 0 .. nb, by one workgroup: a run of blocks
+// per thread.
+constexpr int kBaseBlock = 1024;
+__global__ __launch_bounds__(kBaseBlock) void smc_own_base(const uint4* __restrict__ block, int64_t nb,
+                                                           uint4* __restrict__ base) {
+    __shared__ uint32_t wave_sum[4][kBaseBlock / 64];
+    const int64_t run = (nb + kBaseBlock - 1) / kBaseBlock;
+    const int64_t b0 = min((int64_t)threadIdx.x * run, nb), b1 = min(b0 + run, nb);
+    uint32_t t[4] = {0u, 0u, 0u, 0u};
+    for (int64_t b = b0; b < b1; ++b) {
+        const uint4 v = block[b];
+        t[0] += v.x;
+        t[1] += v.y;
+        t[2] += v.z;
+        t[3] += v.w;
+    }
+    const int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
+    uint32_t at[4];
+    for (int k = 0; k < 4; ++k) {
+        uint32_t sum = t[k];
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t u = __shfl_up(sum, o);
+            if (lane >= o) sum += u;
+        }
+        if (lane == 63) wave_sum[k][w] = sum;
+        at[k] = sum - t[k];
+    }
+    __syncthreads();
+    for (int k = 0; k < 4; ++k)
+        for (int j = 0; j < w; ++j) at[k] += wave_sum[k][j];
+    for (int64_t b = b0; b < b1; ++b) {
+        const uint4 v = block[b];
+        base[b] = make_uint4(at[0], at[1], at[2], at[3]);
+        at[0] += v.x;
+        at[1] += v.y;
+        at[2] += v.z;
+        at[3] += v.w;
+    }
+    if (threadIdx.x == kBaseBlock - 1) base[nb] = make_uint4(at[0], at[1], at[2], at[3]);
 }
 
 // Number of the vertex of the edge along `axis` from lattice point (x, y, z).
 __device__ __forceinline__ uint32_t vertex_number(const Lattice& L, const uint16_t* __restrict__ own,
-                                                  const CellSums* __restrict__ sums, int64_t x, int64_t y, int64_t z,
-                                                  int axis) {
+                                                  const OwnSums& sums, int64_t x, int64_t y, int64_t z, int axis) {
     const uint32_t lower = (1u << (4 * axis)) - 1u;  // the axes before
     uint32_t id = 0;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
         const Place p = place_of(L, lattice_row(L, x - (s & 1), y - (s >> 1)), lattice_z(L, z - 1));
-        id += sums[p.at].edge[s];
+        id += own_before(sums, p.at, s);
         if (p.here) id += (uint32_t)__popc(own[p.at] & stream_mask(s) & (kLowZ | (kHighZ & lower)));
         if (p.next) id += (uint32_t)__popc(own[p.at + p.here] & stream_mask(s) & kLowZ & lower);
     }
     return id;
 }
 
-// A thread per cell: its edges' vertex numbers, the vertices it owns, its triangles.
-__global__ __launch_bounds__(kBlock) void smc_dense_write(const int32_t* __restrict__ coords,
-                                                          const float* __restrict__ corners,
-                                                          const uint8_t* __restrict__ cases,
-                                                          const uint64_t* __restrict__ offsets, int64_t n, Lattice L,
-                                                          const uint16_t* __restrict__ own,
-                                                          const CellSums* __restrict__ sums, float iso,
-                                                          float* __restrict__ verts, int32_t* __restrict__ tris) {
-    __shared__ int32_t id[12][kBlock];
+// A thread per cell: the vertices of the edges it owns, and their numbers at their slots.
+__global__ __launch_bounds__(kBlock) void smc_own_vertices(const int32_t* __restrict__ coords,
+                                                           const float* __restrict__ corners,
+                                                           const uint8_t* __restrict__ cases,
+                                                           const uint64_t* __restrict__ offsets, int64_t n, Lattice L,
+                                                           const uint16_t* __restrict__ own, OwnSums sums, float iso,
+                                                           float* __restrict__ verts, int32_t* __restrict__ map) {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    const uint32_t c = cases[i], mine = own[i];
+    const uint32_t mine = own[i];
+    if (!mine) return;
+    uint32_t mask = 0;
+    const uint32_t c = cases[i], slot = (uint32_t)(offsets[i] >> 32);
+#pragma unroll
+    for (int e = 0; e < 12; ++e) mask |= (((c >> mc::edge_a(e)) ^ (c >> mc::edge_b(e))) & 1u) << edge_bit(e);
     const int64_t x = coords[3 * i], y = coords[3 * i + 1], z = coords[3 * i + 2];
-    for (uint32_t m = edge_mask_of(c); m; m &= m - 1) {
-        const int e = __ffs(m) - 1, a = mc::edge_a(e), b = mc::edge_b(e);
-        const uint32_t v = vertex_number(L, own, sums, x + min(mc::corner_dx(a), mc::corner_dx(b)),
-                                         y + min(mc::corner_dy(a), mc::corner_dy(b)),
-                                         z + min(mc::corner_dz(a), mc::corner_dz(b)), mc::edge_axis(e));
-        id[e][threadIdx.x] = (int32_t)v;
-        if ((mine >> edge_bit(e)) & 1u) store_vertex(coords, corners, i, e, iso, verts + 3 * (int64_t)v);
+    for (uint32_t m = mine; m; m &= m - 1) {
+        const int k = __ffs(m) - 1, axis = k >> 2, u = k & 1, v = (k >> 1) & 1;
+        const uint32_t id = vertex_number(L, own, sums, x + (axis == 0 ? 0 : u), y + (axis == 0 ? u : axis == 2 ? v : 0),
+                                          z + (axis == 2 ? 0 : v), axis);
+        map[slot + bits_below(mask, k)] = (int32_t)id;
+        store_vertex(coords, corners, i, nibble(kEdgeOfBit, k), iso, verts + 3 * (int64_t)id);
     }
+}
+
+__global__ __launch_bounds__(kBlock) void smc_own_triangles(const uint8_t* __restrict__ cases,
+                                                            const uint64_t* __restrict__ offsets, int64_t n,
+                                                            const uint32_t* __restrict__ ref,
+                                                            const int32_t* __restrict__ map, int32_t* __restrict__ tris) {
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t c = cases[i];
     const uint64_t packed = c_triangles[c];
     const int nt = mc::triangle_count(packed);
-    int32_t* o = tris + 3 * (int64_t)(uint32_t)offsets[i];
+    if (!nt) return;
+    uint32_t mask = 0;
+#pragma unroll
+    for (int e = 0; e < 12; ++e) mask |= (((c >> mc::edge_a(e)) ^ (c >> mc::edge_b(e))) & 1u) << edge_bit(e);
+    const uint64_t off = offsets[i];
+    const uint32_t* r = ref + (uint32_t)(off >> 32);
+    auto vertex = [&](int j) { return map[r[bits_below(mask, nibble(kBitOfEdge, mc::triangle_edge(packed, j)))]]; };
+    int32_t* o = tris + 3 * (int64_t)(uint32_t)off;
     for (int t = 0; t < nt; ++t) {
-        o[3 * t] = id[mc::triangle_edge(packed, 3 * t)][threadIdx.x];
-        o[3 * t + 1] = id[mc::triangle_edge(packed, 3 * t + 2)][threadIdx.x];
-        o[3 * t + 2] = id[mc::triangle_edge(packed, 3 * t + 1)][threadIdx.x];
+        o[3 * t] = vertex(3 * t);
+        o[3 * t + 1] = vertex(3 * t + 2);
+        o[3 * t + 2] = vertex(3 * t + 1);
     }
 }
 
@@ -590,9 +694,10 @@ struct SmcState {
     bool dense = false;
     Lattice lattice = {};
     uint16_t* own = nullptr;   // edge bits owned
-    CellSums* counts = nullptr;
-    CellSums* sums = nullptr;  // exclusive, n + 1 of them
-    char* sums_tmp = nullptr;
+    uint32_t* ref = nullptr;   // raw slot -> the owner's raw slot
+    uint64_t* local = nullptr;
+    uint4* block = nullptr;
+    uint4* base = nullptr;
 };
 
 namespace {
@@ -717,27 +822,25 @@ size_t word_scan_bytes(int64_t words) {
     return b;
 }
 
-size_t sums_scan_bytes(int64_t m) {
-    size_t b = 0;
-    hipcub::DeviceScan::ExclusiveScan(nullptr, b, (const CellSums*)nullptr, (CellSums*)nullptr, AddSums(), CellSums{{0, 0, 0, 0}},
-                                      (int)m);
-    return b;
-}
-
-// Region B of ascending cells, and their lattice's bits and prefix counts.
+// Region B of ascending cells (with the arrays per edge where m_raw is known), and their
+// lattice's bits and prefix counts.
 hipError_t dense_lattice(SmcState* st, int64_t words, hipStream_t s) {
-    const int64_t n = st->n;
-    const size_t wbytes = word_scan_bytes(words), sbytes = sums_scan_bytes(n + 1);
+    const int64_t n = st->n, nb = n / kBlock + 1;
+    const size_t wbytes = word_scan_bytes(words);
     uint32_t *bits, *before;
     char* tmp;
     auto lay = [&](Carve& c) {
         bits = c.take<uint32_t>(words);
         before = c.take<uint32_t>(words);
         st->own = c.take<uint16_t>(n);
-        st->counts = c.take<CellSums>(n + 1);
-        st->sums = c.take<CellSums>(n + 1);
+        st->local = c.take<uint64_t>(n + 1);
+        st->block = c.take<uint4>(nb);
+        st->base = c.take<uint4>(nb + 1);
         tmp = c.take<char>((int64_t)wbytes);
-        st->sums_tmp = c.take<char>((int64_t)sbytes);
+        if (st->m_raw > 0) {
+            st->ref = c.take<uint32_t>(st->m_raw);
+            st->map = c.take<int32_t>(st->m_raw);
+        }
     };
     Carve size;
     lay(size);
@@ -756,12 +859,11 @@ hipError_t dense_lattice(SmcState* st, int64_t words, hipStream_t s) {
 
 // The owned edges of ascending cells (classified) and their sums.
 hipError_t dense_edges(SmcState* st, hipStream_t s) {
-    const int64_t n = st->n;
-    hipLaunchKernelGGL(smc_own_edges, dim3(blocks_for(n + 1)), dim3(kBlock), 0, s, st->coords, st->cases, n, st->lattice,
-                       st->own, st->counts);
-    size_t bytes = sums_scan_bytes(n + 1);
-    return hipcub::DeviceScan::ExclusiveScan(st->sums_tmp, bytes, st->counts, st->sums, AddSums(), CellSums{{0, 0, 0, 0}},
-                                             (int)(n + 1), s);
+    const int64_t n = st->n, nb = n / kBlock + 1;
+    hipLaunchKernelGGL(smc_own_edges, dim3((unsigned)nb), dim3(kBlock), 0, s, st->coords, st->cases, st->offsets, n,
+                       st->lattice, st->own, st->ref, st->local, st->block);
+    hipLaunchKernelGGL(smc_own_base, dim3(1), dim3(kBaseBlock), 0, s, st->block, nb, st->base);
+    return hipGetLastError();
 }
 
 // Copies `bytes` from the device once the stream's work is done (through pinned memory
@@ -896,6 +998,9 @@ SmcStatus smc_extract(const int32_t* coords, const float* corners, int64_t n, fl
         e = try_dense();
         if (e != hipSuccess) return bail(hip_status(e, "cell lattice"));
         if (st->dense) {
+            // the corner sort's room holds the arrays per edge
+            st->ref = corner_area.take<uint32_t>(12 * n);
+            st->map = corner_area.take<int32_t>(12 * n);
             hipLaunchKernelGGL(smc_dense_mean, dim3(blocks_for(8 * n)), dim3(kBlock), 0, s, coords, n, st->lattice, corners,
                                mean);
             e = hipGetLastError();
@@ -937,10 +1042,10 @@ SmcStatus smc_extract(const int32_t* coords, const float* corners, int64_t n, fl
     if (st->dense) {
         e = dense_edges(st, s);
         if (e != hipSuccess) return bail(hip_status(e, "edge numbering"));
-        CellSums all;
-        e = read_back(st, st->sums + n, sizeof all, &all, s);
+        uint4 all;
+        e = read_back(st, st->base + (n / kBlock + 1), sizeof all, &all, s);
         if (e != hipSuccess) return bail(hip_status(e, "vertex count"));
-        for (int k = 0; k < 4; ++k) st->m += all.edge[k];
+        st->m = (int64_t)all.x + all.y + all.z + all.w;
         *out = st;
         *n_verts = st->m;
         *n_tris = st->t;
@@ -965,8 +1070,11 @@ SmcStatus smc_write(SmcState* st, float* verts, int32_t* tris, hipStream_t s) {
     SmcStatus r;
     if (st->dense) {
         if (st->m > 0)
-            hipLaunchKernelGGL(smc_dense_write, dim3(blocks_for(st->n)), dim3(kBlock), 0, s, st->coords, st->corners, st->cases,
-                               st->offsets, st->n, st->lattice, st->own, st->sums, st->iso, verts, tris);
+            hipLaunchKernelGGL(smc_own_vertices, dim3(blocks_for(st->n)), dim3(kBlock), 0, s, st->coords, st->corners, st->cases,
+                               st->offsets, st->n, st->lattice, st->own, OwnSums{st->base, st->local}, st->iso, verts, st->map);
+        if (st->t > 0)
+            hipLaunchKernelGGL(smc_own_triangles, dim3(blocks_for(st->n)), dim3(kBlock), 0, s, st->cases, st->offsets, st->n,
+                               st->ref, st->map, tris);
         r = hip_status(hipGetLastError(), "marching cubes kernel launch");
     } else if (st->m_raw > 0) {
         if (st->wide)
