@@ -811,7 +811,7 @@ void launch_vertices(const SmcState* st, float* verts, hipStream_t s) {
 
 // Words of the bounding lattice's bits up to which ascending cells go without the sort (a
 // word costs some 12 bytes of traffic, the sort's passes over a cell's edges about 300).
-int64_t dense_words_most(int64_t n) { return 8 * n + (1 << 14); }
+int64_t dense_words_most(int64_t n) { return std::min<int64_t>(8 * n + (1 << 14), INT32_MAX); }
 
 using WordIter = hipcub::TransformInputIterator<uint32_t, WordCells, hipcub::CountingInputIterator<int64_t>>;
 
