@@ -546,9 +546,9 @@ def run_extras(dev, steps, warmup, out, gpu_build=True):
     _, t = _time_kernel(lambda: cubvh_amd.floodfill(occ), steps, 1)
     out["floodfill_256"] = {"ms": t * 1e3, "Mvoxels_s": occ.numel() / t / 1e6,
                             "GB_s_5B_per_voxel": 5 * occ.numel() / t / 1e9,
-                            "roofline": dict(roofline_block("floodfill_grid256", "ff_tiles + 3 ff_merge_axis + ff_flatten",
+                            "roofline": dict(roofline_block("floodfill_grid256", "ff_tiles + ff_merge + ff_flatten",
                                                             t, units=occ.numel(), algo_bytes_per_unit=5),
-                                             time_basis="whole call (5 kernel launches)")}
+                                             time_basis="whole call (3 kernel launches)")}
     del G, d, occ
 
     # soup: camera rays (16 x 1920 x 1080) and raystab on 2^22 points
