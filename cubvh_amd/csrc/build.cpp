@@ -500,7 +500,15 @@ void compute_face_bounds(HostBvh& bvh) {
         face_vertices(bvh, s, v);
         face_normal(v, n);
         for (int k = 0; k < 3; ++k) c[k] = (v[0][k] + v[1][k] + v[2][k]) / 3.0;
-        store_disk(v, 3, c, n, &bvh.tbnd[8 * s]);
+        float* disk = &bvh.tbnd[8 * s];
+        store_disk(v, 3, c, n, disk);
+        double ab2 = 0.0, ac2 = 0.0, n2 = 0.0;
+        for (int k = 0; k < 3; ++k) {
+            ab2 += (v[1][k] - v[0][k]) * (v[1][k] - v[0][k]);
+            ac2 += (v[2][k] - v[0][k]) * (v[2][k] - v[0][k]);
+            n2 += n[k] * n[k];
+        }
+        if (!line_test_applies(ab2, ac2, n2)) disk[7] = -disk[7];
     }
     // leaves: centre of the vertex box and the area-weighted mean normal
     for (const WideNode& w : bvh.nodes) {

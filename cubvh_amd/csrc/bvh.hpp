@@ -13,8 +13,10 @@
 //   tbnd  : float4[2 * n_faces] in leaf order, a bounding disk per face:
 //           tbnd[2t+0] = (centre, radius), tbnd[2t+1] = (unit normal, thickness).
 //           Every point of the face lies within `radius` of the centre in the plane
-//           through the centre with that normal, and within `thickness` of that plane.
-//           It gives a cheap lower bound on the squared distance to the face.
+//           through the centre with that normal, and within |thickness| of that plane.
+//           It gives a cheap lower bound on the squared distance to the face.  The
+//           thickness is negative for a face that the rays' line test must not reject
+//           (line_test_applies below).
 //   lbnd  : float4[2 * n_faces], the same kind of disk around all faces of a leaf,
 //           stored at the leaf's first slot: lbnd[2f+0..1] for the leaf starting at
 //           triangle f (other slots unused).  One test can skip a whole leaf.
@@ -52,6 +54,15 @@ constexpr int32_t make_leaf_ref(int64_t first, int count) {
 }
 constexpr int32_t leaf_ref_first(int32_t ref) { return (int32_t)(((uint32_t)ref & 0x7fffffffu) >> LEAF_COUNT_BITS); }
 constexpr int32_t leaf_ref_count(int32_t ref) { return (ref & (MAX_LEAF_SIZE - 1)) + 1; }
+
+// Whether tri_ray's rounding on a face is small enough for the rays' test against the
+// face's bounding sphere (ray_line.hpp): from the squared lengths of b - a, c - a and their
+// cross product, the sine of the angle between them is at least 1/16, and the product of the
+// lengths neither under- nor overflows in the intersector.  False with NaN anywhere.
+constexpr bool line_test_applies(double ab2, double ac2, double n2) {
+    const double p = ab2 * ac2;
+    return p >= 1e-48 && p <= 1e36 && n2 >= p * (1.0 / 256.0);
+}
 
 struct alignas(16) WideNode {
     float lo_x[4], hi_x[4];

@@ -1227,6 +1227,15 @@ __global__ __launch_bounds__(256) void face_records(int64_t n, const float4* __r
     const double2 ext = face_extent(fr, tris, s);
     store_disk(fr, ext.x, ext.y, tbnd + 2 * s);
     const float4 r0 = tris[3 * s], r1 = tris[3 * s + 1], r2 = tris[3 * s + 2];
+    const double ab[3] = {(double)r1.x - r0.x, (double)r1.y - r0.y, (double)r1.z - r0.z};
+    const double ac[3] = {(double)r2.x - r0.x, (double)r2.y - r0.y, (double)r2.z - r0.z};
+    double ab2 = 0.0, ac2 = 0.0, n2 = 0.0;
+    for (int k = 0; k < 3; ++k) {
+        ab2 += ab[k] * ab[k];
+        ac2 += ac[k] * ac[k];
+        n2 += acc.n[k] * acc.n[k];
+    }
+    if (!line_test_applies(ab2, ac2, n2)) tbnd[2 * s + 1].w = -tbnd[2 * s + 1].w;
     const V3 a{r0.x, r0.y, r0.z}, b{r1.x, r1.y, r1.z}, c{r2.x, r2.y, r2.z};
     const V3 v21 = vsub(b, a), v32 = vsub(c, b), v13 = vsub(a, c);
     const V3 nn = vcross(v21, v13);

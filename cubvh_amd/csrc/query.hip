@@ -25,6 +25,7 @@
 #include "bvh.hpp"
 #include "geom.hpp"
 #include "query.hpp"
+#include "ray_line.hpp"
 
 namespace cubvh_amd {
 namespace dev {
@@ -59,7 +60,7 @@ __device__ __forceinline__ float disk_bound(f3 p, float4 cb, float4 nb) {
     f3 d = mk3(p.x - cb.x, p.y - cb.y, p.z - cb.z);
     float dd = dot3(d, d);
     float h = dot3(mk3(nb.x, nb.y, nb.z), d);
-    float ah = fmaxf(fabsf(h) - nb.w, 0.0f);
+    float ah = fmaxf(fabsf(h) - fabsf(nb.w), 0.0f);  // a face's thickness may be negative (bvh.hpp)
     float rho = __builtin_amdgcn_sqrtf(fmaxf(dd - h * h, 0.0f));
     float t = fmaxf(rho - cb.w, 0.0f);
     float lb = ah * ah + t * t;
@@ -874,34 +875,6 @@ __device__ __forceinline__ void run_exact_ray(const Tree& T, ExactQueue& q, int3
     }
     qn = base;
     wave_fence();
-}
-
-// A ray as its line's test against bounding spheres takes it: unit direction, and the
-// margin that a sphere's radius needs for the fp32 rounding of tri_ray.
-struct RayLine {
-    f3 o, dn;
-    float margin;
-};
-
-// reach: no vertex is farther from o.  tri_ray's u, v place the hit with an error of at
-// most |error of cross(o - a, d)| / cos, cos the angle's between ray and face normal: 3.6e-7
-// reach / cos by the roundings of that product, 2^-16 reach at cos = 1/20.  Directions
-// whose length under- or overflows when squared get no test (an infinite margin).
-__device__ __forceinline__ RayLine ray_line(f3 o, f3 d, float reach) {
-    const float n2 = dot3(d, d), s = 1.0f / sqrtf(n2);
-    RayLine r;
-    r.o = o;
-    r.dn = mk3(d.x * s, d.y * s, d.z * s);
-    r.margin = n2 > 1e-12f && n2 < 1e12f ? reach * 1.52587890625e-05f : INFINITY;
-    return r;
-}
-
-// True when the line passes the sphere around a face's disk so far out that tri_ray gives
-// a miss; never for a face seen at less than 3 degrees, nor with NaN anywhere.
-__device__ __forceinline__ bool line_rejects(const RayLine& r, float4 cb, float4 nb) {
-    const f3 x = cross3(mk3(cb.x - r.o.x, cb.y - r.o.y, cb.z - r.o.z), r.dn);
-    const float reach = (cb.w + nb.w) * 1.015625f + r.margin;
-    return dot3(x, x) > reach * reach && fabsf(dot3(mk3(nb.x, nb.y, nb.z), r.dn)) > 0.05f;
 }
 
 // Packet form of closest_hit: every lane traces its own ray; node and face records
