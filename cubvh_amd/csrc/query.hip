@@ -418,17 +418,85 @@ __device__ int any_hit_line(const Tree& T, f3 o, f3 d, LaneStack<BLOCK, LDS_N>& 
     }
 }
 
-// Mean unit normal of every face within squared distance NORMAL_EPS of point c
-// (src/bvh.cu:356-396).  The sum is accumulated in double so that it does not
-// depend on the visiting order, then rounded to float and divided by the count.
-template <int BLOCK, int LDS_N>
-__device__ f3 avg_normal(const Tree& T, f3 c, LaneStack<BLOCK, LDS_N>& st) {
-    double sx = 0.0, sy = 0.0, sz = 0.0;
-    float cnt = 0.0f;
+// Sum of face normals that does not depend on the order they are added in, so that a query
+// gets the same sign from a lane, a wave and any tree.  The first walk adds in double, which
+// is exact when every component is 0 or at least 2^-28 times the count (components of 24
+// bits: the sum spans at most 53).  Otherwise (1 + 1e-20 - 1, as on back-to-back sheets
+// built with sines and cosines) further walks add one part of every component each: the
+// multiples of 2^-27, then of 2^-54 and so on, the sixth part the rest (multiples of
+// 2^-149).  A part holds at most 2^27 units of a component of magnitude 1, so 2^25 of them
+// add up without rounding; the parts' sums wait in `keep` (18 doubles) and are added up as a
+// value and its rounding error.
+struct NormalSum {
+    double x = 0.0, y = 0.0, z = 0.0;
+    float n = 0.0f;
+    uint32_t least = 0xffffffffu;  // bits of the smallest component but 0, less 1
+
+    __device__ __forceinline__ void add(f3 v) {
+        least = min(least, min((__float_as_uint(v.x) & 0x7fffffffu) - 1u,
+                               min((__float_as_uint(v.y) & 0x7fffffffu) - 1u, (__float_as_uint(v.z) & 0x7fffffffu) - 1u)));
+        x += (double)v.x;
+        y += (double)v.y;
+        z += (double)v.z;
+        n += 1.0f;
+    }
+    __device__ __forceinline__ bool exact() const { return least >= __float_as_uint(n * 0x1p-28f); }
+    __device__ __forceinline__ f3 mean() const { return mk3((float)x / n, (float)y / n, (float)z / n); }
+};
+struct NormalParts {
+    double* keep;
+    double x, y, z;
+    int part = 0;
+    bool more;  // components hold lower parts
+
+    __device__ __forceinline__ void start() {
+        x = y = z = 0.0;
+        more = false;
+    }
+    __device__ __forceinline__ double part_of(float v) {
+        double r = (double)v, big = 0x1.8p25, h = 0.0;  // 1.5 * 2^52 units of 2^-27
+        for (int j = 0; j <= part; ++j) {
+            h = j < 5 ? (r + big) - big : r;
+            r -= h;
+            big *= 0x1p-27;
+        }
+        more = more || r != 0.0;
+        return h;
+    }
+    __device__ __forceinline__ void add(f3 v) {
+        x += part_of(v.x);
+        y += part_of(v.y);
+        z += part_of(v.z);
+    }
+    // After a walk: whether another one is needed.
+    __device__ __forceinline__ bool next() {
+        keep[3 * part] = x;
+        keep[3 * part + 1] = y;
+        keep[3 * part + 2] = z;
+        return ++part < 6 && more;
+    }
+    __device__ __forceinline__ f3 mean(float n) const {
+        double v[3];
+        for (int k = 0; k < 3; ++k) {
+            double h = 0.0, e = 0.0;
+            for (int j = 0; j < part; ++j) {
+                const double s = keep[3 * j + k], t = h + s, w = t - h;
+                e += (h - (t - w)) + (s - w);
+                h = t;
+            }
+            v[k] = h + e;
+        }
+        return mk3((float)v[0] / n, (float)v[1] / n, (float)v[2] / n);
+    }
+};
+
+// Adds the unit normal of every face within squared distance NORMAL_EPS of point c.
+template <int BLOCK, int LDS_N, class Sum>
+__device__ __forceinline__ void add_normals(const Tree& T, f3 c, LaneStack<BLOCK, LDS_N>& st, Sum& sum) {
+    if (has_nan(c)) return;  // no face is within NORMAL_EPS of it
     int32_t ref = 0;
     st.sp = 0;
     for (;;) {
-        if (has_nan(c)) break;  // no face is within NORMAL_EPS of it: the mean is 0 / 0
         if (ref >= 0) {
             WideNode nd = load_node(T.nodes, ref);
             float k[4];
@@ -446,20 +514,29 @@ __device__ f3 avg_normal(const Tree& T, f3 c, LaneStack<BLOCK, LDS_N>& st) {
                 f3 a, b, cc;
                 int32_t id;
                 load_tri(T.tris, first + j, a, b, cc, id);
-                if (tri_dist2(a, b, cc, c) < NORMAL_EPS) {
-                    f3 n = tri_normal(a, b, cc);
-                    sx += (double)n.x;
-                    sy += (double)n.y;
-                    sz += (double)n.z;
-                    cnt += 1.0f;
-                }
+                if (tri_dist2(a, b, cc, c) < NORMAL_EPS) sum.add(tri_normal(a, b, cc));
             }
         }
         if (st.sp == 0) break;
         --st.sp;
         ref = st.ref_at(st.sp);
     }
-    return mk3((float)sx / cnt, (float)sy / cnt, (float)sz / cnt);
+}
+
+// Mean unit normal of every face within squared distance NORMAL_EPS of point c
+// (src/bvh.cu:356-396): the sum rounded to float and divided by the count (0 / 0 for none).
+template <int BLOCK, int LDS_N>
+__device__ f3 avg_normal(const Tree& T, f3 c, LaneStack<BLOCK, LDS_N>& st) {
+    NormalSum sum;
+    add_normals(T, c, st, sum);
+    if (sum.exact()) return sum.mean();
+    double keep[18];
+    NormalParts parts{keep};
+    do {
+        parts.start();
+        add_normals(T, c, st, parts);
+    } while (parts.next());
+    return parts.mean(sum.n);
 }
 
 // ---------------------------------------------------------------------------

@@ -38,7 +38,7 @@ constexpr int kWaveNodes = 16;   // nodes of a round
 constexpr int kWaveDive = 4;     // the same until a first face is known
 constexpr int kWaveLeaves = 4;   // leaves of a face round (16 lanes each)
 static_assert(MAX_LEAF_SIZE == 16, "a face round gives a leaf 16 lanes");
-struct WaveLists {
+struct alignas(8) WaveLists {
     int32_t ref[kWaveStack];
     float key[kWaveStack];
     int32_t leaf[64];
@@ -269,11 +269,10 @@ __device__ void closest_face_wave(const Tree& T, int32_t root, f3 p, WaveLists& 
     best_d2 = __uint_as_float(best);
 }
 
-// avg_normal over one wave (c wave-uniform; the sum in double does not depend on the order).
-__device__ f3 avg_normal_wave(const Tree& T, f3 c, WaveLists& L) {
+// add_normals over one wave (c and sum wave-uniform).
+template <class Sum>
+__device__ __forceinline__ void add_normals_wave(const Tree& T, f3 c, WaveLists& L, Sum& sum) {
     const int lane = (int)(threadIdx.x & 63);
-    double sx = 0.0, sy = 0.0, sz = 0.0;
-    float cnt = 0.0f;
     WaveWork w{L};
     w.start(0);
     if (has_nan(c)) w.sp = 0;
@@ -307,16 +306,27 @@ __device__ f3 avg_normal_wave(const Tree& T, f3 c, WaveLists& L) {
             }
             for (uint64_t m = ballot(on); m != 0; m &= m - 1) {
                 const int l = (int)__builtin_ctzll(m);
-                sx += (double)lane_value(n.x, l);
-                sy += (double)lane_value(n.y, l);
-                sz += (double)lane_value(n.z, l);
-                cnt += 1.0f;
+                sum.add(mk3(lane_value(n.x, l), lane_value(n.y, l), lane_value(n.z, l)));
             }
         } else {
             break;
         }
     }
-    return mk3((float)sx / cnt, (float)sy / cnt, (float)sz / cnt);
+}
+
+// avg_normal over one wave (c wave-uniform).
+__device__ f3 avg_normal_wave(const Tree& T, f3 c, WaveLists& L) {
+    NormalSum sum;
+    add_normals_wave(T, c, L, sum);
+    if (sum.exact()) return sum.mean();
+    NormalParts parts{reinterpret_cast<double*>(L.face)};  // no faces wait here
+    do {
+        parts.start();
+        add_normals_wave(T, c, L, parts);
+        wave_fence();
+    } while (parts.next());
+    wave_fence();
+    return parts.mean(sum.n);
 }
 
 // Closest hit of the ray (wave-uniform arguments and results), as closest_hit; best / bslot

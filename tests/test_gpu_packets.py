@@ -1,5 +1,7 @@
 """Packet walks (64 queries or rays a wave) where they can go wrong, held to the wave walks
 and to the oracle."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -38,3 +40,30 @@ def test_thin_faces_ray_packets_equal_waves(gpu, check, builder, aspect):  # noq
     large = bvh.ray_trace(o.repeat_interleave(COPIES, 0), d.repeat_interleave(COPIES, 0))
     same_bits([x[::COPIES] for x in large], small)
     assert (small[1] >= 0).any()
+
+
+@pytest.mark.parametrize("builder", ["host", "gpu", "gpu_lbvh"])
+@pytest.mark.parametrize("n_faces", [12, 90, 700])
+def test_watertight_sign_is_the_exact_normal_sums(gpu, n_faces, builder):
+    """Sheets back to back whose normals cancel, with small ones left over: the sign is the
+    exact sum's, whatever the order of the faces, by waves and by packets."""
+    rng = np.random.default_rng(n_faces)
+    up = np.array([[0, 0, 0], [1, 0, 0], [0, 1, 0]], np.float32)
+    small = [1e-9, 1e-12, 3e-17, 1e-20, 1e-25, 2.5e-30, 1e-36]
+    for trial in range(24):
+        pairs = n_faces // 3
+        # normals (-1, 0, -x) of faces that go down from the edge shared by all
+        left = rng.choice(small[trial % 4:], n_faces - 2 * pairs) * rng.choice([-1.0, 1.0], n_faces - 2 * pairs)
+        left[1::2] = -left[:-1:2][: len(left[1::2])]  # in turn cancelled, but for the last
+        left = np.append(left[:-1], rng.choice(small[3:]) * rng.choice([-1.0, 1.0])).astype(np.float32)
+        faces = [up, up[[0, 2, 1]]] * pairs + [np.array([[0, 0, 0], [0, 1, 0], [x, 0, -1]], np.float32) for x in left]
+        faces = np.stack([faces[i] for i in rng.permutation(n_faces)])
+        inside = -math.fsum(left.tolist()) < 0.0
+        bvh = cubvh_amd.cuBVH(faces.reshape(-1, 3), np.arange(3 * n_faces, dtype=np.int32).reshape(-1, 3), build=builder)
+        p = torch.zeros(100, 3, device=gpu)
+        p[:, 1] = torch.linspace(0.1, 0.9, 100, device=gpu)
+        p[:, 2] = torch.linspace(0.01, 0.5, 100, device=gpu)
+        waves = bvh.signed_distance(p)
+        packets = bvh.distance_ordered(p, torch.arange(100, dtype=torch.int32, device=gpu), signed=True)
+        same_bits(waves[:2], packets[:2])
+        assert bool((torch.signbit(waves[0]) == inside).all())
