@@ -877,22 +877,8 @@ int cubvh_distance_ordered(cubvh_bvh* bvh, int device, int64_t n, int32_t kind, 
     q.out_id = face_id;
     q.out_v = uvw;
     q.packet = true;
-    // a captured call allocates nothing: its walks all run to their end
-    hipStream_t hs = (hipStream_t)stream;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    hipError_t e = hipStreamIsCapturing(hs, &cs);
-    if (e != hipSuccess) return fail_hip(e, "hipStreamIsCapturing");
-    if (cs == hipStreamCaptureStatusNone && n < kRestLast) {
-        rc = ensure_pool(device);
-        if (rc != CUBVH_OK) return rc;
-        e = hipMallocAsync(&q.rest, rest_bytes(n), hs);
-        if (e != hipSuccess) return fail_hip(e, "hipMallocAsync(rest of the walks)");
-    }
-    e = launch_distance(q, kind);
-    if (q.rest) {
-        const hipError_t e2 = hipFreeAsync(q.rest, hs);
-        if (e == hipSuccess) e = e2;
-    }
+    // allocates nothing, so its walks all run to their end (q.rest is null)
+    hipError_t e = launch_distance(q, kind);
     if (e != hipSuccess) return fail_hip(e, "distance kernel launch");
     return CUBVH_OK;
     CUBVH_GUARD_END

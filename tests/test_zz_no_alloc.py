@@ -82,3 +82,39 @@ def test_noalloc_refuses_before_device_work(gpu):
     _lib.check(_call(lib.cubvh_unsigned_distance, bvh, P, ref))
     torch.cuda.synchronize()
     assert all(torch.equal(a, b) for a, b in zip(out, ref))
+
+
+def _pool_high(dev, call):
+    """Bytes that `call` takes from the device's stream-ordered pool at most."""
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    used_high = 0x8  # hipMemPoolAttrUsedMemHigh
+    pool, v = ctypes.c_void_p(), ctypes.c_uint64(0)
+    assert hip.hipDeviceGetDefaultMemPool(ctypes.byref(pool), dev.index) == 0
+    torch.cuda.synchronize(dev)
+    assert hip.hipMemPoolSetAttribute(pool, used_high, ctypes.byref(v)) == 0
+    call()
+    torch.cuda.synchronize(dev)
+    assert hip.hipMemPoolGetAttribute(pool, used_high, ctypes.byref(v)) == 0
+    return v.value
+
+
+def test_calls_that_promise_it_allocate_nothing(gpu):
+    """cubvh_distance_ordered and the allocation-free call take nothing from the pool; an
+    unordered call of that size does (so the count would show it)."""
+    lib = _lib.load()
+    v, f, _ = S.perturbed_sphere(6, seed=3)
+    bvh = cubvh_amd.cuBVH(v, f)
+    n = 300_001
+    P = torch.from_numpy(S.uniform_points(n, seed=1)).to(gpu)
+    order = cubvh_amd.morton_order(P)
+    out = _outputs(n, gpu)
+    s = ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)
+    for kind in (0, 1):
+        def ordered():
+            _lib.check(lib.cubvh_distance_ordered(bvh._h, gpu.index, n, kind, P.data_ptr(), order.data_ptr(),
+                                                  *[x.data_ptr() for x in out], s))
+
+        ordered()  # the tree goes to the device
+        assert _pool_high(gpu, ordered) == 0
+    assert _pool_high(gpu, lambda: _lib.check(_call(lib.cubvh_unsigned_distance_noalloc, bvh, P, out))) == 0
+    assert _pool_high(gpu, lambda: _lib.check(_call(lib.cubvh_unsigned_distance, bvh, P, out))) > 4 * n
