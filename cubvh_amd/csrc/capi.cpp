@@ -36,8 +36,6 @@ int fail_hip(hipError_t e, const char* what) {
 
 constexpr int kMaxDevices = 64;
 constexpr int kDefaultLeaf = 16;  // faces per leaf unless the caller asks otherwise
-// A captured raystab call of fewer queries walks one lane per query, without scratch.
-constexpr int64_t kMortonMin = 1 << 11;
 
 // Keeps freed stream-ordered allocations in the device's default pool instead of
 // returning them to the driver at every synchronization.
@@ -353,18 +351,12 @@ int run_distance(cubvh_bvh* bvh, int device, int64_t n, int kmode, const float* 
     q.out_id = face_id;
     q.out_v = uvw;
     hipStream_t hs = (hipStream_t)stream;
-    // Large batches are walked in Morton order, and raystab needs lists (stream-ordered
-    // scratch from the device's default memory pool, released after the launch).  A captured
-    // raystab call of few queries allocates nothing: it walks one lane per query.
+    // Large batches are walked in Morton order, and raystab from kStabFew queries on needs
+    // lists (stream-ordered scratch from the device's default memory pool, released after
+    // the launch).
     void* scratch = nullptr;
     const bool ordered = n >= kWaveMax && n < ((int64_t)1 << 31);
-    bool lists = kmode == 2 && n < ((int64_t)1 << 31);
-    if (lists && n < kMortonMin) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        hipError_t e = hipStreamIsCapturing(hs, &cs);
-        if (e != hipSuccess) return fail_hip(e, "hipStreamIsCapturing");
-        lists = cs == hipStreamCaptureStatusNone;
-    }
+    const bool lists = kmode == 2 && n >= kStabFew && n < ((int64_t)1 << 31);
     if (ordered || lists) {
         rc = ensure_pool(device);
         if (rc != CUBVH_OK) return rc;
@@ -391,6 +383,9 @@ int run_distance(cubvh_bvh* bvh, int device, int64_t n, int kmode, const float* 
         // raystab: the distances, then the stab rays
         e = launch_distance(q, 0);
         if (e == hipSuccess) e = launch_stab_sign(q, scratch);
+    } else if (kmode == 2 && n < kStabFew) {
+        e = launch_distance(q, 0);
+        if (e == hipSuccess) e = launch_stab_few(q);
     } else {
         e = launch_distance(q, kmode);
     }

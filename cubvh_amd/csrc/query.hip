@@ -1437,6 +1437,29 @@ __global__ __launch_bounds__(64) void stab_wave(uint32_t batch, uint32_t* __rest
     }
 }
 
+// Raystab signs of few queries without lists or scratch: a workgroup per query, a wave per
+// line, WAVES lines a round until one misses.  Every query's first WAVES lines are walked,
+// where the lists walk most queries' first only: worth it while the chip is not full.
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void stab_few(const float* __restrict__ positions, float* __restrict__ distances,
+                                                       Tree T) {
+    __shared__ WaveLists lists[WAVES];
+    __shared__ int missed[32 / WAVES];  // per round: a wave may be a round ahead of another
+    const uint32_t q = blockIdx.x, wave = (uint32_t)uniform((int32_t)(threadIdx.x >> 6));
+    if (threadIdx.x < 32 / WAVES) missed[threadIdx.x] = 0;
+    __syncthreads();
+    Pcg32 rng;
+    rng.advance((uint64_t)(uint32_t)(q * 2u));
+    const float ox = rng.next_float(), oy = rng.next_float();
+    const f3 p = load_pt(positions, q);
+    for (uint32_t r = 0; r < 32 / WAVES; ++r) {
+        if (any_hit_line_wave(T, p, fibonacci_dir32(r * WAVES + wave, ox, oy), lists[wave]) != 3) missed[r] = 1;
+        __syncthreads();
+        if (missed[r]) return;
+    }
+    if (threadIdx.x == 0) distances[q] = -distances[q];
+}
+
 // The unmarked entries of list_in (count_in of them) make list_out (count_out).
 __global__ __launch_bounds__(256) void stab_keep(const uint32_t* __restrict__ list_in, const uint32_t* __restrict__ count_in,
                                                  uint32_t* __restrict__ list_out, uint32_t* __restrict__ count_out) {
@@ -1684,6 +1707,7 @@ constexpr uint32_t kRestBlocks = 8192;  // one-wave workgroups of a rest launch:
 // and many.  Lanes that hand walks of more than 32 to 256 steps to waves were no better.
 constexpr int64_t kStabWaveMax = (int64_t)1 << 20;
 constexpr int64_t kStabWaveBlocks = 16384;
+constexpr int kStabFewWaves = 8;
 
 // Runs of consecutive workgroups per XCD for a grid of nb one-wave workgroups over a
 // Morton order: the largest power of two <= nb / 128, so that each XCD's L2 serves one
@@ -1849,6 +1873,14 @@ hipError_t launch_stab_sign(const QueryArgs& q, void* ws) {
     }
     hipLaunchKernelGGL(dev::stab_negate, dim3(keep_grid), dim3(256), 0, s, lists[dev::kStabBatches & 1],
                        counts + 1 + dev::kStabBatches, q.out_f);
+    return hipGetLastError();
+}
+
+hipError_t launch_stab_few(const QueryArgs& q) {
+    if (q.n <= 0) return hipSuccess;
+    if (stack_capacity_for(q.stack_need) < 0 || q.n >= kStabFew) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(dev::stab_few<kStabFewWaves>, dim3((unsigned)q.n), dim3(64 * kStabFewWaves), 0, (hipStream_t)q.stream,
+                       q.in0, q.out_f, dev::make_tree(q.tree, q.face0_slot));
     return hipGetLastError();
 }
 

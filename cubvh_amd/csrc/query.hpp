@@ -63,6 +63,9 @@ hipError_t launch_ray(const QueryArgs& q);
 // ws holds stab_workspace_bytes(q.n) bytes.
 size_t stab_workspace_bytes(int64_t n);
 hipError_t launch_stab_sign(const QueryArgs& q, void* ws);
+// The same for fewer than kStabFew queries, without scratch.
+constexpr int64_t kStabFew = 1 << 11;
+hipError_t launch_stab_few(const QueryArgs& q);
 
 // The VALU issue-ceiling probe (probe.hip): `blocks` workgroups of 256 threads, each
 // thread kValuProbeChains independent fp32 fma chains of `iters` steps; form 0 = VGPR

@@ -118,3 +118,39 @@ def test_calls_that_promise_it_allocate_nothing(gpu):
         assert _pool_high(gpu, ordered) == 0
     assert _pool_high(gpu, lambda: _lib.check(_call(lib.cubvh_unsigned_distance_noalloc, bvh, P, out))) == 0
     assert _pool_high(gpu, lambda: _lib.check(_call(lib.cubvh_unsigned_distance, bvh, P, out))) > 4 * n
+
+
+@pytest.mark.parametrize("n", [1, 7, 600, 2047])
+def test_raystab_of_few_points_allocates_nothing(gpu, n):
+    """Raystab below 2,048 points takes nothing from the pool and can be captured: replays
+    between eager work give the eager signs, which are the larger calls' and the oracle's."""
+    from oracle import oracle as O
+
+    for closed in (True, False):
+        v, f = S.icosphere(3, 0.5) if closed else S.soup(3, seed=3, n_random=300)
+        bvh = cubvh_amd.cuBVH(v, f)
+        p = S.uniform_points(2300, seed=n)
+        p[: n // 2] *= 0.2
+        P = torch.from_numpy(p).to(gpu)
+        large = bvh.signed_distance(P, mode="raystab")
+        ref = bvh.signed_distance(P[:n], mode="raystab")
+        assert torch.equal(ref[0].view(torch.int32), large[0][:n].view(torch.int32)) and torch.equal(ref[1], large[1][:n])
+        od, of, _ = O.sdf_brute(v, f, p[:n], 1, return_uvw=False)
+        np.testing.assert_array_equal(ref[0].cpu().numpy(), od)
+        np.testing.assert_array_equal(ref[1].cpu().numpy(), of)
+        out = _outputs(n, gpu)
+        lib, x = _lib.load(), P[:n].contiguous()
+
+        def call():
+            s = ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)
+            _lib.check(lib.cubvh_signed_distance(bvh._h, gpu.index, n, 1, x.data_ptr(), *[t.data_ptr() for t in out], s))
+
+        assert _pool_high(gpu, call) == 0
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            call()
+        for _ in range(3):
+            out[0].zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out[0].view(torch.int32), ref[0].view(torch.int32)) and torch.equal(out[1], ref[1])
