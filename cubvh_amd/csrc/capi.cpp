@@ -375,6 +375,7 @@ int run_distance(cubvh_bvh* bvh, int device, int64_t n, int kmode, const float* 
                 return fail_hip(e, "query ordering");
             }
             q.order = order;
+            q.permutation = true;
         }
     }
     q.packet = ordered;

@@ -446,11 +446,13 @@ struct NormalSum {
 struct NormalParts {
     double* keep;
     double x, y, z;
+    float n;
     int part = 0;
     bool more;  // components hold lower parts
 
     __device__ __forceinline__ void start() {
         x = y = z = 0.0;
+        n = 0.0f;
         more = false;
     }
     __device__ __forceinline__ double part_of(float v) {
@@ -467,6 +469,7 @@ struct NormalParts {
         x += part_of(v.x);
         y += part_of(v.y);
         z += part_of(v.z);
+        n += 1.0f;
     }
     // After a walk: whether another one is needed.
     __device__ __forceinline__ bool next() {
@@ -475,7 +478,7 @@ struct NormalParts {
         keep[3 * part + 2] = z;
         return ++part < 6 && more;
     }
-    __device__ __forceinline__ f3 mean(float n) const {
+    __device__ __forceinline__ f3 mean() const {
         double v[3];
         for (int k = 0; k < 3; ++k) {
             double h = 0.0, e = 0.0;
@@ -526,17 +529,20 @@ __device__ __forceinline__ void add_normals(const Tree& T, f3 c, LaneStack<BLOCK
 // Mean unit normal of every face within squared distance NORMAL_EPS of point c
 // (src/bvh.cu:356-396): the sum rounded to float and divided by the count (0 / 0 for none).
 template <int BLOCK, int LDS_N>
-__device__ f3 avg_normal(const Tree& T, f3 c, LaneStack<BLOCK, LDS_N>& st) {
-    NormalSum sum;
-    add_normals(T, c, st, sum);
-    if (sum.exact()) return sum.mean();
+__device__ f3 avg_normal_parts(const Tree& T, f3 c, LaneStack<BLOCK, LDS_N>& st) {
     double keep[18];
     NormalParts parts{keep};
     do {
         parts.start();
         add_normals(T, c, st, parts);
     } while (parts.next());
-    return parts.mean(sum.n);
+    return parts.mean();
+}
+template <int BLOCK, int LDS_N>
+__device__ f3 avg_normal(const Tree& T, f3 c, LaneStack<BLOCK, LDS_N>& st) {
+    NormalSum sum;
+    add_normals(T, c, st, sum);
+    return sum.exact() ? sum.mean() : avg_normal_parts(T, c, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -1488,7 +1494,10 @@ __global__ __launch_bounds__(256) void stab_negate(const uint32_t* __restrict__ 
 constexpr int kNormalLds = 4;  // LDS entries per lane of the per-lane normal search
 
 // Writes query q's outputs from its nearest face (slot < 0: none within MAX_DIST, which
-// reports distance 0 to face 0).  Lanes with valid = false write nothing.
+// reports distance 0 to face 0).  Lanes with valid = false write nothing.  MODE 1 leaves the
+// sign of a query whose normals have to be added in exact parts to sign_parts, with the
+// complement of its face's slot for the face id: that code's registers, inlined here, cost
+// every query 2 to 10% (7,000,000 points near 320 faces 1,020 us without, 1,114 with it).
 template <int MODE, int WAVES>
 __device__ __forceinline__ void finish_query(const Tree& T, int32_t face0_slot, bool valid, int64_t q, f3 p, float d2,
                                              int32_t slot, float* __restrict__ distances,
@@ -1517,14 +1526,64 @@ __device__ __forceinline__ void finish_query(const Tree& T, int32_t face0_slot, 
         st.tid = (int)threadIdx.x;
         st.sp = 0;
         if (valid) {
-            f3 nrm = avg_normal(T, cp, st);
-            dist = copysignf(dist, dot3(nrm, sub3(p, cp)));
+            NormalSum sum;
+            add_normals(T, cp, st, sum);
+            dist = copysignf(dist, dot3(sum.mean(), sub3(p, cp)));
+            if (!sum.exact()) id = ~slot;
         }
     }
     if (!valid) return;
     distances[q] = dist;
     face_id[q] = (int64_t)id;
     if (uvw) store_pt(uvw, q, tri_barycentric(a, b, c, cp));
+}
+
+// The signs that finish_query left (of the queries in order, or of all n).  Nearly always a
+// read of the face ids, kPartsScan at once per lane: 15 us for 7,000,000.
+constexpr int kPartsScan = 8;
+__device__ __forceinline__ void sign_part(const float* __restrict__ positions, float* __restrict__ distances,
+                                          int64_t* __restrict__ face_id, const Tree& T, int64_t q, int32_t slot,
+                                          LaneStack<64, kNormalLds>& st) {
+    const f3 p = load_pt(positions, q);
+    f3 a, b, c;
+    int32_t id;
+    load_tri(T.tris, slot, a, b, c, id);
+    const f3 cp = tri_closest_pt(a, b, c, p);
+    distances[q] = copysignf(distances[q], dot3(avg_normal_parts(T, cp, st), sub3(p, cp)));
+    face_id[q] = (int64_t)id;
+}
+__global__ __launch_bounds__(64) void sign_parts(int64_t n, const uint32_t* __restrict__ order,
+                                                 const float* __restrict__ positions, float* __restrict__ distances,
+                                                 int64_t* __restrict__ face_id, Tree T) {
+    __shared__ int32_t s_ref[kNormalLds * 64];
+    __shared__ float s_key[kNormalLds * 64];
+    LaneStack<64, kNormalLds> st;
+    st.ref = s_ref;
+    st.key = s_key;
+    st.tid = (int)threadIdx.x;
+    for (int64_t at = (int64_t)blockIdx.x * (64 * kPartsScan); at < n; at += (int64_t)gridDim.x * (64 * kPartsScan)) {
+        int64_t q[kPartsScan], left[kPartsScan];
+#pragma unroll
+        for (int k = 0; k < kPartsScan; ++k) {
+            const int64_t i = at + 64 * k + threadIdx.x;
+            q[k] = i < n ? (order ? (int64_t)order[i] : i) : n;
+        }
+        bool any = false;
+#pragma unroll
+        for (int k = 0; k < kPartsScan; ++k) {
+            left[k] = q[k] < n ? face_id[q[k]] : 0;
+            any = any || left[k] < 0;
+        }
+        if (ballot(any) == 0) continue;
+        for (int k = 0; k < kPartsScan; ++k) {
+            const int64_t i = at + 64 * k + threadIdx.x;
+            if (i >= n) break;
+            const int64_t qk = order ? (int64_t)order[i] : i;
+            if (qk >= n) continue;
+            const int64_t l = face_id[qk];
+            if (l < 0) sign_part(positions, distances, face_id, T, qk, (int32_t)~l, st);
+        }
+    }
 }
 
 // Packet kernel for the unsigned (MODE 0) and watertight signed (MODE 1) distance, WAVES
@@ -1756,6 +1815,11 @@ hipError_t launch_distance_impl(const QueryArgs& q, int mode) {
             hipLaunchKernelGGL((mode == 0 ? dev::distance_rest_kernel<0> : dev::distance_rest_kernel<1>),
                                dim3(std::min<uint32_t>(rest_cap(q.n), kRestBlocks)), dim3(64), 0, s, rest, q.in0, q.out_f, q.out_id,
                                q.out_v, T);
+        if (mode == 1) {  // every face id is written by now
+            constexpr int64_t P = 64 * dev::kPartsScan;
+            hipLaunchKernelGGL(dev::sign_parts, dim3((unsigned)std::min<int64_t>((q.n + P - 1) / P, kRestBlocks)), dim3(64), 0, s, q.n,
+                               q.permutation ? nullptr : q.order, q.in0, q.out_f, q.out_id, T);
+        }
         return hipGetLastError();
     }
     const unsigned grid = (unsigned)((q.n + kBlock - 1) / kBlock);

@@ -23,6 +23,7 @@ struct QueryArgs {
     const float* in0 = nullptr;  // positions or ray origins [n,3]
     const float* in1 = nullptr;  // ray directions [n,3]
     const uint32_t* order = nullptr;  // optional query permutation [n] (lane i handles query order[i])
+    bool permutation = false;    // order holds every query (a caller's may not)
     float* out_f = nullptr;      // distances or depth [n]
     int64_t* out_id = nullptr;   // face ids [n]
     float* out_v = nullptr;      // uvw or hit positions [n,3]

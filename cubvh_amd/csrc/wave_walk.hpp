@@ -326,7 +326,7 @@ __device__ f3 avg_normal_wave(const Tree& T, f3 c, WaveLists& L) {
         wave_fence();
     } while (parts.next());
     wave_fence();
-    return parts.mean(sum.n);
+    return parts.mean();
 }
 
 // Closest hit of the ray (wave-uniform arguments and results), as closest_hit; best / bslot

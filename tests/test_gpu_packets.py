@@ -1,5 +1,6 @@
 """Packet walks (64 queries or rays a wave) where they can go wrong, held to the wave walks
 and to the oracle."""
+import ctypes
 import math
 
 import numpy as np
@@ -67,3 +68,28 @@ def test_watertight_sign_is_the_exact_normal_sums(gpu, n_faces, builder):
         packets = bvh.distance_ordered(p, torch.arange(100, dtype=torch.int32, device=gpu), signed=True)
         same_bits(waves[:2], packets[:2])
         assert bool((torch.signbit(waves[0]) == inside).all())
+
+
+def test_ordered_calls_leave_skipped_queries_alone(gpu):
+    """Order entries past the end: the queries they leave out keep their outputs, whatever is
+    in them, and the others get theirs, small normals among the sheets or not."""
+    faces = np.array([[[0, 0, 0], [1, 0, 0], [0, 1, 0]], [[0, 0, 0], [0, 1, 0], [1, 0, 0]], [[0, 0, 0], [0, 1, 0], [-1e-20, 0, -1]]],
+                     np.float32)[[0, 1, 2] * 4]
+    bvh = cubvh_amd.cuBVH(faces.reshape(-1, 3), np.arange(36, dtype=np.int32).reshape(-1, 3))
+    n = 5000
+    p = torch.rand(n, 3, device=gpu)
+    p[:, 0] = 0.0
+    order = torch.randperm(n, device=gpu).to(torch.int32)
+    skipped = order[::3].long()
+    order[::3] = n + 7
+    d = torch.full((n,), 3.0, device=gpu)
+    f = torch.full((n,), -12345, dtype=torch.int64, device=gpu)
+    lib = cubvh_amd._lib.load()
+    stream = ctypes.c_void_p(torch.cuda.current_stream(gpu).cuda_stream)
+    cubvh_amd._lib.check(lib.cubvh_distance_ordered(bvh._h, gpu.index, n, 1, p.data_ptr(), order.data_ptr(), d.data_ptr(),
+                                                    f.data_ptr(), None, stream))
+    ref = bvh.signed_distance(p)
+    kept = torch.ones(n, dtype=torch.bool, device=gpu)
+    kept[skipped] = False
+    assert bool((d[skipped] == 3.0).all()) and bool((f[skipped] == -12345).all())
+    same_bits([d[kept], f[kept]], [ref[0][kept], ref[1][kept]])
