@@ -210,6 +210,7 @@ struct cubvh_bvh {
         q.n = n;
         q.tree = dev[device].view;
         q.face0_slot = host.face0_slot;
+        q.n_faces = host.n_faces;
         q.stack_need = host.stack_need;
         q.stream = stream;
         return q;
@@ -226,6 +227,7 @@ struct cubvh_forest {
     std::vector<int32_t> mesh_info;  // 4 per mesh: root, face-0 slot, n_faces, 0
     int32_t n_meshes = 0;
     int64_t n_faces = 0;
+    int64_t most_faces = 0;  // of one mesh
     int64_t n_nodes = 0;
     int32_t stack_need = 0;
     // >= 0: assembled on that device from trees built there; no host arrays
@@ -363,12 +365,12 @@ int run_distance(cubvh_bvh* bvh, int device, int64_t n, int kmode, const float* 
         // the stab passes' lists, then the order, the rest of the walks and the ordering workspace
         const size_t sb = lists ? ((stab_workspace_bytes(n) + 255) & ~(size_t)255) : 0;
         const size_t ob = ordered ? ((size_t)n * 4 + 255) & ~(size_t)255 : 0;
-        const size_t rb = ordered ? rest_bytes(n) : 0;
+        const size_t rb = ordered ? rest_bytes(n, q.n_faces) : 0;
         hipError_t e = hipMallocAsync(&scratch, sb + ob + rb + (ordered ? morton_workspace_bytes(n) : 0), hs);
         if (e != hipSuccess) return fail_hip(e, "hipMallocAsync(query order)");
         if (ordered) {
             uint32_t* order = (uint32_t*)((char*)scratch + sb);
-            q.rest = (char*)scratch + sb + ob;
+            if (rb) q.rest = (char*)scratch + sb + ob;
             e = morton_order(n, positions, (char*)scratch + sb + ob + rb, order, hs);
             if (e != hipSuccess) {
                 (void)hipFreeAsync(scratch, hs);
@@ -779,11 +781,11 @@ int cubvh_unsigned_distance_noalloc(cubvh_bvh* bvh, int device, int64_t n, const
         hipError_t e = noalloc_scratch(device, &ws);
         if (e != hipSuccess) return fail_hip(e, "hipGetSymbolAddress(scratch)");
         const size_t ob = ((size_t)n * 4 + 255) & ~(size_t)255;
-        const size_t rb = rest_bytes(n);
+        const size_t rb = rest_bytes(n, q.n_faces);
         if (ob + rb + morton_workspace_bytes(n) > kNoAllocScratchBytes)
             return fail(CUBVH_ERR_STATE, "the ordering workspace does not fit the static scratch");
         uint32_t* order = (uint32_t*)ws;
-        q.rest = (char*)ws + ob;
+        if (rb) q.rest = (char*)ws + ob;
         e = morton_order(n, positions, (char*)ws + ob + rb, order, hs);
         if (e != hipSuccess) return fail_hip(e, "query ordering");
         q.order = order;
@@ -913,10 +915,10 @@ int cubvh_ray_trace(cubvh_bvh* bvh, int device, int64_t n, const float* rays_o, 
         rc = ensure_pool(device);
         if (rc != CUBVH_OK) return rc;
         const size_t ob = ((size_t)n * 4 + 255) & ~(size_t)255;
-        const size_t rb = rest_bytes(n);
+        const size_t rb = ray_rest_bytes(n, q.n_faces);
         hipError_t e = hipMallocAsync(&scratch, ob + rb + morton_workspace_bytes(n), hs);
         if (e != hipSuccess) return fail_hip(e, "hipMallocAsync(ray order)");
-        q.rest = (char*)scratch + ob;
+        if (rb) q.rest = (char*)scratch + ob;
         e = ray_order(n, rays_o, rays_d, (char*)scratch + ob + rb, (uint32_t*)scratch, hs);
         if (e != hipSuccess) {
             (void)hipFreeAsync(scratch, hs);
@@ -1057,6 +1059,7 @@ int forest_create_on_device(cubvh_bvh* const* bvhs, int32_t n_meshes, int32_t de
         f->mesh_info[4 * m + 2] = (int32_t)b->host.n_faces;
         f->n_nodes += b->n_nodes;
         f->n_faces += b->host.n_faces;
+        f->most_faces = std::max(f->most_faces, b->host.n_faces);
         f->stack_need = std::max(f->stack_need, b->host.stack_need);
     }
     if (stack_capacity_for(f->stack_need) < 0) {
@@ -1151,6 +1154,7 @@ int cubvh_forest_create(cubvh_bvh* const* bvhs, int32_t n_meshes, cubvh_forest**
         f->mesh_info[4 * m + 1] = (int32_t)(tri_base + h.face0_slot);
         f->mesh_info[4 * m + 2] = (int32_t)h.n_faces;
         f->n_faces += h.n_faces;
+        f->most_faces = std::max(f->most_faces, h.n_faces);
         f->stack_need = std::max(f->stack_need, h.stack_need);
     }
     f->n_nodes = (int64_t)f->nodes.size();
@@ -1252,6 +1256,7 @@ int cubvh_forest_unsigned_distance(cubvh_forest* forest, int device, int64_t n, 
     a.uvw = uvw;
     a.tree = c.tree.view;
     a.mesh_info = c.mesh_info;
+    a.most_faces = forest->most_faces;
     a.persistent = persistent;
     a.waves_per_cu = wpc;
     a.waves_per_block = wpb;

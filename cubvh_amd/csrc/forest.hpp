@@ -41,6 +41,7 @@ struct ForestArgs {
     float* uvw = nullptr;
     TreeArrays tree;
     const int4* mesh_info = nullptr;  // per mesh: root node, face-0 slot, n_faces, 0
+    int64_t most_faces = 0;           // of one mesh
     int32_t persistent = 0;
     int32_t waves_per_cu = 8;
     int32_t waves_per_block = 4;  // 1, 2, 4 or 8 (workgroups of 64..512 lanes)

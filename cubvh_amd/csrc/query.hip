@@ -253,9 +253,9 @@ __device__ __forceinline__ f3 ray_inverse(f3 d) {
     return mk3(1.0f / x, 1.0f / y, 1.0f / z);
 }
 
-// Closest hit.  Returns the leaf slot (-1 on a miss) and t in best_t; budget is left
-// negative by a walk that has more to visit after that many steps (nodes and faces).
-template <int BLOCK, int LDS_N>
+// Closest hit.  Returns the leaf slot (-1 on a miss) and t in best_t; with REST, budget is
+// left negative by a walk that has more to visit after that many steps (nodes and faces).
+template <bool REST, int BLOCK, int LDS_N>
 __device__ int32_t closest_hit(const Tree& T, f3 o, f3 d, LaneStack<BLOCK, LDS_N>& st, float& best_t, int32_t& budget) {
     f3 inv = ray_inverse(d);
     float best = MAX_DIST;
@@ -264,7 +264,7 @@ __device__ int32_t closest_hit(const Tree& T, f3 o, f3 d, LaneStack<BLOCK, LDS_N
     int32_t ref = 0;
     st.sp = 0;
     for (;;) {
-        --budget;
+        if (REST) --budget;
         if (ref >= 0) {
             WideNode nd = load_node(T.nodes, ref);
             float k[4];
@@ -281,7 +281,7 @@ __device__ int32_t closest_hit(const Tree& T, f3 o, f3 d, LaneStack<BLOCK, LDS_N
         } else {
             int32_t first, count;
             leaf_range(ref, first, count);
-            budget -= count;
+            if (REST) budget -= count;
             for (int j = 0; j < count; ++j) {
                 f3 a, b, c;
                 int32_t id;
@@ -304,10 +304,10 @@ __device__ int32_t closest_hit(const Tree& T, f3 o, f3 d, LaneStack<BLOCK, LDS_N
             }
         }
         if (ref == CHILD_EMPTY) {
-            budget = 0;
+            if (REST) budget = 0;
             break;
         }
-        if (budget < 0) break;
+        if (REST && budget < 0) break;
     }
     best_t = best;
     return bslot;
@@ -985,6 +985,7 @@ __device__ __forceinline__ float slab_entry(float lx, float hx, float ly, float 
     return (tn <= tf && tf >= 0.0f) ? tn : INFINITY;
 }
 
+template <bool REST>
 __device__ uint64_t closest_hit_packet(const Tree& T, f3 o, f3 d, bool active, float& best, int32_t& bslot,
                                        int32_t& bid, float reach, ExactQueue& q, PacketRest* rest,
                                        int32_t& base) {
@@ -1000,9 +1001,9 @@ __device__ uint64_t closest_hit_packet(const Tree& T, f3 o, f3 d, bool active, f
     if (mask == 0) return 0;
     WaveStack st;
     int32_t ref = 0;
-    int32_t budget = rest ? kRaySteps : INT32_MAX;
+    int32_t budget = kRaySteps;
     for (;;) {
-        --budget;
+        if (REST) --budget;
         if (ref >= 0) {
             UNode nd = load_unode(T.nodes, ref);
             float k0 = nd.child.x != CHILD_EMPTY ? slab_entry(nd.lx.x, nd.hx.x, nd.ly.x, nd.hy.x, nd.lz.x, nd.hz.x, o, inv) : INFINITY;
@@ -1034,7 +1035,7 @@ __device__ uint64_t closest_hit_packet(const Tree& T, f3 o, f3 d, bool active, f
         } else {
             int32_t first, count;
             leaf_range(ref, first, count);
-            budget -= count;
+            if (REST) budget -= count;
             const int32_t nl = __builtin_popcountll(mask);
             if (nl > kRayStepLanes) {
                 for (int j = 0; j < count; ++j) {
@@ -1089,7 +1090,7 @@ __device__ uint64_t closest_hit_packet(const Tree& T, f3 o, f3 d, bool active, f
         }
         if (!st.pop(ref, mask)) break;
         ref = uniform(ref);
-        if (budget < 0) {
+        if (REST && budget < 0) {
             left = mask | st.lanes();
             base = reserve_rest(rest, left);
             if (base >= 0) break;
@@ -1147,14 +1148,14 @@ union PacketLds {
 // 1.3 M faces, 35 with the distances known); the wave's walk costs about 5% of a tile's
 // instructions.  256^3 grid 12.77 -> 11.29 ms, 2^20 points forward and backward 1.59 ->
 // 1.39, 48-mesh batch 2.68 -> 2.40, 128^3 watertight grid 2.45 -> 2.26 ms.
-__device__ __forceinline__ void seed_packet(const Tree& T, int32_t root, f3 p, bool active, WaveLists& L, float& best,
-                                            int32_t& bslot, int32_t& bid) {
+__device__ __forceinline__ void seed_packet(const Tree& T, int32_t root, f3 p, bool active, bool seed, WaveLists& L,
+                                            float& best, int32_t& bslot, int32_t& bid) {
     best = MAX_DIST_SQ;
     bslot = -1;
     bid = 0x7fffffff;
     const bool in = active && !has_nan(p);
     const uint64_t mask = ballot(in);
-    if (mask == 0) return;
+    if (!seed || mask == 0) return;
     f3 c = in ? p : mk3(0.0f, 0.0f, 0.0f);
     for (int o = 32; o > 0; o >>= 1) c = mk3(c.x + __shfl_xor(c.x, o), c.y + __shfl_xor(c.y, o), c.z + __shfl_xor(c.z, o));
     const float w = 1.0f / (float)__builtin_popcountll(mask);
@@ -1595,7 +1596,7 @@ __global__ __launch_bounds__(64 * WAVES, 8) void distance_packet_kernel(int64_t 
                                                               const uint32_t* __restrict__ order,
                                                               float* __restrict__ distances,
                                                               int64_t* __restrict__ face_id, float* __restrict__ uvw,
-                                                              Tree T, uint32_t xchunk,
+                                                              Tree T, uint32_t xchunk, bool seed,
                                                               PacketRest* rest) {
     const int64_t i = (int64_t)xcd_remap(blockIdx.x, gridDim.x, xchunk) * (64 * WAVES) + threadIdx.x;
     int64_t q = i;
@@ -1607,7 +1608,7 @@ __global__ __launch_bounds__(64 * WAVES, 8) void distance_packet_kernel(int64_t 
     int32_t slot, bid, base;
     __shared__ PacketLds lds[WAVES];
     PacketLds& L = lds[threadIdx.x >> 6];
-    seed_packet(T, 0, p, valid, L.lists, d2, slot, bid);
+    seed_packet(T, 0, p, valid, seed, L.lists, d2, slot, bid);
     const uint64_t left = closest_face_packet<REST>(T, 0, p, valid, d2, slot, bid, L.queue, rest, i >> 6, base);
     if (REST && left != 0) leave_rest(rest, left, base, q, d2, slot >= 0 ? slot : ~(int32_t)T.face0_slot, 0);
     const bool mine = valid && !(REST && ((left >> (threadIdx.x & 63)) & 1));
@@ -1617,7 +1618,7 @@ __global__ __launch_bounds__(64 * WAVES, 8) void distance_packet_kernel(int64_t 
 // Unsigned distance over a forest: one wave per 64-slot tile of the padded query
 // order; every tile belongs to one mesh, whose root node and face-0 slot come from
 // mesh_info.  PERSISTENT waves take tiles from an atomic counter until none is left.
-template <int PERSISTENT, int WAVES>
+template <int PERSISTENT, int WAVES, bool REST>
 __global__ __launch_bounds__(64 * WAVES, PERSISTENT ? 7 : 8) void forest_distance_kernel(const float* __restrict__ positions,
                                                               const uint32_t* __restrict__ order,
                                                               const int64_t* __restrict__ pbase, int32_t n_meshes,
@@ -1625,7 +1626,7 @@ __global__ __launch_bounds__(64 * WAVES, PERSISTENT ? 7 : 8) void forest_distanc
                                                               float* __restrict__ distances,
                                                               int64_t* __restrict__ face_id, float* __restrict__ uvw,
                                                               TreeArrays arrays, uint32_t* counter,
-                                                              int64_t max_tiles, uint32_t xcd_chunk, PacketRest* rest) {
+                                                              int64_t max_tiles, uint32_t xcd_chunk, bool seed, PacketRest* rest) {
     __shared__ PacketLds lds[WAVES];
     PacketLds& L = lds[threadIdx.x >> 6];
     const int lane = (int)(threadIdx.x & 63);
@@ -1657,10 +1658,10 @@ __global__ __launch_bounds__(64 * WAVES, PERSISTENT ? 7 : 8) void forest_distanc
         float d2;
         int32_t slot, bid, base;
         const int32_t root = uniform(mi.x);
-        seed_packet(T, root, p, valid, L.lists, d2, slot, bid);
-        const uint64_t left = closest_face_packet<true>(T, root, p, valid, d2, slot, bid, L.queue, rest, tile, base);
-        if (left != 0) leave_rest(rest, left, base, (int64_t)qi, d2, slot >= 0 ? slot : ~mi.y, mi.x);
-        const bool mine = valid && !((left >> lane) & 1);
+        seed_packet(T, root, p, valid, seed, L.lists, d2, slot, bid);
+        const uint64_t left = closest_face_packet<REST>(T, root, p, valid, d2, slot, bid, L.queue, rest, tile, base);
+        if (REST && left != 0) leave_rest(rest, left, base, (int64_t)qi, d2, slot >= 0 ? slot : ~mi.y, mi.x);
+        const bool mine = valid && !(REST && ((left >> lane) & 1));
         finish_query<0, WAVES>(T, mi.y, mine, (int64_t)qi, p, d2, slot, distances, face_id, uvw);
         // One back edge: without it the compiler may thread a lane test at the loop's end
         // to the one at its start, sending some lanes around without lane 0.
@@ -1675,7 +1676,7 @@ __global__ __launch_bounds__(64 * WAVES, PERSISTENT ? 7 : 8) void forest_distanc
 // any other wave walks lane by lane.  Both give closest_hit's results.
 constexpr int kRayLds = 8;
 constexpr int32_t kLaneSteps = 512;  // steps of a lane's walk before a wave takes over
-template <int WAVES>
+template <int WAVES, bool REST>
 __global__ __launch_bounds__(64 * WAVES, 8) void ray_packet_kernel(int64_t n, const float* __restrict__ rays_o,
                                                          const float* __restrict__ rays_d,
                                                          const uint32_t* __restrict__ order,
@@ -1722,24 +1723,25 @@ __global__ __launch_bounds__(64 * WAVES, 8) void ray_packet_kernel(int64_t n, co
     int32_t slot = -1, bid = 0, base = -1;
     uint64_t left;
     if (ballot(near) == ~0ull) {
-        left = closest_hit_packet(T, o, d, valid, t, slot, bid, reach, lds.queue[0], rest, base);
+        left = closest_hit_packet<REST>(T, o, d, valid, t, slot, bid, reach, lds.queue[0], rest, base);
     } else {
         LaneStack<64 * WAVES, kRayLds> st;
         st.ref = lds.lanes.ref;
         st.key = lds.lanes.key;
         st.tid = (int)threadIdx.x;
-        for (int32_t budget = rest ? kLaneSteps : INT32_MAX;; budget = INT32_MAX) {
+        left = 0;
+        for (int32_t budget = kLaneSteps;; budget = INT32_MAX) {
             int32_t b = valid ? budget : 0;
-            if (valid) slot = closest_hit(T, o, d, st, t, b);
-            left = ballot(b < 0);
+            if (valid) slot = closest_hit<REST>(T, o, d, st, t, b);
+            if (REST) left = ballot(b < 0);
             if (left == 0) break;
             base = reserve_rest(rest, left);
             if (base >= 0) break;  // else no room: the wave walks to the end
         }
         if (slot >= 0) bid = __float_as_int(T.tris[3 * slot].w);
     }
-    if (left != 0) leave_rest(rest, left, base, i, t, slot, 0);
-    if (!valid || ((left >> (threadIdx.x & 63)) & 1)) return;
+    if (REST && left != 0) leave_rest(rest, left, base, i, t, slot, 0);
+    if (!valid || (REST && ((left >> (threadIdx.x & 63)) & 1))) return;
     depth[i] = t;
     store_pt(positions, i, mk3(__builtin_fmaf(t, d.x, o.x), __builtin_fmaf(t, d.y, o.y), __builtin_fmaf(t, d.z, o.z)));
     face_id[i] = slot >= 0 ? (int64_t)bid : -1;
@@ -1806,11 +1808,11 @@ hipError_t launch_distance_impl(const QueryArgs& q, int mode) {
         const unsigned grid = (unsigned)((q.n + 64 * W - 1) / (64 * W));
         const uint32_t xchunk = xcd_chunk_for(grid);
         dev::PacketRest* rest = (dev::PacketRest*)q.rest;
-        if (q.n >= kRestLast) rest = nullptr;
         if (rest) launch_rest_init(rest, q.n, mode == 0 ? 2.5 : 3.5, s);
         const auto kernel = mode == 0 ? (rest ? dev::distance_packet_kernel<0, W, true> : dev::distance_packet_kernel<0, W, false>)
                                       : (rest ? dev::distance_packet_kernel<1, W, true> : dev::distance_packet_kernel<1, W, false>);
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), 0, s, q.n, q.in0, q.order, q.out_f, q.out_id, q.out_v, T, xchunk, rest);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), 0, s, q.n, q.in0, q.order, q.out_f, q.out_id, q.out_v, T, xchunk,
+                           q.n / kSeedQueries < q.n_faces, rest);
         if (rest)
             hipLaunchKernelGGL((mode == 0 ? dev::distance_rest_kernel<0> : dev::distance_rest_kernel<1>),
                                dim3(std::min<uint32_t>(rest_cap(q.n), kRestBlocks)), dim3(64), 0, s, rest, q.in0, q.out_f, q.out_id,
@@ -1848,21 +1850,18 @@ namespace {
 template <int WAVES>
 hipError_t launch_forest_shape(const ForestArgs& a, const ForestWorkspace& ws, hipStream_t s) {
     const int64_t max_tiles = ws.npad_max / 64;
-    dev::PacketRest* rest = (dev::PacketRest*)ws.rest;
-    launch_rest_init(rest, ws.npad_max, 2.5, s);
-    if (a.persistent) {
-        const unsigned blocks = (unsigned)std::max(1, a.n_cu * a.waves_per_cu / WAVES);
-        hipLaunchKernelGGL((dev::forest_distance_kernel<1, WAVES>), dim3(blocks), dim3(64 * WAVES), 0, s, a.positions,
-                           ws.order, ws.pbase, a.n_meshes, a.mesh_info, a.distances, a.face_id, a.uvw, a.tree,
-                           ws.counter, max_tiles, 0u, rest);
-    } else {
-        const unsigned blocks = (unsigned)((max_tiles + WAVES - 1) / WAVES);
-        hipLaunchKernelGGL((dev::forest_distance_kernel<0, WAVES>), dim3(blocks), dim3(64 * WAVES), 0, s, a.positions,
-                           ws.order, ws.pbase, a.n_meshes, a.mesh_info, a.distances, a.face_id, a.uvw, a.tree,
-                           ws.counter, max_tiles, (uint32_t)a.xcd_chunk, rest);
-    }
-    hipLaunchKernelGGL(dev::distance_rest_kernel<0>, dim3(std::min<uint32_t>(rest_cap(ws.npad_max), kRestBlocks)), dim3(64), 0, s, rest,
-                       a.positions, a.distances, a.face_id, a.uvw, dev::make_tree(a.tree, 0));
+    dev::PacketRest* rest = hands_over(ws.npad_max, a.most_faces) ? (dev::PacketRest*)ws.rest : nullptr;
+    if (rest) launch_rest_init(rest, ws.npad_max, 2.5, s);
+    const auto kernel = a.persistent ? (rest ? dev::forest_distance_kernel<1, WAVES, true> : dev::forest_distance_kernel<1, WAVES, false>)
+                                     : (rest ? dev::forest_distance_kernel<0, WAVES, true> : dev::forest_distance_kernel<0, WAVES, false>);
+    const unsigned blocks = a.persistent ? (unsigned)std::max(1, a.n_cu * a.waves_per_cu / WAVES)
+                                         : (unsigned)((max_tiles + WAVES - 1) / WAVES);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * WAVES), 0, s, a.positions, ws.order, ws.pbase, a.n_meshes, a.mesh_info,
+                       a.distances, a.face_id, a.uvw, a.tree, ws.counter, max_tiles, a.persistent ? 0u : (uint32_t)a.xcd_chunk,
+                       a.n / kSeedQueries < a.most_faces, rest);
+    if (rest)
+        hipLaunchKernelGGL(dev::distance_rest_kernel<0>, dim3(std::min<uint32_t>(rest_cap(ws.npad_max), kRestBlocks)), dim3(64), 0, s,
+                           rest, a.positions, a.distances, a.face_id, a.uvw, dev::make_tree(a.tree, 0));
     return hipGetLastError();
 }
 
@@ -1960,7 +1959,7 @@ hipError_t launch_ray(const QueryArgs& q) {
         hipStream_t s = (hipStream_t)q.stream;
         dev::PacketRest* rest = (dev::PacketRest*)q.rest;
         if (rest) launch_rest_init(rest, q.n, 1.0, s);
-        hipLaunchKernelGGL(dev::ray_packet_kernel<W>, dim3(grid), dim3(64 * W), 0, s, q.n, q.in0, q.in1, q.order, q.out_v,
+        hipLaunchKernelGGL((rest ? dev::ray_packet_kernel<W, true> : dev::ray_packet_kernel<W, false>), dim3(grid), dim3(64 * W), 0, s, q.n, q.in0, q.in1, q.order, q.out_v,
                            q.out_id, q.out_f, T, rest);
         if (rest)
             hipLaunchKernelGGL(dev::ray_rest_kernel, dim3(std::min<uint32_t>(rest_cap(q.n), kRestBlocks)), dim3(64), 0, s, rest, q.in0,

@@ -29,6 +29,7 @@ struct QueryArgs {
     float* out_v = nullptr;      // uvw or hit positions [n,3]
     TreeArrays tree;
     int64_t face0_slot = 0;
+    int64_t n_faces = 0;
     int32_t stack_need = 0;
     bool packet = true;  // walk as wave packets (queries in Morton order)
     void* rest = nullptr;  // packets: rest_bytes(n) bytes for the queries of given-up walks, or null: none is
@@ -50,11 +51,37 @@ int stack_capacity_for(int need);
 // Queries one call's packet walks may hand on to waves of their own (query.hip); the
 // walks past that many run to their end.
 constexpr int64_t kRestMax = 1 << 19;
-// Calls of this many queries hand nothing over: their 20 and more rounds of tiles cover the
-// long walks, and without the hand-over the walk needs no scratch (2^24 grid points on 1.3 M
-// faces: 12.45 ms without, 12.76 with; on 327,680: 7.12 and 7.29).
+// Distance calls hand over below kRestLast queries, and from 16,384 on (walks end by the
+// average of every 16th tile's, and fewer tiles never report enough), on trees of kRestFaces
+// faces and more that have at most kRestQueries queries per face.  On smaller trees no walk is
+// long and the two launches cost 3 to 8%: 2,000,000 points 371 us with, 356 without on 320
+// faces, 425 and 410 on 1,280, but 600,000 near 5,120 jittered faces 479 and 655; many rounds
+// of tiles cover the long walks: 7,000,000 points on 5,120 faces 1,340 us with, 1,305 without,
+// on 20,480 1,742 and 1,680, on 81,920 2,482 and 2,415, but near 327,680 1,836 and 2,705; 2^24
+// grid points on 1.3 M faces 12.76 and 12.45 ms.
+constexpr int64_t kRestFaces = (int64_t)1 << 11;
+constexpr int64_t kRestQueries = (int64_t)1 << 8;
+constexpr int64_t kRestFirst = (int64_t)1 << 14;
 constexpr int64_t kRestLast = (int64_t)1 << 23;
+// Ray calls, whose walks are shorter: 307,200 camera rays on 1.3 M faces 455 us with, 692
+// without, 263,000 scattered ones 754 and 880, 2,000,000 2,023 and 2,067, 7,000,000 5,575 and
+// 5,627 (with the budget that both lane walks counted then); on 81,920 faces 566 and 559.
+constexpr int64_t kRayRestFaces = (int64_t)1 << 18;
+constexpr int64_t kRayRestLast = (int64_t)1 << 22;
+inline bool hands_over(int64_t n, int64_t n_faces) {
+    return n >= kRestFirst && n < kRestLast && n_faces >= kRestFaces && n / kRestQueries < n_faces;
+}
 size_t rest_bytes(int64_t n);
+inline size_t rest_bytes(int64_t n, int64_t n_faces) { return hands_over(n, n_faces) ? rest_bytes(n) : 0; }
+inline size_t ray_rest_bytes(int64_t n, int64_t n_faces) {
+    return n < kRayRestLast && n_faces >= kRayRestFaces ? rest_bytes(n) : 0;
+}
+
+// Packets seed their walks (query.hip) while a face has fewer queries than this: with more,
+// a walk finds its first face at once.  Seeded against not: 320 faces 263,000 points 180 / 201
+// us, 2,000,000 353 / 337, 7,000,000 918 / 834; 5,120 faces 2,000,000 546 / 633, 16,000,000
+// 2,866 / 2,775; 20,480 faces 7,000,000 1,684 / 1,858, 16,000,000 3,515 / 3,581.
+constexpr int64_t kSeedQueries = 1 << 10;
 
 // mode 0 unsigned distance, 1 signed (watertight), 2 signed (raystab)
 hipError_t launch_distance(const QueryArgs& q, int mode);
