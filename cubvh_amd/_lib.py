@@ -48,6 +48,8 @@ SIGNATURES = {
         c_int,
         [c_void_p, c_int, c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
     ),
+    "cubvh_bvh_walk_control": (c_int, [c_void_p, POINTER(c_int32), POINTER(c_uint32)]),
+    "cubvh_forest_walk_control": (c_int, [c_void_p, POINTER(c_int32), POINTER(c_uint32)]),
     "cubvh_floodfill": (c_int, [c_int, c_void_p, c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p]),
     "cubvh_forest_create": (c_int, [c_void_p, c_int32, POINTER(c_void_p)]),
     "cubvh_forest_destroy": (None, [c_void_p]),

@@ -138,6 +138,8 @@ struct DeviceTree {
 struct cubvh_bvh {
     HostBvh host;
     std::mutex mu;
+    WalkControl control;
+    uint32_t handed = 0;  // queries the last call under a control handed over
     DeviceTree dev[kMaxDevices];
 
     ~cubvh_bvh() {
@@ -205,6 +207,13 @@ struct cubvh_bvh {
         return CUBVH_OK;
     }
 
+    // Under a control: how many queries the call's walks handed over (synchronizes).
+    hipError_t count_handed(const QueryArgs& q) {
+        if (!q.control.active()) return hipSuccess;
+        handed = 0;
+        return q.rest ? rest_count(q.rest, (hipStream_t)q.stream, &handed) : hipSuccess;
+    }
+
     QueryArgs args(int device, int64_t n, void* stream) const {
         QueryArgs q;
         q.n = n;
@@ -212,6 +221,7 @@ struct cubvh_bvh {
         q.face0_slot = host.face0_slot;
         q.n_faces = host.n_faces;
         q.stack_need = host.stack_need;
+        q.control = control;
         q.stream = stream;
         return q;
     }
@@ -232,6 +242,8 @@ struct cubvh_forest {
     int32_t stack_need = 0;
     // >= 0: assembled on that device from trees built there; no host arrays
     int32_t resident_device = -1;
+    WalkControl control;
+    uint32_t handed = 0;
     std::mutex mu;
     struct DevCopy {
         DeviceTree tree;
@@ -357,7 +369,8 @@ int run_distance(cubvh_bvh* bvh, int device, int64_t n, int kmode, const float* 
     // lists (stream-ordered scratch from the device's default memory pool, released after
     // the launch).
     void* scratch = nullptr;
-    const bool ordered = n >= kWaveMax && n < ((int64_t)1 << 31);
+    q.walk = walk_of(q.control, n, waves_pay(n, q.n_faces, kmode));
+    const bool ordered = q.walk == Walk::packets;
     const bool lists = kmode == 2 && n >= kStabFew && n < ((int64_t)1 << 31);
     if (ordered || lists) {
         rc = ensure_pool(device);
@@ -365,7 +378,7 @@ int run_distance(cubvh_bvh* bvh, int device, int64_t n, int kmode, const float* 
         // the stab passes' lists, then the order, the rest of the walks and the ordering workspace
         const size_t sb = lists ? ((stab_workspace_bytes(n) + 255) & ~(size_t)255) : 0;
         const size_t ob = ordered ? ((size_t)n * 4 + 255) & ~(size_t)255 : 0;
-        const size_t rb = ordered ? rest_bytes(n, q.n_faces) : 0;
+        const size_t rb = ordered ? rest_bytes(n, q.n_faces, q.control) : 0;
         hipError_t e = hipMallocAsync(&scratch, sb + ob + rb + (ordered ? morton_workspace_bytes(n) : 0), hs);
         if (e != hipSuccess) return fail_hip(e, "hipMallocAsync(query order)");
         if (ordered) {
@@ -380,7 +393,6 @@ int run_distance(cubvh_bvh* bvh, int device, int64_t n, int kmode, const float* 
             q.permutation = true;
         }
     }
-    q.packet = ordered;
     hipError_t e;
     if (lists) {
         // raystab: the distances, then the stab rays
@@ -392,6 +404,7 @@ int run_distance(cubvh_bvh* bvh, int device, int64_t n, int kmode, const float* 
     } else {
         e = launch_distance(q, kmode);
     }
+    if (e == hipSuccess) e = bvh->count_handed(q);
     if (scratch) {
         hipError_t e2 = hipFreeAsync(scratch, hs);
         if (e == hipSuccess) e = e2;
@@ -774,14 +787,15 @@ int cubvh_unsigned_distance_noalloc(cubvh_bvh* bvh, int device, int64_t n, const
     q.out_f = distances;
     q.out_id = face_id;
     q.out_v = uvw;
-    q.packet = false;
+    q.walk = walk_of(WalkControl(), n, waves_pay(n, q.n_faces, 0));
+    q.control = WalkControl();
     hipStream_t hs = (hipStream_t)stream;
-    if (n >= kWaveMax) {
+    if (q.walk == Walk::packets) {
         void* ws = nullptr;
         hipError_t e = noalloc_scratch(device, &ws);
         if (e != hipSuccess) return fail_hip(e, "hipGetSymbolAddress(scratch)");
         const size_t ob = ((size_t)n * 4 + 255) & ~(size_t)255;
-        const size_t rb = rest_bytes(n, q.n_faces);
+        const size_t rb = rest_bytes(n, q.n_faces, q.control);
         if (ob + rb + morton_workspace_bytes(n) > kNoAllocScratchBytes)
             return fail(CUBVH_ERR_STATE, "the ordering workspace does not fit the static scratch");
         uint32_t* order = (uint32_t*)ws;
@@ -789,7 +803,7 @@ int cubvh_unsigned_distance_noalloc(cubvh_bvh* bvh, int device, int64_t n, const
         e = morton_order(n, positions, (char*)ws + ob + rb, order, hs);
         if (e != hipSuccess) return fail_hip(e, "query ordering");
         q.order = order;
-        q.packet = true;
+        q.permutation = true;
     }
     hipError_t e = launch_distance(q, 0);
     if (e != hipSuccess) return fail_hip(e, "distance kernel launch");
@@ -874,7 +888,6 @@ int cubvh_distance_ordered(cubvh_bvh* bvh, int device, int64_t n, int32_t kind, 
     q.out_f = distances;
     q.out_id = face_id;
     q.out_v = uvw;
-    q.packet = true;
     // allocates nothing, so its walks all run to their end (q.rest is null)
     hipError_t e = launch_distance(q, kind);
     if (e != hipSuccess) return fail_hip(e, "distance kernel launch");
@@ -886,6 +899,29 @@ int cubvh_signed_distance(cubvh_bvh* bvh, int device, int64_t n, uint32_t mode, 
                           float* distances, int64_t* face_id, float* uvw, void* stream) {
     // src/bvh.cu:440-465: mode 0 is watertight, every other value raystab
     return run_distance(bvh, device, n, mode == 0 ? 1 : 2, positions, distances, face_id, uvw, stream);
+}
+
+namespace {
+int set_control(WalkControl& c, const uint32_t& count, const int32_t* control, uint32_t* handed) {
+    if (handed) *handed = count;
+    if (!control) return CUBVH_OK;
+    if (control[0] < 0 || control[0] > 2) return fail(CUBVH_ERR_ARG, "route must be 0, 1 (waves) or 2 (packets)");
+    c.route = control[0];
+    c.cap = control[1];
+    c.first = control[2];
+    c.factor = control[3];
+    return CUBVH_OK;
+}
+}  // namespace
+
+int cubvh_bvh_walk_control(cubvh_bvh* bvh, const int32_t control[4], uint32_t* handed) {
+    if (!bvh) return fail(CUBVH_ERR_ARG, "bvh is null");
+    return set_control(bvh->control, bvh->handed, control, handed);
+}
+
+int cubvh_forest_walk_control(cubvh_forest* forest, const int32_t control[4], uint32_t* handed) {
+    if (!forest) return fail(CUBVH_ERR_ARG, "forest is null");
+    return set_control(forest->control, forest->handed, control, handed);
 }
 
 int cubvh_ray_trace(cubvh_bvh* bvh, int device, int64_t n, const float* rays_o, const float* rays_d,
@@ -908,14 +944,14 @@ int cubvh_ray_trace(cubvh_bvh* bvh, int device, int64_t n, const float* rays_o, 
     q.out_f = depth;
     // packets are walked in an order that keeps rays of close origins and directions
     // together (stream-ordered scratch, released after the launch)
-    q.packet = n >= kWaveMax;
+    q.walk = walk_of(q.control, n, ray_waves_pay(n));
     hipStream_t hs = (hipStream_t)stream;
     void* scratch = nullptr;
-    if (q.packet && n < ((int64_t)1 << 31)) {
+    if (q.walk == Walk::packets) {
         rc = ensure_pool(device);
         if (rc != CUBVH_OK) return rc;
         const size_t ob = ((size_t)n * 4 + 255) & ~(size_t)255;
-        const size_t rb = ray_rest_bytes(n, q.n_faces);
+        const size_t rb = ray_rest_bytes(n, q.n_faces, q.control);
         hipError_t e = hipMallocAsync(&scratch, ob + rb + morton_workspace_bytes(n), hs);
         if (e != hipSuccess) return fail_hip(e, "hipMallocAsync(ray order)");
         if (rb) q.rest = (char*)scratch + ob;
@@ -927,6 +963,7 @@ int cubvh_ray_trace(cubvh_bvh* bvh, int device, int64_t n, const float* rays_o, 
         q.order = (const uint32_t*)scratch;
     }
     hipError_t e = launch_ray(q);
+    if (e == hipSuccess) e = bvh->count_handed(q);
     if (scratch) {
         hipError_t e2 = hipFreeAsync(scratch, hs);
         if (e == hipSuccess) e = e2;
@@ -1257,6 +1294,7 @@ int cubvh_forest_unsigned_distance(cubvh_forest* forest, int device, int64_t n, 
     a.tree = c.tree.view;
     a.mesh_info = c.mesh_info;
     a.most_faces = forest->most_faces;
+    a.control = forest->control;
     a.persistent = persistent;
     a.waves_per_cu = wpc;
     a.waves_per_block = wpb;
@@ -1264,6 +1302,10 @@ int cubvh_forest_unsigned_distance(cubvh_forest* forest, int device, int64_t n, 
     a.n_cu = c.n_cu;
     e = launch_forest_distance(a, ws, hs);
     if (e != hipSuccess) return fail_hip(e, "forest kernel launch");
+    if (a.control.cap >= 0) {
+        e = rest_count(ws.rest, hs, &forest->handed);
+        if (e != hipSuccess) return fail_hip(e, "handed-over count");
+    }
     return CUBVH_OK;
     CUBVH_GUARD_END
 }

@@ -721,17 +721,21 @@ struct PacketRest {
     uint32_t factor;  // a walk ends after factor / 16 times the average walk's steps
     uint32_t tiles;   // sampled walks that have ended, and their steps
     unsigned long long steps;
-    uint32_t pad[58];  // the list follows: (query, best so far bits, its face slot, root)
+    uint32_t pad[26];
+    uint32_t first;   // steps before a walk may end early; every wave reads it, so not in the
+                      // line that the counters keep busy (2,000,000 points 855 us there, 710 here)
+    uint32_t pad2[31];  // the list follows: (query, best so far bits, its face slot, root)
     __host__ __device__ int4* list() const { return (int4*)(this + 1); }
 };
 static_assert(sizeof(PacketRest) == 256, "the list is 256-byte aligned");
 constexpr int32_t kFirstCheck = 512;  // steps before a walk is compared with the average
+constexpr int32_t kRaySteps = 2048;   // steps of a packet of rays; a lane's walk has a quarter of them
 
 // Steps at which a walk of `steps` steps ends, or is looked at again, from the walks that
 // have ended so far.
 __device__ __forceinline__ int32_t step_limit(const PacketRest* rest, int32_t steps) {
     const uint32_t n = __hip_atomic_load(&rest->tiles, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (n < 16) return steps + kFirstCheck / 4;  // too few to tell
+    if (n < 16) return steps + uniform((int32_t)(rest->first / 4));  // too few to tell
     const unsigned long long s = __hip_atomic_load(&rest->steps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return uniform((int32_t)min((s * rest->factor) / (16ull * n), (unsigned long long)INT32_MAX));
 }
@@ -744,12 +748,13 @@ __device__ __forceinline__ void report_steps(PacketRest* rest, int64_t tile, int
     }
 }
 
-__global__ void rest_init(PacketRest* rest, uint32_t cap, uint32_t factor) {
+__global__ void rest_init(PacketRest* rest, uint32_t cap, uint32_t factor, uint32_t first) {
     if (threadIdx.x == 0) {
         rest->count = rest->tiles = 0;
         rest->steps = 0;
         rest->cap = cap;
         rest->factor = factor;
+        rest->first = first;
     }
 }
 
@@ -794,7 +799,7 @@ __device__ uint64_t closest_face_packet(const Tree& T, int32_t root, f3 p, bool 
     int32_t qn = 0;  // queued pairs (wave-uniform)
     int32_t ref = uniform(root);
     uint64_t left = 0;
-    int32_t steps = 0, check = kFirstCheck;
+    int32_t steps = 0, check = REST ? uniform((int32_t)rest->first) : 0;
     for (;;) {
         ++steps;
         if (ref >= 0) {
@@ -975,7 +980,6 @@ __device__ __forceinline__ void run_exact_ray(const Tree& T, ExactQueue& q, int3
 // pairs; kRayStepLanes 16 .. 64 and kRayFlush 8 .. 48 within 2%.
 constexpr int kRayFlush = 32;
 constexpr int kRayStepLanes = 32;
-constexpr int32_t kRaySteps = 2000;
 __device__ __forceinline__ float slab_entry(float lx, float hx, float ly, float hy, float lz, float hz, f3 o, f3 inv) {
     const float tx0 = (lx - o.x) * inv.x, tx1 = (hx - o.x) * inv.x;
     const float ty0 = (ly - o.y) * inv.y, ty1 = (hy - o.y) * inv.y;
@@ -1001,7 +1005,7 @@ __device__ uint64_t closest_hit_packet(const Tree& T, f3 o, f3 d, bool active, f
     if (mask == 0) return 0;
     WaveStack st;
     int32_t ref = 0;
-    int32_t budget = kRaySteps;
+    int32_t budget = REST ? uniform((int32_t)rest->first) : 0;
     for (;;) {
         if (REST) --budget;
         if (ref >= 0) {
@@ -1675,7 +1679,6 @@ __global__ __launch_bounds__(64 * WAVES, PERSISTENT ? 7 : 8) void forest_distanc
 // of its first ray, origins within 1% of the scene's diagonal) walks as a packet;
 // any other wave walks lane by lane.  Both give closest_hit's results.
 constexpr int kRayLds = 8;
-constexpr int32_t kLaneSteps = 512;  // steps of a lane's walk before a wave takes over
 template <int WAVES, bool REST>
 __global__ __launch_bounds__(64 * WAVES, 8) void ray_packet_kernel(int64_t n, const float* __restrict__ rays_o,
                                                          const float* __restrict__ rays_d,
@@ -1730,7 +1733,7 @@ __global__ __launch_bounds__(64 * WAVES, 8) void ray_packet_kernel(int64_t n, co
         st.key = lds.lanes.key;
         st.tid = (int)threadIdx.x;
         left = 0;
-        for (int32_t budget = kLaneSteps;; budget = INT32_MAX) {
+        for (int32_t budget = REST ? (int32_t)(rest->first / 4) : 0;; budget = INT32_MAX) {
             int32_t b = valid ? budget : 0;
             if (valid) slot = closest_hit<REST>(T, o, d, st, t, b);
             if (REST) left = ballot(b < 0);
@@ -1789,26 +1792,27 @@ uint32_t rest_cap(int64_t n) { return (uint32_t)std::min<int64_t>(n, kRestMax); 
 // 1.33 with 3, 1.73 with 6, 3.06 without; 2^23 uniform points on 1.3 M faces: 9.0 ms with
 // slope 0.3, 9.9 with 0.6, 13.6 without).  The watertight sign needs more of a walk's wave:
 // 2^21 grid points on 327,680 faces 2.83 ms with 2, 2.40 with 3, 2.37 with 4, 2.58 with 6.
-void launch_rest_init(dev::PacketRest* rest, int64_t n, double least, hipStream_t s) {
+void launch_rest_init(dev::PacketRest* rest, int64_t n, double least, int32_t first, const WalkControl& c, hipStream_t s) {
     const double rounds = (double)n / (64.0 * kRestBlocks);
-    const uint32_t factor = (uint32_t)(16.0 * std::max(least, 0.4 * rounds));
-    hipLaunchKernelGGL(dev::rest_init, dim3(1), dim3(64), 0, s, rest, rest_cap(n), factor);
+    const uint32_t factor = c.factor >= 0 ? (uint32_t)c.factor : (uint32_t)(16.0 * std::max(least, 0.4 * rounds));
+    const uint32_t cap = c.cap >= 0 ? std::min((uint32_t)c.cap, rest_cap(n)) : rest_cap(n);
+    hipLaunchKernelGGL(dev::rest_init, dim3(1), dim3(64), 0, s, rest, cap, factor, (uint32_t)(c.first > 0 ? c.first : first));
 }
 
 hipError_t launch_distance_impl(const QueryArgs& q, int mode) {
     const dev::Tree T = dev::make_tree(q.tree, q.face0_slot);
     hipStream_t s = (hipStream_t)q.stream;
-    if (mode != 2 && q.n < kWaveMax && !q.order) {
+    if (mode != 2 && q.walk == Walk::waves) {
         hipLaunchKernelGGL((mode == 0 ? dev::distance_wave_kernel<0> : dev::distance_wave_kernel<1>), dim3((unsigned)q.n),
                            dim3(64), 0, s, q.in0, q.out_f, q.out_id, q.out_v, T);
         return hipGetLastError();
     }
-    if ((mode == 0 || mode == 1) && q.packet) {
+    if (mode != 2 && q.walk == Walk::packets) {
         constexpr int W = kDistanceWaves;
         const unsigned grid = (unsigned)((q.n + 64 * W - 1) / (64 * W));
         const uint32_t xchunk = xcd_chunk_for(grid);
         dev::PacketRest* rest = (dev::PacketRest*)q.rest;
-        if (rest) launch_rest_init(rest, q.n, mode == 0 ? 2.5 : 3.5, s);
+        if (rest) launch_rest_init(rest, q.n, mode == 0 ? 2.5 : 3.5, dev::kFirstCheck, q.control, s);
         const auto kernel = mode == 0 ? (rest ? dev::distance_packet_kernel<0, W, true> : dev::distance_packet_kernel<0, W, false>)
                                       : (rest ? dev::distance_packet_kernel<1, W, true> : dev::distance_packet_kernel<1, W, false>);
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), 0, s, q.n, q.in0, q.order, q.out_f, q.out_id, q.out_v, T, xchunk,
@@ -1850,8 +1854,8 @@ namespace {
 template <int WAVES>
 hipError_t launch_forest_shape(const ForestArgs& a, const ForestWorkspace& ws, hipStream_t s) {
     const int64_t max_tiles = ws.npad_max / 64;
-    dev::PacketRest* rest = hands_over(ws.npad_max, a.most_faces) ? (dev::PacketRest*)ws.rest : nullptr;
-    if (rest) launch_rest_init(rest, ws.npad_max, 2.5, s);
+    dev::PacketRest* rest = a.control.cap >= 0 || hands_over(ws.npad_max, a.most_faces) ? (dev::PacketRest*)ws.rest : nullptr;
+    if (rest) launch_rest_init(rest, ws.npad_max, 2.5, dev::kFirstCheck, a.control, s);
     const auto kernel = a.persistent ? (rest ? dev::forest_distance_kernel<1, WAVES, true> : dev::forest_distance_kernel<1, WAVES, false>)
                                      : (rest ? dev::forest_distance_kernel<0, WAVES, true> : dev::forest_distance_kernel<0, WAVES, false>);
     const unsigned blocks = a.persistent ? (unsigned)std::max(1, a.n_cu * a.waves_per_cu / WAVES)
@@ -1878,6 +1882,11 @@ hipError_t launch_forest_distance(const ForestArgs& a, const ForestWorkspace& ws
     }
 }
 
+hipError_t rest_count(const void* rest, hipStream_t s, uint32_t* count) {
+    hipError_t e = hipMemcpyAsync(count, rest, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
+    return e == hipSuccess ? hipStreamSynchronize(s) : e;
+}
+
 size_t rest_bytes(int64_t n) { return (sizeof(dev::PacketRest) + 16 * (size_t)rest_cap(n) + 255) & ~(size_t)255; }
 
 int stack_capacity_for(int need) { return need <= dev::STACK_TOTAL ? dev::STACK_TOTAL : -1; }
@@ -1897,7 +1906,7 @@ hipError_t launch_stab_sign(const QueryArgs& q, void* ws) {
     if (q.n <= 0) return hipSuccess;
     if (stack_capacity_for(q.stack_need) < 0) return hipErrorInvalidValue;
     // bit 31 marks list entries; the lane walks need the Morton order
-    if (!ws || q.n >= ((int64_t)1 << 31) || (q.n >= kWaveMax && !q.order)) return hipErrorInvalidValue;
+    if (!ws || q.n >= ((int64_t)1 << 31) || (q.walk != Walk::waves && !q.order)) return hipErrorInvalidValue;
     const dev::Tree T = dev::make_tree(q.tree, q.face0_slot);
     hipStream_t s = (hipStream_t)q.stream;
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
@@ -1921,7 +1930,7 @@ hipError_t launch_stab_sign(const QueryArgs& q, void* ws) {
     const unsigned first_grid = (unsigned)((q.n + SB - 1) / SB);
     for (int b = 0; b <= dev::kStabBatches; ++b) {
         uint32_t* list = lists[b == 0 ? 0 : (b - 1) & 1];
-        if (q.n < (b == 0 ? kWaveMax : kStabWaveMax))
+        if (b == 0 ? q.walk == Walk::waves : q.n < kStabWaveMax)
             hipLaunchKernelGGL(dev::stab_wave, dim3((unsigned)std::min<int64_t>(q.n * (b == 0 ? 1 : 20), kStabWaveBlocks)),
                                dim3(64), 0, s, (uint32_t)b, list, counts, q.in0, offs, T);
         else if (b == 0)
@@ -1951,14 +1960,14 @@ hipError_t launch_ray(const QueryArgs& q) {
     if (q.n <= 0) return hipSuccess;
     if (stack_capacity_for(q.stack_need) < 0) return hipErrorInvalidValue;
     const dev::Tree T = dev::make_tree(q.tree, q.face0_slot);
-    if (q.packet) {
+    if (q.walk != Walk::waves) {  // packets, and any number of rays in the caller's order
         constexpr int W = kDistanceWaves;  // one wave per workgroup, as the distance kernels (3119 vs 2899 Mrays/s with 4)
         // no runs per XCD here: ray costs differ between image regions, and runs put the
         // costly ones on one XCD (camera rays 2475 Mrays/s with the distance kernels' runs)
         const unsigned grid = (unsigned)((q.n + 64 * W - 1) / (64 * W));
         hipStream_t s = (hipStream_t)q.stream;
         dev::PacketRest* rest = (dev::PacketRest*)q.rest;
-        if (rest) launch_rest_init(rest, q.n, 1.0, s);
+        if (rest) launch_rest_init(rest, q.n, 1.0, dev::kRaySteps, q.control, s);
         hipLaunchKernelGGL((rest ? dev::ray_packet_kernel<W, true> : dev::ray_packet_kernel<W, false>), dim3(grid), dim3(64 * W), 0, s, q.n, q.in0, q.in1, q.order, q.out_v,
                            q.out_id, q.out_f, T, rest);
         if (rest)

@@ -18,6 +18,19 @@ struct TreeArrays {
     const float4* tpre = nullptr;  // per-face constants of the distance formula
 };
 
+// How a call walks: lanes one query each, waves one query each in the caller's order, or
+// packets of 64 queries, ordered first.
+enum class Walk { lanes, waves, packets };
+
+// Overrides for tests and measurements, per tree or forest (cubvh_bvh_walk_control).
+struct WalkControl {
+    int32_t route = 0;  // 1 waves, 2 packets, 0 by the rules below
+    int32_t cap = -1;   // places of the hand-over's list; -1 by the rules, which may mean none
+    int32_t first = 0;  // steps of a walk before it may be handed over; 0: the default
+    int32_t factor = -1;  // sixteenths of the average walk's steps; -1: the default
+    bool active() const { return route != 0 || cap >= 0 || first > 0 || factor >= 0; }
+};
+
 struct QueryArgs {
     int64_t n = 0;
     const float* in0 = nullptr;  // positions or ray origins [n,3]
@@ -31,19 +44,41 @@ struct QueryArgs {
     int64_t face0_slot = 0;
     int64_t n_faces = 0;
     int32_t stack_need = 0;
-    bool packet = true;  // walk as wave packets (queries in Morton order)
+    Walk walk = Walk::packets;
+    WalkControl control;
     void* rest = nullptr;  // packets: rest_bytes(n) bytes for the queries of given-up walks, or null: none is
     void* stream = nullptr;
 };
 
-// Distance calls and ray calls of fewer queries walk one wave per query in the caller's
-// order; larger ones are ordered first and walk as packets of 64.  A wave per query costs
-// 2.1 us per 1,000 points on 5,120 faces and 6 us on 1.3 M; packets share each fetch, but
-// one call lasts at least as long as its slowest tile.  Measured, waves against packets, at
-// 100,000 points: 234 / 484 us (5,120 faces), 407 / 3,845 (81,920, jittered), 618 / 10,074
-// (1.3 M); at 300,000: 639 / 527, 1,111 / 3,624, 1,770 / 7,501.  Scattered rays at 300,000:
-// 309 / 348, 389 / 453, 456 / 892; camera rays at 262,144: 157 / 494, 410 / 1,768.
+// Small calls walk one wave per query in the caller's order, larger ones are ordered first
+// and walk as packets of 64: a packet shares each fetch and test among its queries, but the
+// ordering takes 60 to 120 us and a call lasts as long as its slowest tile, the more faces the
+// longer.  Where both take the same time, in thousands of queries (points uniform, near the
+// surface, normal, on a grid; smooth, jittered and soup meshes):
+//   faces                    20   320  1,280  5,120  20,480  81,920  327,680  1.3 M
+//   unsigned, raystab    95-340   120    130    170     190     220  240-300  360-500
+//   watertight              150    90    105    140     170     190  200-300  330-450
+//   rays, scattered         680   400    390    410     570     520      900    950
+//   rays, camera            800   520    510    500     520     600      880   1,200
+// 250,000 points near 320 faces, packets and waves: 208 / 387 us, 5,120 faces 273 / 511;
+// below 2^18 rays waves always win.
 constexpr int64_t kWaveMax = (int64_t)1 << 18;
+inline bool waves_pay(int64_t n, int64_t n_faces, int mode) {  // mode as launch_distance's
+    if (n_faces >= (int64_t)1 << 18) return n < kWaveMax;
+    int64_t most = n_faces < 4096 ? (int64_t)1 << 17 : (int64_t)3 << 16;
+    if (n_faces < 64 && mode != 2) most = kWaveMax;  // one node: a wave's round tests most of the mesh
+    if (n_faces >= (int64_t)1 << 16 && mode == 2) most = kWaveMax;  // 76,377 loose faces: 250,000 points 1.35 ms by waves, 1.52 else
+    if (mode == 1) most -= most / 4;                 // a packet's lanes search their normals at once
+    return n < most;
+}
+inline bool ray_waves_pay(int64_t n) { return n < kWaveMax; }
+// Never more waves than this: a launch has fewer than 2^32 threads.
+constexpr int64_t kWaveMost = (int64_t)1 << 24;
+inline Walk walk_of(const WalkControl& c, int64_t n, bool waves) {
+    if (n >= (int64_t)1 << 31) return Walk::lanes;
+    if (c.route == 1 && n < kWaveMost) return Walk::waves;
+    return c.route == 2 || !waves ? Walk::packets : Walk::waves;
+}
 
 // Stack capacity instantiated for a tree that needs `need` entries (-1 if none).
 int stack_capacity_for(int need);
@@ -72,10 +107,14 @@ inline bool hands_over(int64_t n, int64_t n_faces) {
     return n >= kRestFirst && n < kRestLast && n_faces >= kRestFaces && n / kRestQueries < n_faces;
 }
 size_t rest_bytes(int64_t n);
-inline size_t rest_bytes(int64_t n, int64_t n_faces) { return hands_over(n, n_faces) ? rest_bytes(n) : 0; }
-inline size_t ray_rest_bytes(int64_t n, int64_t n_faces) {
-    return n < kRayRestLast && n_faces >= kRayRestFaces ? rest_bytes(n) : 0;
+inline size_t rest_bytes(int64_t n, int64_t n_faces, const WalkControl& c) {
+    return c.cap >= 0 || hands_over(n, n_faces) ? rest_bytes(n) : 0;
 }
+inline size_t ray_rest_bytes(int64_t n, int64_t n_faces, const WalkControl& c) {
+    return c.cap >= 0 || (n < kRayRestLast && n_faces >= kRayRestFaces) ? rest_bytes(n) : 0;
+}
+// Queries handed over by the walks of a launch with this list so far (synchronizes).
+hipError_t rest_count(const void* rest, hipStream_t s, uint32_t* count);
 
 // Packets seed their walks (query.hip) while a face has fewer queries than this: with more,
 // a walk finds its first face at once.  Seeded against not: 320 faces 263,000 points 180 / 201
@@ -87,7 +126,7 @@ constexpr int64_t kSeedQueries = 1 << 10;
 hipError_t launch_distance(const QueryArgs& q, int mode);
 hipError_t launch_ray(const QueryArgs& q);
 // Negates q.out_f[i] of every query whose 64 raystab rays all hit (distances from mode 0),
-// walking the queries of q.order (required from kWaveMax on, n < 2^31) in passes over the undecided ones;
+// walking the queries of q.order (required by packets, n < 2^31) in passes over the undecided ones;
 // ws holds stab_workspace_bytes(q.n) bytes.
 size_t stab_workspace_bytes(int64_t n);
 hipError_t launch_stab_sign(const QueryArgs& q, void* ws);

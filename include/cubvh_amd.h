@@ -168,6 +168,16 @@ int cubvh_distance_ordered(cubvh_bvh* bvh, int device, int64_t n, int32_t kind, 
 int cubvh_ray_trace(cubvh_bvh* bvh, int device, int64_t n, const float* rays_o, const float* rays_d,
                     float* positions, int64_t* face_id, float* depth, void* stream);
 
+/* For tests and measurements (no counterpart in the reference): overrides of how a tree's
+ * or a forest's queries walk, kept until the next call; results are the same whatever is
+ * set.  control: [0] route: 0 by the library's rules, 1 a wave per query, 2 packets;
+ * [1] places of the list that long packet walks hand queries over to, -1 by the rules;
+ * [2] steps of a walk before it may be handed over and [3] sixteenths of the average walk's
+ * steps after which it is, 0 and -1 for the defaults.  NULL changes nothing.  handed (or
+ * NULL) receives the number of queries that the last call under a control handed over;
+ * such calls synchronize.  Not to be changed while queries run. */
+int cubvh_bvh_walk_control(cubvh_bvh* bvh, const int32_t control[4], uint32_t* handed);
+
 /* Replaces floodfill (src/api_gpu.cu:136-152, _floodfill_batch
  * include/gpu/floodfill.cuh:157-272).  grid: uint8/bool [B,H,W,D] (nonzero =
  * occupied); labels int32 [B,H,W,D]: -1 for occupied voxels, otherwise the minimum
@@ -262,6 +272,9 @@ int cubvh_forest_reserve(cubvh_forest* forest, int device, int64_t max_queries, 
 int cubvh_forest_unsigned_distance(cubvh_forest* forest, int device, int64_t n, const float* positions,
                                    const int64_t* query_offsets, float* distances, int64_t* face_id, float* uvw,
                                    const int32_t* tuning, int32_t n_tuning, void* stream);
+
+/* As cubvh_bvh_walk_control. */
+int cubvh_forest_walk_control(cubvh_forest* forest, const int32_t control[4], uint32_t* handed);
 
 /* ---------------------------------------------------------------------------
  * Sparse-voxel hash table: a static open-addressed table of int32 keys of D words

@@ -1,5 +1,6 @@
 """Packet walks (64 queries or rays a wave) where they can go wrong, held to the wave walks
 and to the oracle."""
+import contextlib
 import ctypes
 import math
 
@@ -8,6 +9,7 @@ import pytest
 import torch
 
 import cubvh_amd
+from cubvh_amd import synthetic as S
 from test_ray_line_host import check, rim_rays, thin_faces  # noqa: F401 (a fixture)
 
 pytestmark = pytest.mark.gpu
@@ -93,3 +95,45 @@ def test_ordered_calls_leave_skipped_queries_alone(gpu):
     kept[skipped] = False
     assert bool((d[skipped] == 3.0).all()) and bool((f[skipped] == -12345).all())
     same_bits([d[kept], f[kept]], [ref[0][kept], ref[1][kept]])
+
+
+@contextlib.contextmanager
+def walks(handle, route=0, cap=-1, first=0, factor=-1):
+    """The tree's (or forest's) queries walk as told; yields a function that says how many
+    queries the last call handed over."""
+    lib = cubvh_amd._lib.load()
+    fn = lib.cubvh_forest_walk_control if isinstance(handle, cubvh_amd.cuBVHForest) else lib.cubvh_bvh_walk_control
+
+    def control(*values):
+        cubvh_amd._lib.check(fn(handle._h, (ctypes.c_int32 * 4)(*values), None))
+
+    def handed():
+        count = ctypes.c_uint32(0)
+        cubvh_amd._lib.check(fn(handle._h, None, ctypes.byref(count)))
+        return count.value
+
+    control(route, cap, first, factor)
+    try:
+        yield handed
+    finally:
+        control(0, -1, 0, -1)
+
+
+@pytest.mark.parametrize("level", [0, 2, 4, 6])
+def test_routes_agree_around_their_limits(gpu, level):
+    """Calls just below and above the sizes where the route changes: the same bits from the
+    route taken and from the other one."""
+    v, f = S.icosphere(level, 0.5)
+    bvh = cubvh_amd.cuBVH(v, f)
+    for n in (98_303, 98_304, 131_072, 147_456, 196_607, 196_608, 262_144):
+        p = torch.from_numpy(S.uniform_points(n, seed=n)).to(gpu)
+        o, d = (torch.from_numpy(x).to(gpu) for x in S.sphere_rays(n, seed=n))
+        calls = [lambda: bvh.unsigned_distance(p, return_uvw=True), lambda: bvh.signed_distance(p)[:2],
+                 lambda: bvh.ray_trace(o, d)]
+        if n in (131_072, 196_607):
+            calls.append(lambda: bvh.signed_distance(p, mode="raystab")[:2])
+        for call in calls:
+            out = call()
+            for route in (1, 2):
+                with walks(bvh, route):
+                    same_bits(out, call())
