@@ -7,7 +7,8 @@
 //
 //   1. tiles  : each workgroup labels one tile of 64 x 8 x 8 voxels (64 along the last
 //               axis: one row per wave, a lane per voxel, so that occupancy is one ballot,
-//               loads and stores are whole lines, and runs are bit arithmetic).
+//               loads and stores are whole lines, and runs are bit arithmetic), or of
+//               16 x 16 x 16, four rows per wave, where the last axis has at most 16.
 //               Union-find in LDS between overlapping runs of neighbouring rows; every
 //               free voxel gets the global index of its tile-local root, others -1.
 //   2. merge  : voxels on a tile's low faces union themselves with their free
@@ -25,6 +26,8 @@
 // lanes) and for flatten by its 134 MB.  With tiles of 16^3 loaded a byte per lane, a
 // union per row of every face and a root search per voxel these were 118, 287 and 54 us.
 // A third of the voxels occupied at random: 760 -> 187 us; 64^3: 78 -> 38 us.
+// Axes of one voxel do not matter to the labels: a last axis of 1 is dropped, so that the
+// next one takes its place.
 //
 // The result equals the reference's converged output (the minimum linear index of
 // each free component, -1 for occupied voxels, indices global across the batch)
@@ -32,6 +35,8 @@
 // shape; the reference decodes coordinates as if H == W == D.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "query.hpp"
 
@@ -80,11 +85,29 @@ __device__ __forceinline__ void unite(int32_t* L, int32_t a, int32_t b) {
     }
 }
 
-constexpr int TD = 64, TW = 8, TH = 8;  // tile edges along the last, middle and first axis
-constexpr int TILE_ROWS = TW * TH;
+// A tile has TD x TW x TH voxels along the last, middle and first axis; 64 / TD rows along the
+// last axis share a wave pass.
 constexpr int TILE_WAVES = 4;
-constexpr int WAVE_ROWS = TILE_ROWS / TILE_WAVES;
-static_assert(TH == TILE_ROWS / TW && 2 * (2 * TILE_ROWS - TW - TH) <= 64 * TILE_WAVES, "threads of the row pairs");
+constexpr int TILE_PASSES = 64;  // 4,096 voxels
+constexpr int WAVE_PASSES = TILE_PASSES / TILE_WAVES;
+template <int TD>
+struct Tile {
+    static_assert(TD == 64 || TD == 16, "cubic but for the order of the lanes");
+    static constexpr int TW = TD == 64 ? 8 : 16, TH = TW;
+    static constexpr int ROWS = TW * TH, PER_PASS = 64 / TD;  // rows, and those of a pass
+    static constexpr uint64_t ROW = TD == 64 ? ~0ull : (1ull << (TD & 63)) - 1ull;
+    static constexpr int HALVES = TD == 64 ? 2 : 1;  // threads for a pair of neighbouring rows
+    static_assert(ROWS * TD == 64 * TILE_PASSES, "a lane per voxel");
+    int32_t d0, w0, h0, base;  // the tile's first voxel; of its grid (the whole has fewer than 2^31)
+    __device__ __forceinline__ Tile(uint32_t tile, int32_t H, int32_t W, int32_t D) {
+        const uint32_t nd = (D + TD - 1) / TD, nw = (W + TW - 1) / TW, nh = (H + TH - 1) / TH;
+        d0 = (int32_t)(tile % nd) * TD;
+        w0 = (int32_t)((tile / nd) % nw) * TW;
+        const uint32_t rest = tile / (nd * nw);
+        h0 = (int32_t)(rest % nh) * TH;
+        base = (int32_t)(rest / nh) * H * W * D;
+    }
+};
 
 __device__ __forceinline__ int32_t lds_parent(const int32_t* L, int32_t x) {
     return __hip_atomic_load(L + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -117,79 +140,81 @@ __device__ __forceinline__ int run_start(uint64_t free, int lane) {
     return gaps ? 64 - __builtin_clzll(gaps) : 0;
 }
 
-// One workgroup per tile; tiles numbered along the last axis fastest, then w, h, b.  Voxel
-// `lane` of row r (w = r % TW, h = r / TW) has the local index 64 r + lane, which orders
-// voxels like the tile's linear index; only the first voxel of a run is a union-find node.
+// One workgroup per tile (from tile `first` on); tiles numbered along the last axis fastest,
+// then w, h, b.  Voxel c of row r (w = r % TW, h = r / TW) has the local index TD r + c, which
+// orders voxels like the tile's linear index; only the first voxel of a run is a union-find
+// node.
+template <int TD>
 __global__ __launch_bounds__(64 * TILE_WAVES) void ff_tiles(const uint8_t* __restrict__ grid, int32_t* __restrict__ out,
-                                                            int32_t H, int32_t W, int32_t D) {
-    __shared__ int32_t L[64 * TILE_ROWS];
-    __shared__ uint64_t rows[TILE_ROWS];
-    const int32_t nd = (D + TD - 1) / TD, nw = (W + TW - 1) / TW, nh = (H + TH - 1) / TH;
-    const uint32_t tile = blockIdx.x;
-    const int32_t d0 = (int32_t)(tile % nd) * TD;
-    const int32_t w0 = (int32_t)((tile / nd) % nw) * TW;
-    const uint32_t rest = tile / ((uint32_t)nd * nw);
-    const int32_t h0 = (int32_t)(rest % nh) * TH;
-    const int32_t base = (int32_t)(rest / nh) * H * W * D;  // the whole grid has fewer than 2^31 voxels
-    const int lane = (int)threadIdx.x & 63, r0 = ((int)threadIdx.x >> 6) * WAVE_ROWS;
-    const int32_t d = d0 + lane;
-    uint8_t occ[WAVE_ROWS];
+                                                            uint32_t first, int32_t H, int32_t W, int32_t D) {
+    using T = Tile<TD>;
+    constexpr int TW = T::TW, TH = T::TH;
+    __shared__ int32_t L[64 * TILE_PASSES];
+    __shared__ uint64_t rows[TILE_PASSES];
+    const T t(first + blockIdx.x, H, W, D);
+    const int lane = (int)threadIdx.x & 63, p0 = ((int)threadIdx.x >> 6) * WAVE_PASSES, c = lane % TD;
+    const int32_t d = t.d0 + c;
+    uint8_t occ[WAVE_PASSES];
 #pragma unroll
-    for (int k = 0; k < WAVE_ROWS; ++k) {
-        const int r = r0 + k, h = h0 + r / TW, w = w0 + r % TW;
+    for (int k = 0; k < WAVE_PASSES; ++k) {
+        const int r = (p0 + k) * T::PER_PASS + lane / TD, h = t.h0 + r / TW, w = t.w0 + r % TW;
         occ[k] = 1;  // outside the grid counts as occupied
-        if (h < H && w < W && d < D) occ[k] = grid[base + (h * W + w) * D + d];
+        if (h < H && w < W && d < D) occ[k] = grid[t.base + (h * W + w) * D + d];
     }
-    uint64_t free[WAVE_ROWS];
+    uint64_t free[WAVE_PASSES];
 #pragma unroll
-    for (int k = 0; k < WAVE_ROWS; ++k) {
+    for (int k = 0; k < WAVE_PASSES; ++k) {
         free[k] = __builtin_amdgcn_ballot_w64(occ[k] == 0);
-        rows[r0 + k] = free[k];  // every lane the same value
-        L[64 * (r0 + k) + lane] = 64 * (r0 + k) + lane;
+        rows[p0 + k] = free[k];  // every lane the same value
+        L[64 * (p0 + k) + lane] = 64 * (p0 + k) + lane;
     }
     __syncthreads();
-    // two threads (one per half of the row) for each pair of neighbouring rows: two runs meet
-    // in one contiguous segment, united at its first voxel
-    const int pr = (int)threadIdx.x >> 1;
-    if (pr < 2 * TILE_ROWS - TW - TH) {
-        const bool along_w = pr < TILE_ROWS - TH;
-        const int r = along_w ? pr / (TW - 1) * TW + pr % (TW - 1) + 1 : pr - (TILE_ROWS - TH) + TW;
+    auto row = [&](int r) { return (rows[r / T::PER_PASS] >> (TD * (r % T::PER_PASS))) & T::ROW; };
+    // a thread (two, one per half of the row, where rows are long) for each pair of neighbouring
+    // rows: two runs meet in one contiguous segment, united at its first voxel
+    for (int pt = (int)threadIdx.x; pt < T::HALVES * (2 * T::ROWS - TW - TH); pt += 64 * TILE_WAVES) {
+        const int pr = pt / T::HALVES;
+        const bool along_w = pr < T::ROWS - TH;
+        const int r = along_w ? pr / (TW - 1) * TW + pr % (TW - 1) + 1 : pr - (T::ROWS - TH) + TW;
         const int o = along_w ? r - 1 : r - TW;  // the row at w - 1, or at h - 1
-        const uint64_t mine = rows[r], other = rows[o], both = mine & other;
-        uint64_t segments = both & ~(both << 1) & (0xffffffffull << (32 * (threadIdx.x & 1)));
+        const uint64_t mine = row(r), other = row(o), both = mine & other;
+        uint64_t segments = both & ~(both << 1);
+        if (T::HALVES == 2) segments &= 0xffffffffull << (32 * (pt & 1));
         for (; segments != 0; segments &= segments - 1) {
             const int l = __builtin_ctzll(segments);
-            lds_unite(L, 64 * r + run_start(mine, l), 64 * o + run_start(other, l));
+            lds_unite(L, TD * r + run_start(mine, l), TD * o + run_start(other, l));
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < WAVE_ROWS; ++k) {
-        const int r = r0 + k, h = h0 + r / TW, w = w0 + r % TW;
+    for (int k = 0; k < WAVE_PASSES; ++k) {
+        const int r = (p0 + k) * T::PER_PASS + lane / TD, h = t.h0 + r / TW, w = t.w0 + r % TW;
         if (h >= H || w >= W || d >= D) continue;
         int32_t lab = -1;
         if ((free[k] >> lane) & 1) {
-            const int32_t root = lds_root(L, 64 * r + run_start(free[k], lane)), rr = root >> 6;
-            lab = base + ((h0 + rr / TW) * W + (w0 + rr % TW)) * D + d0 + (root & 63);
+            const uint64_t mine = (free[k] >> (TD == 64 ? 0 : lane - c)) & T::ROW;
+            const int32_t root = lds_root(L, TD * r + run_start(mine, c)), rr = root / TD;
+            lab = t.base + ((t.h0 + rr / TW) * W + (t.w0 + rr % TW)) * D + t.d0 + root % TD;
         }
-        out[base + (h * W + w) * D + d] = lab;
+        out[t.base + (h * W + w) * D + d] = lab;
     }
 }
 
 // Unions across the tile faces: the voxels on a tile's low faces with their neighbour one
-// step back, one wave per face normal to the middle or the first axis (8 rows of 64 pairs),
+// step back, one wave per face normal to the middle or the first axis (8 passes of 64 pairs,
+// or 4 of 4 rows),
 // and per 512 pairs of the faces normal to the last axis.  Pairs with the same two labels
 // are the same union: a pair that repeats the one before it in its lane is dropped, the
 // others leave their number in a small table, and one that finds another pair's number
 // there with the same labels is done (a pair whose entry was taken by different labels is
 // united as often as it occurs).  A wave per face and not a workgroup: the unions are
 // chains of dependent loads by a few lanes, so what counts is the faces in flight.
-constexpr int MERGE_ROWS = 8;
 constexpr uint32_t MERGE_SLOTS = 1024;
-static_assert(MERGE_ROWS == TW && MERGE_ROWS == TH && TD == 64, "one wave per face");
-
+template <int TD>
 __global__ __launch_bounds__(64) void ff_merge(int32_t* L, int32_t B, int32_t H, int32_t W, int32_t D, uint32_t b0,
                                                uint32_t b1) {
+    using T = Tile<TD>;
+    constexpr int TW = T::TW, TH = T::TH, MERGE_ROWS = TW / T::PER_PASS;  // one wave per face
     __shared__ int32_t low[64 * MERGE_ROWS], high[64 * MERGE_ROWS];
     __shared__ uint16_t owner[MERGE_SLOTS];
     const int t = (int)threadIdx.x;
@@ -210,13 +235,13 @@ __global__ __launch_bounds__(64) void ff_merge(int32_t* L, int32_t B, int32_t H,
     } else {
         const bool middle = blockIdx.x < b0 + b1;
         const uint32_t k = blockIdx.x - b0 - (middle ? 0 : b1), q = k / nd;
-        const int32_t d = (int32_t)(k % nd) * TD + t;
+        const int32_t d = (int32_t)(k % nd) * TD + t % TD;
         const uint32_t cw = middle ? nw - 1 : nw, ch = middle ? nh : nh - 1;  // faces along w and h
         const int32_t w0 = (int32_t)(q % cw + (middle ? 1 : 0)) * TW, h0 = (int32_t)(q / cw % ch + (middle ? 0 : 1)) * TH;
         const int32_t b = (int32_t)(q / cw / ch), step = middle ? D : D * W;
 #pragma unroll
         for (int r = 0; r < MERGE_ROWS; ++r) {
-            const int32_t w = middle ? w0 : w0 + r, h = middle ? h0 + r : h0;
+            const int32_t o = r * T::PER_PASS + t / TD, w = middle ? w0 : w0 + o, h = middle ? h0 + o : h0;
             if (d >= D || w >= W || h >= H) continue;
             const int32_t i = ((b * H + h) * W + w) * D + d;
             li[r] = L[i];
@@ -246,27 +271,24 @@ __global__ __launch_bounds__(64) void ff_merge(int32_t* L, int32_t B, int32_t H,
 // label[i] = root(i), a workgroup per tile.  A tile's voxels have few distinct labels (its
 // local roots), whose roots are kept in a table: most voxels find theirs there.
 constexpr uint32_t FLAT_SLOTS = 512;
-__global__ __launch_bounds__(64 * TILE_WAVES) void ff_flatten(int32_t* L, int32_t H, int32_t W, int32_t D) {
+template <int TD>
+__global__ __launch_bounds__(64 * TILE_WAVES) void ff_flatten(int32_t* L, uint32_t first, int32_t H, int32_t W, int32_t D) {
+    using T = Tile<TD>;
     __shared__ unsigned long long known[FLAT_SLOTS];  // (label, root)
-    const int32_t nd = (D + TD - 1) / TD, nw = (W + TW - 1) / TW, nh = (H + TH - 1) / TH;
-    const uint32_t tile = blockIdx.x;
-    const int32_t d = (int32_t)(tile % nd) * TD + ((int)threadIdx.x & 63);
-    const int32_t w0 = (int32_t)((tile / nd) % nw) * TW;
-    const uint32_t rest = tile / ((uint32_t)nd * nw);
-    const int32_t h0 = (int32_t)(rest % nh) * TH;
-    const int32_t base = (int32_t)(rest / nh) * H * W * D;
-    const int r0 = ((int)threadIdx.x >> 6) * WAVE_ROWS;
+    const T t(first + blockIdx.x, H, W, D);
+    const int lane = (int)threadIdx.x & 63, p0 = ((int)threadIdx.x >> 6) * WAVE_PASSES;
+    const int32_t d = t.d0 + lane % TD;
     for (int k = (int)threadIdx.x; k < (int)FLAT_SLOTS; k += 64 * TILE_WAVES) known[k] = ~0ull;
-    int32_t lab[WAVE_ROWS];
+    int32_t lab[WAVE_PASSES];
 #pragma unroll
-    for (int k = 0; k < WAVE_ROWS; ++k) {
-        const int r = r0 + k, h = h0 + r / TW, w = w0 + r % TW;
+    for (int k = 0; k < WAVE_PASSES; ++k) {
+        const int r = (p0 + k) * T::PER_PASS + lane / TD, h = t.h0 + r / T::TW, w = t.w0 + r % T::TW;
         lab[k] = -1;
-        if (h < H && w < W && d < D) lab[k] = L[base + (h * W + w) * D + d];
+        if (h < H && w < W && d < D) lab[k] = L[t.base + (h * W + w) * D + d];
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < WAVE_ROWS; ++k) {
+    for (int k = 0; k < WAVE_PASSES; ++k) {
         if (lab[k] < 0) continue;  // occupied, or outside the grid
         unsigned long long* at = known + (((uint32_t)lab[k] * 0x9e3779b1u) >> 23);
         const unsigned long long e = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -276,31 +298,51 @@ __global__ __launch_bounds__(64 * TILE_WAVES) void ff_flatten(int32_t* L, int32_
             __hip_atomic_store(at, ((unsigned long long)(uint32_t)lab[k] << 32) | (uint32_t)root, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_WORKGROUP);
         }
-        const int r = r0 + k, h = h0 + r / TW, w = w0 + r % TW;
-        if (root != lab[k]) L[base + (h * W + w) * D + d] = root;
+        const int r = (p0 + k) * T::PER_PASS + lane / TD, h = t.h0 + r / T::TW, w = t.w0 + r % T::TW;
+        if (root != lab[k]) L[t.base + (h * W + w) * D + d] = root;
     }
 }
 
 }  // namespace dev
 
-hipError_t launch_floodfill(const uint8_t* grid, int32_t B, int32_t H, int32_t W, int32_t D, int32_t* labels,
-                            hipStream_t stream) {
-    const int64_t ntot64 = (int64_t)B * H * W * D;
-    if (ntot64 <= 0) return hipSuccess;
-    const int64_t n_tiles = (int64_t)B * ((H + dev::TH - 1) / dev::TH) * ((W + dev::TW - 1) / dev::TW) *
-                            ((D + dev::TD - 1) / dev::TD);
-    hipLaunchKernelGGL(dev::ff_tiles, dim3((unsigned)n_tiles), dim3(64 * dev::TILE_WAVES), 0, stream, grid, labels, H, W,
-                       D);
-    // waves of the faces normal to the last, the middle and the first axis
-    const int64_t nd = (D + dev::TD - 1) / dev::TD, nw = (W + dev::TW - 1) / dev::TW, nh = (H + dev::TH - 1) / dev::TH;
-    const uint32_t b0 = (uint32_t)(((int64_t)B * (nd - 1) * W * H + 64 * dev::MERGE_ROWS - 1) /
-                                   (64 * dev::MERGE_ROWS));
+namespace {
+
+// A launch has fewer than 2^32 threads: tiles in runs of 2^23 workgroups.
+constexpr int64_t kTileRun = (int64_t)1 << 23;
+
+template <int TD>
+hipError_t launch_tiles(const uint8_t* grid, int32_t B, int32_t H, int32_t W, int32_t D, int32_t* labels, hipStream_t stream) {
+    using T = dev::Tile<TD>;
+    const int64_t nd = (D + TD - 1) / TD, nw = (W + T::TW - 1) / T::TW, nh = (H + T::TH - 1) / T::TH;
+    const int64_t n_tiles = B * nh * nw * nd;
+    for (int64_t at = 0; at < n_tiles; at += kTileRun)
+        hipLaunchKernelGGL(dev::ff_tiles<TD>, dim3((unsigned)std::min(n_tiles - at, kTileRun)), dim3(64 * dev::TILE_WAVES), 0,
+                           stream, grid, labels, (uint32_t)at, H, W, D);
+    // waves of the faces normal to the last, the middle and the first axis: at most an eighth of
+    // the voxels each, a wave to 64 of the first and 16 or more of the others
+    constexpr int64_t pairs = 64 * T::TW / T::PER_PASS;
+    const uint32_t b0 = (uint32_t)((B * (nd - 1) * W * H + pairs - 1) / pairs);
     const uint32_t b1 = (uint32_t)(B * nh * (nw - 1) * nd), b2 = (uint32_t)(B * (nh - 1) * nw * nd);
     if (b0 + b1 + b2 > 0) {  // labels of one tile are final already
-        hipLaunchKernelGGL(dev::ff_merge, dim3(b0 + b1 + b2), dim3(64), 0, stream, labels, B, H, W, D, b0, b1);
-        hipLaunchKernelGGL(dev::ff_flatten, dim3((unsigned)n_tiles), dim3(64 * dev::TILE_WAVES), 0, stream, labels, H, W, D);
+        hipLaunchKernelGGL(dev::ff_merge<TD>, dim3(b0 + b1 + b2), dim3(64), 0, stream, labels, B, H, W, D, b0, b1);
+        for (int64_t at = 0; at < n_tiles; at += kTileRun)
+            hipLaunchKernelGGL(dev::ff_flatten<TD>, dim3((unsigned)std::min(n_tiles - at, kTileRun)), dim3(64 * dev::TILE_WAVES),
+                               0, stream, labels, (uint32_t)at, H, W, D);
     }
     return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_floodfill(const uint8_t* grid, int32_t B, int32_t H, int32_t W, int32_t D, int32_t* labels,
+                            hipStream_t stream) {
+    if ((int64_t)B * H * W * D <= 0) return hipSuccess;
+    for (int k = 0; k < 2 && D == 1; ++k) {
+        D = W;
+        W = H;
+        H = 1;
+    }
+    return D <= 16 ? launch_tiles<16>(grid, B, H, W, D, labels, stream) : launch_tiles<64>(grid, B, H, W, D, labels, stream);
 }
 
 }  // namespace cubvh_amd

@@ -78,3 +78,26 @@ def test_floodfill_across_tiles(gpu, oracle, shape, kind):
         g[:, ::2, 3::4, 0] = False
     lab = cubvh_amd.floodfill(torch.from_numpy(g).to(gpu)).cpu().numpy()
     np.testing.assert_array_equal(lab, oracle.floodfill_bfs(g))
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (5, 1, 1, 1), (1, 1, 1, 70), (1, 1, 70, 1), (3, 70, 1, 1), (2, 33, 50, 1), (1, 1, 17, 9),
+                                   (1, 40, 1, 12), (1, 16, 16, 16), (2, 17, 33, 2), (1, 50, 35, 16), (1, 50, 35, 17),
+                                   (3, 9, 70, 7), (1, 100, 90, 1), (70, 4, 4, 4)])
+@pytest.mark.parametrize("free", [0.4, 0.65, 0.9, 1.0])
+def test_floodfill_short_axes(gpu, oracle, shape, free):
+    """A short last axis (tiles of 16 x 16 x 16), around their sizes, and axes of one voxel."""
+    g = np.random.default_rng(sum(shape)).random(shape) >= free
+    lab = cubvh_amd.floodfill(torch.from_numpy(g).to(gpu)).cpu().numpy()
+    np.testing.assert_array_equal(lab, oracle.floodfill_bfs(g))
+
+
+def test_floodfill_flat_grid_of_more_than_2_30_voxels(gpu):
+    """2^15 x (2^15 + 8) x 1: more tiles than one launch takes if tiles are laid along the last
+    axis.  Two occupied rows leave three components, each labelled by its first voxel."""
+    h, w = 1 << 15, (1 << 15) + 8
+    g = torch.zeros((1, h, w, 1), dtype=torch.bool, device=gpu)
+    g[0, 1000] = True
+    g[0, 20_001] = True
+    lab = cubvh_amd.floodfill(g)[0, :, :, 0]
+    for first, last, value in ((0, 1000, 0), (1000, 1001, -1), (1001, 20_001, 1001 * w), (20_001, 20_002, -1), (20_002, h, 20_002 * w)):
+        assert bool((lab[first:last] == value).all())
