@@ -2,6 +2,7 @@
 and to the oracle."""
 import contextlib
 import ctypes
+import inspect
 import math
 
 import numpy as np
@@ -10,6 +11,7 @@ import torch
 
 import cubvh_amd
 from cubvh_amd import synthetic as S
+import test_gpu_queries
 from test_ray_line_host import check, rim_rays, thin_faces  # noqa: F401 (a fixture)
 
 pytestmark = pytest.mark.gpu
@@ -137,3 +139,79 @@ def test_routes_agree_around_their_limits(gpu, level):
             for route in (1, 2):
                 with walks(bvh, route):
                     same_bits(out, call())
+
+
+# route, places of the list, steps before a walk may end, sixteenths of the average
+CONTROLS = {"packets": (2, -1, 0, -1), "handed over": (2, 1 << 19, 8, 0), "list full": (2, 37, 8, 0), "no list": (2, 0, 8, 0)}
+
+
+@pytest.mark.parametrize("control", CONTROLS)
+@pytest.mark.parametrize("name", [
+    "test_udf_leading_dims_and_far_points", "test_udf_perturbed_level6_bit_exact", "test_rays_bit_exact_and_vs_fp64",
+    "test_sdf_watertight_bit_exact", "test_sdf_raystab_threshold_sizes_and_empty_lists", "test_duplicate_faces_tie_to_lowest_index",
+    "test_camera_rays_packet_path_bit_exact", "test_nan_and_inf_queries", "test_degenerate_faces_bit_exact",
+    "test_ray_edge_cases_bit_exact", "test_points_on_the_surface_bit_exact", "test_random_soups_bit_exact"])
+def test_oracle_by_packets(gpu, request, monkeypatch, name, control):
+    """The oracle tests of the query calls, whose sizes the library gives to waves, with every
+    query in packets, whose walks all end where told or may hand over after a few steps."""
+    init = cubvh_amd.cuBVH.__init__
+
+    def controlled(self, *args, **kwargs):
+        init(self, *args, **kwargs)
+        walks(self, *CONTROLS[control]).__enter__()
+
+    monkeypatch.setattr(cubvh_amd.cuBVH, "__init__", controlled)
+    test = getattr(test_gpu_queries, name)
+    given = {"seed": 103} if name == "test_random_soups_bit_exact" else {}
+    for arg in inspect.signature(test).parameters:
+        if arg not in given:
+            given[arg] = request.getfixturevalue(arg)
+    test(**given)
+
+
+def _cells_of(case, gpu):
+    """Mesh and calls of a hand-over case: name -> call, the same queries at their own order."""
+    rng = np.random.default_rng(11)
+    v, f = S.soup(5, seed=3, n_random=4000)
+    n = 60_011
+    p = S.uniform_points(n, seed=12)
+    p[: n // 3] = (v[f[rng.integers(0, len(f), n // 3)]].mean(axis=1) + rng.normal(0, 0.01, (n // 3, 3))).astype(np.float32)
+    p[:5] = [[np.nan, 0, 0], [0, np.inf, 0], [np.nan] * 3, [2000, 0, 0], [0, 0, 0]]
+    P = torch.from_numpy(p[rng.permutation(n)]).to(gpu)
+    if case == "lanes":
+        rays = S.sphere_rays(n, seed=13)
+    else:
+        rays = S.camera_rays(width=320, height=96, n_poses=2, seed=3)
+    O, D = (torch.from_numpy(x).to(gpu) for x in rays)
+    bvh = cubvh_amd.cuBVH(v, f)
+    return bvh, {"unsigned": lambda: bvh.unsigned_distance(P, return_uvw=True), "watertight": lambda: bvh.signed_distance(P, return_uvw=True),
+                 "lanes": lambda: bvh.ray_trace(O, D), "camera": lambda: bvh.ray_trace(O, D)}[case]
+
+
+@pytest.mark.parametrize("case", ["unsigned", "watertight", "lanes", "camera"])
+def test_handed_over_walks_equal_waves(gpu, case):
+    """Lists that hold every walk that ends early, some of them (places in the middle of a
+    wave's run stay empty), and none: the same bits, and the list was used, or too short."""
+    bvh, call = _cells_of(case, gpu)
+    with walks(bvh, 1):
+        ref = call()
+    for cap in (1 << 19, 5000, 100, 1, 0):
+        for factor in (0, 24):
+            with walks(bvh, 2, cap, 8, factor) as handed:
+                same_bits(ref, call())
+                assert handed() > (cap if cap <= 100 or (cap == 5000 and factor == 0) else 0)
+
+
+@pytest.mark.parametrize("tuning", [(4, 0, 8, 1), (4, 0, 8, 8), (4, 1, 4, 2), (0, 1, 16, 4)])
+def test_handed_over_forest_walks_equal_single_meshes(gpu, tuning):
+    meshes = [S.soup(4, seed=s, n_random=500) for s in range(5)] + [S.icosphere(1, 0.4)]
+    bvhs = [cubvh_amd.cuBVH(*m) for m in meshes]
+    counts = [9000, 0, 12_345, 70, 8000, 3000]
+    off = torch.from_numpy(np.concatenate([[0], np.cumsum(counts)]))
+    P = torch.from_numpy(S.uniform_points(sum(counts), seed=5)).to(gpu)
+    forest = cubvh_amd.cuBVHForest(bvhs)
+    ref = [torch.cat(x) for x in zip(*[b.unsigned_distance(P[a:e], return_uvw=True) for b, a, e in zip(bvhs, off, off[1:]) if e > a])]
+    for cap in (1 << 19, 1000, 100, 0):
+        with walks(forest, 0, cap, 8, 0) as handed:
+            same_bits(ref, forest.unsigned_distance(P, off, return_uvw=True, tuning=tuning))
+            assert handed() > (0 if cap == 1 << 19 else cap)
