@@ -1,7 +1,8 @@
 // query.hip -- BVH traversal kernels for gfx950 (wave64).
 //
-// Three forms: one lane per query (stab rays, incoherent rays), a packet of 64 queries per
-// wave (below, "Packet traversal") and one wave per query (wave_walk.hpp).
+// Three forms: one lane per query (stab lines of large calls, incoherent rays), a packet of
+// 64 queries per wave (below, "Packet traversal") and one wave per query (wave_walk.hpp);
+// query.hpp says which calls take which.
 //
 // One lane per query: each lane walks the 4-wide tree nearest-child-first: the
 // four child bounds of a node arrive as six 16-byte loads (structure-of-arrays
@@ -18,6 +19,9 @@
 //   distance: smallest fp32 squared distance, ties to the lowest original face id
 //   ray:      smallest hit parameter t < 1000, ties to the lowest original face id
 //   any-hit:  exists a face with t < 1000
+// The ray rule holds where a hit's rounded t is not below its leaf's box entry.  A ray almost
+// in a face's plane can meet it at a t before that; whether another face with the same t, or
+// such a hit behind a nearer one, is then seen hangs on the order of the walk.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -430,17 +434,18 @@ __device__ int any_hit_line(const Tree& T, f3 o, f3 d, LaneStack<BLOCK, LDS_N>& 
 struct NormalSum {
     double x = 0.0, y = 0.0, z = 0.0;
     float n = 0.0f;
-    uint32_t least = 0xffffffffu;  // bits of the smallest component but 0, less 1
+    uint32_t least = 0xffffffffu;  // twice the bits of the smallest component but 0, less 1
 
     __device__ __forceinline__ void add(f3 v) {
-        least = min(least, min((__float_as_uint(v.x) & 0x7fffffffu) - 1u,
-                               min((__float_as_uint(v.y) & 0x7fffffffu) - 1u, (__float_as_uint(v.z) & 0x7fffffffu) - 1u)));
+        const uint32_t lx = (__float_as_uint(v.x) << 1) - 1u, ly = (__float_as_uint(v.y) << 1) - 1u,
+                       lz = (__float_as_uint(v.z) << 1) - 1u;
+        least = min(min(lx, ly), min(lz, least));
         x += (double)v.x;
         y += (double)v.y;
         z += (double)v.z;
         n += 1.0f;
     }
-    __device__ __forceinline__ bool exact() const { return least >= __float_as_uint(n * 0x1p-28f); }
+    __device__ __forceinline__ bool exact() const { return least >= __float_as_uint(n * 0x1p-28f) << 1; }
     __device__ __forceinline__ f3 mean() const { return mk3((float)x / n, (float)y / n, (float)z / n); }
 };
 struct NormalParts {
@@ -1763,8 +1768,8 @@ constexpr int kLdsEntries = 12;
 constexpr int kDistanceWaves = 1;
 constexpr uint32_t kRestBlocks = 8192;  // one-wave workgroups of a rest launch: what the chip holds at once
 
-// Raystab calls of fewer queries walk their lines 1 .. 31 a wave per line (line 0 below
-// kWaveMax).  Measured, waves against lanes: 2,100 points 0.08-0.14 / 2.1-8.5 ms (the lanes
+// Raystab calls of fewer queries walk their lines 1 .. 31 a wave per line (line 0 where
+// query.hpp gives the distances to waves).  Measured, waves against lanes: 2,100 points 0.08-0.14 / 2.1-8.5 ms (the lanes
 // with the distances as packets, on 20,480 to 1.3 M faces), 200,000 1.0-1.6 / 2.6-6.4;
 // 600,011 2.0 / 3.2, 3.1 / 5.7, 4.1 / 7.9 ms on soups, 3.5 / 3.8 on a closed mesh; 2,000,000
 // 4.0 / 5.2, 5.8 / 8.5, 7.7 / 11.9, but 8.7 / 7.2 on the closed mesh, whose lines are short
