@@ -98,11 +98,11 @@ constexpr int64_t kRestFaces = (int64_t)1 << 11;
 constexpr int64_t kRestQueries = (int64_t)1 << 8;
 constexpr int64_t kRestFirst = (int64_t)1 << 14;
 constexpr int64_t kRestLast = (int64_t)1 << 23;
-// Ray calls, whose walks are shorter: 307,200 camera rays on 1.3 M faces 455 us with, 692
-// without, 263,000 scattered ones 754 and 880, 2,000,000 2,023 and 2,067, 7,000,000 5,575 and
-// 5,627 (with the budget that both lane walks counted then); on 81,920 faces 566 and 559.
+// Ray calls, whose walks are shorter: on 1.3 M faces 307,200 camera rays 455 us with, 692
+// without, 8.3 M 1,148 and 1,195; 263,000 scattered ones 754 and 880, 7,000,000 5,575 and
+// 5,627; on 81,920 faces 566 and 559.  Very many rays cover their long walks as above.
 constexpr int64_t kRayRestFaces = (int64_t)1 << 18;
-constexpr int64_t kRayRestLast = (int64_t)1 << 22;
+constexpr int64_t kRayRestLast = (int64_t)1 << 24;
 inline bool hands_over(int64_t n, int64_t n_faces) {
     return n >= kRestFirst && n < kRestLast && n_faces >= kRestFaces && n / kRestQueries < n_faces;
 }
