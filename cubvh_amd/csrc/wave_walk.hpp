@@ -12,12 +12,14 @@
 // always taken nearest first (640 exact face tests a query, now 143).
 //
 // What bounds it: instruction issue.  A query on 81,920 faces takes 8 node, 5 face and 2
-// exact rounds, some 1,730 vector and as many scalar instructions (each 84% of the issue
-// slots of a full chip); the bytes (about 20 KB a query) come out of L2 and the Infinity
+// exact rounds, some 1,730 vector instructions (57% of their lanes active) and as many scalar
+// ones: 0.17 of each per SIMD-cycle, where the fma probe reads 0.42 with vector operands and
+// 0.22 with a scalar one; the bytes (about 20 KB a query) come out of L2 and the Infinity
 // Cache.  Exact tests recompute the face's terms from its 48-byte record: the 144-byte
 // record that packets read made 250,000 points on 1.3 M faces 1.48 ms instead of 1.19.
 // Measured: 777 points on 5,120 faces 16 us (351 us with a lane each); 50,003 on 81,920
-// 0.22 ms (3.8 ms as packets); 1,501 rays on 81,920 14 us (146).  Not taken: 16 lanes per
+// 0.21 ms (3.8 ms as packets, before their seeds and hand-over; query.hpp has both routes'
+// times now); 1,501 rays on 81,920 14 us (146).  Not taken: 16 lanes per
 // query, four walks a wave (0.9-1.4 times as long), and queries in Morton order (5%, less
 // than the ordering costs).
 #pragma once
