@@ -8,7 +8,8 @@
 //   1. tiles  : each workgroup labels one tile of 64 x 8 x 8 voxels (64 along the last
 //               axis: one row per wave, a lane per voxel, so that occupancy is one ballot,
 //               loads and stores are whole lines, and runs are bit arithmetic), or of
-//               16 x 16 x 16, four rows per wave, where the last axis has at most 16.
+//               16 x 16 x 16, four rows per wave, where the last axis has at most 16 and the
+//               grids are many or large.
 //               Union-find in LDS between overlapping runs of neighbouring rows; every
 //               free voxel gets the global index of its tile-local root, others -1.
 //   2. merge  : voxels on a tile's low faces union themselves with their free
@@ -309,6 +310,7 @@ namespace {
 
 // A launch has fewer than 2^32 threads: tiles in runs of 2^23 workgroups.
 constexpr int64_t kTileRun = (int64_t)1 << 23;
+constexpr int64_t kNarrowTiles = 1024;
 
 template <int TD>
 hipError_t launch_tiles(const uint8_t* grid, int32_t B, int32_t H, int32_t W, int32_t D, int32_t* labels, hipStream_t stream) {
@@ -342,7 +344,12 @@ hipError_t launch_floodfill(const uint8_t* grid, int32_t B, int32_t H, int32_t W
         W = H;
         H = 1;
     }
-    return D <= 16 ? launch_tiles<16>(grid, B, H, W, D, labels, stream) : launch_tiles<64>(grid, B, H, W, D, labels, stream);
+    // Rows of 64 leave three lanes of four idle when the last axis has at most 16, but while
+    // they make fewer than four workgroups a CU there is room for them: 64 grids of 16^3
+    // (256 workgroups, or 64 of narrow tiles) 26-36 and 28-42 us, 512 of them 47-63 and 31-48.
+    const int64_t wide = (int64_t)B * ((H + 7) / 8) * ((W + 7) / 8);
+    return D <= 16 && wide >= kNarrowTiles ? launch_tiles<16>(grid, B, H, W, D, labels, stream)
+                                           : launch_tiles<64>(grid, B, H, W, D, labels, stream);
 }
 
 }  // namespace cubvh_amd

@@ -424,7 +424,7 @@ __device__ int any_hit_line(const Tree& T, f3 o, f3 d, LaneStack<BLOCK, LDS_N>& 
 
 // Sum of face normals that does not depend on the order they are added in, so that a query
 // gets the same sign from a lane, a wave and any tree.  The first walk adds in double, which
-// is exact when every component is 0 or at least 2^-28 times the count (components of 24
+// is exact when every component is 0 or above 2^-27 times the count (components of 24
 // bits: the sum spans at most 53).  Otherwise (1 + 1e-20 - 1, as on back-to-back sheets
 // built with sines and cosines) further walks add one part of every component each: the
 // multiples of 2^-27, then of 2^-54 and so on, the sixth part the rest (multiples of
@@ -445,7 +445,7 @@ struct NormalSum {
         z += (double)v.z;
         n += 1.0f;
     }
-    __device__ __forceinline__ bool exact() const { return least >= __float_as_uint(n * 0x1p-28f) << 1; }
+    __device__ __forceinline__ bool exact() const { return least >= __float_as_uint(n * 0x1p-27f) << 1; }
     __device__ __forceinline__ f3 mean() const { return mk3((float)x / n, (float)y / n, (float)z / n); }
 };
 struct NormalParts {

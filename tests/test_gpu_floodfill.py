@@ -82,10 +82,12 @@ def test_floodfill_across_tiles(gpu, oracle, shape, kind):
 
 @pytest.mark.parametrize("shape", [(1, 1, 1, 1), (5, 1, 1, 1), (1, 1, 1, 70), (1, 1, 70, 1), (3, 70, 1, 1), (2, 33, 50, 1), (1, 1, 17, 9),
                                    (1, 40, 1, 12), (1, 16, 16, 16), (2, 17, 33, 2), (1, 50, 35, 16), (1, 50, 35, 17),
-                                   (3, 9, 70, 7), (1, 100, 90, 1), (70, 4, 4, 4)])
+                                   (3, 9, 70, 7), (1, 100, 90, 1), (70, 4, 4, 4), (1023, 5, 6, 3), (1024, 5, 6, 3), (256, 16, 16, 16),
+                                   (130, 17, 19, 2), (1, 257, 249, 16), (1, 250, 265, 9), (3, 129, 300, 5), (300, 15, 9, 13)])
 @pytest.mark.parametrize("free", [0.4, 0.65, 0.9, 1.0])
 def test_floodfill_short_axes(gpu, oracle, shape, free):
-    """A short last axis (tiles of 16 x 16 x 16), around their sizes, and axes of one voxel."""
+    """A short last axis (tiles of 16 x 16 x 16 from 1,024 tiles of 64 x 8 x 8 on), around their
+    sizes, and axes of one voxel."""
     g = np.random.default_rng(sum(shape)).random(shape) >= free
     lab = cubvh_amd.floodfill(torch.from_numpy(g).to(gpu)).cpu().numpy()
     np.testing.assert_array_equal(lab, oracle.floodfill_bfs(g))
