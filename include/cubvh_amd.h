@@ -157,7 +157,7 @@ int cubvh_signed_distance(cubvh_bvh* bvh, int device, int64_t n, uint32_t mode, 
  * identical to the unordered calls for any permutation; order entries >= n are
  * skipped (their queries are not written).  Neither call keeps a reference to the
  * caller's buffers; cubvh_morton_order allocates stream-ordered scratch,
- * cubvh_distance_ordered allocates nothing. */
+ * cubvh_distance_ordered allocates nothing, and all its walks run to their end. */
 int cubvh_morton_order(int device, int64_t n, const float* positions, uint32_t* order, void* stream);
 int cubvh_distance_ordered(cubvh_bvh* bvh, int device, int64_t n, int32_t kind, const float* positions,
                            const uint32_t* order, float* distances, int64_t* face_id, float* uvw, void* stream);
